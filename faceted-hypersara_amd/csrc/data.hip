@@ -64,23 +64,31 @@ constexpr int FB_THREADS = 512;
 constexpr int NXCD = 8;   // MI355X: 8 XCDs, each with its own L2
 
 // Workgroups of a launch are dispatched to the XCDs round-robin (linear id
-// mod 8).  The per-channel kernels below are launched as a 1-D grid of
-// NXCD * ceil(L / NXCD) * units workgroups and remapped so that XCD x only
-// runs channels x, x + 8, ...: one channel's v2 / coefficients / grid
-// region is then shared by one L2 instead of being pulled into all eight.
-// Units are interleaved over those channels (unit-major), so the first
+// mod 8).  The per-channel kernels below are launched as a 1-D grid and
+// remapped so that every XCD gets the same share of every launch and as few
+// channels as that allows, since one channel's v2 / coefficients / grid
+// region then sits in one L2.  With g = gcd(L, 8), channel l belongs to the
+// group l mod g, whose 8 / g XCDs split each channel's units between them
+// (unit mod 8 / g): L = 16 keeps a channel on one XCD, L = 4 puts it on two,
+// an odd L on all eight.  (One XCD per channel whatever L left 7 of 8 idle at
+// L = 1 and half of them at L = 4: the data step of 4 channels took 2.41 ms at
+// 2048 x 2048 with 500k w-projected rows each, 1.00 ms in the DR form of
+// 256 x 256 images, against 1.86 and 0.60 ms with this map.)
+// Units are interleaved over an XCD's channels (unit-major), so the first
 // units of every channel (the heaviest adjoint tiles) start first.
+__host__ __device__ __forceinline__ int xcd_groups(int L) { return L & 1 ? 1 : L & 2 ? 2 : L & 4 ? 4 : NXCD; }
+
 __device__ __forceinline__ bool xcd_map(int L, int units, int& chan, int& unit) {
-  const int b = blockIdx.x;
-  const int xcd = b % NXCD, s = b / NXCD;
-  const int cpx = (L + NXCD - 1) / NXCD;   // channels per XCD
-  chan = xcd + NXCD * (s % cpx);
-  unit = s / cpx;
-  return chan < L && unit < units;
+  const int g = xcd_groups(L), parts = NXCD / g, cpx = L / g;   // cpx: channels of a group
+  const int xcd = blockIdx.x % NXCD, s = blockIdx.x / NXCD;
+  chan = xcd % g + g * (s % cpx);
+  unit = (s / cpx) * parts + xcd / g;
+  return unit < units;
 }
 
 inline unsigned xcd_grid(int L, int units) {
-  return (unsigned)(NXCD * ((L + NXCD - 1) / NXCD) * units);
+  const int g = xcd_groups(L), parts = NXCD / g;
+  return (unsigned)(NXCD * (L / g) * cdiv(units, parts));
 }
 
 __global__ __launch_bounds__(256) void k_data_forward(const GDev* __restrict__ gd,
