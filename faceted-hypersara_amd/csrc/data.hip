@@ -27,7 +27,6 @@ struct fhs_data {
   int adj_grid = 0;                    // max adjoint units + grid-tail units over CSC channels
   int tile_grid = 0;                   // max tile work items over tile-gridded channels
   int red_grid = 0;                    // max split tiles over tile-gridded channels
-  size_t tile_lds = 0;                 // LDS bytes of a tile workgroup (max over channels)
   int kmax = 0;                        // slots per axis of the tiled channels' separable rows
   int fwd_grid = 0;                    // max forward work items over tile-gridded channels
   bool any_rows = false;               // some channel without tile gridding (row kernels)
@@ -594,34 +593,28 @@ __global__ __launch_bounds__(ADJ_THREADS) void k_data_adjoint(const GDev* __rest
 }
 
 // g2_l = G_l' (lam .* v2_l) for the channels with a tile-gridded separable G
-// (one workgroup per grid tile; never the DR form, whose H is square).
+// (one wave per patch job; never the DR form, whose H is square).
 template <bool LAM, int KM>
 __global__ __launch_bounds__(ADJ_THREADS) void k_data_adjoint_tiled(const GDev* __restrict__ gd,
                                                                     const int64_t* __restrict__ row_off,
                                                                     const float2* __restrict__ v2,
                                                                     const float* __restrict__ lam, int64_t No,
                                                                     float2* __restrict__ g2, int L, int units) {
-  extern __shared__ __align__(16) unsigned char t[];
   int l, u;
   if (!xcd_map(L, units, l, u)) return;
-  const GDev g = gd[l];
+  const GDev& g = gd[l];
   if (!g.tiled || u >= g.nunits) return;
-  const float2* __restrict__ v = v2 + row_off[l];
-  const float* __restrict__ lm = LAM ? lam + row_off[l] : nullptr;
-  if (LAM)
-    g_adjoint_tile<KM>(g, u, [=](int r) { return cscale(v[r], lm[r]); }, g2 + (size_t)l * No, t);
-  else
-    g_adjoint_tile<KM>(g, u, [=](int r) { return v[r]; }, g2 + (size_t)l * No, t);
+  g_adjoint_patches<KM, LAM>(g, u, v2 + row_off[l], LAM ? lam + row_off[l] : nullptr, g2 + (size_t)l * No);
 }
 
-// sums of the partial tiles of the tiles split over several work items
+// sums of the partial patches of the patches split over several jobs
 __global__ __launch_bounds__(ADJ_THREADS) void k_data_adjoint_reduce(const GDev* __restrict__ gd, int64_t No,
                                                                      float2* __restrict__ g2, int L, int units) {
   int l, u;
   if (!xcd_map(L, units, l, u)) return;
   const GDev g = gd[l];
   if (!g.tiled || u >= g.nred) return;
-  g_adjoint_tile_reduce(g, u, g2 + (size_t)l * No);
+  g_adjoint_reduce(g, u, g2 + (size_t)l * No);
 }
 
 void launch_data_adjoint(fhs_ctx* ctx, const fhs_data* D, const float2* v2, const float* lam, int dr) {
@@ -635,9 +628,8 @@ void launch_data_adjoint(fhs_ctx* ctx, const fhs_data* D, const float2* v2, cons
   }
   if (D->tile_grid > 0) {
     auto go = [&](auto kern) {
-      allow_dynamic_lds((const void*)kern, D->tile_lds);
-      kern<<<xcd_grid(L, D->tile_grid), ADJ_THREADS, D->tile_lds, ctx->stream>>>(D->gdev, D->d_row_off, v2, lam,
-                                                                                 D->No, D->g2, L, D->tile_grid);
+      kern<<<xcd_grid(L, D->tile_grid), ADJ_THREADS, 0, ctx->stream>>>(D->gdev, D->d_row_off, v2, lam, D->No, D->g2,
+                                                                       L, D->tile_grid);
     };
     if (D->kmax == 8)
       lam ? go(k_data_adjoint_tiled<true, 8>) : go(k_data_adjoint_tiled<false, 8>);
@@ -964,7 +956,6 @@ int fhs_data_create(fhs_ctx* ctx, const fhs_nufft* A, int L, const fhs_gmat* con
         D->kmax = G[l]->d.kmax;
         D->tile_grid = std::max<int>(D->tile_grid, G[l]->d.nunits);
         D->red_grid = std::max<int>(D->red_grid, G[l]->d.nred);
-        D->tile_lds = std::max(D->tile_lds, tile_lds_bytes(G[l]->d.Ky, G[l]->d.Kx));
         D->fwd_grid = std::max<int>(D->fwd_grid, G[l]->d.nfitems);
       } else {
         D->any_rows = true;

@@ -83,73 +83,61 @@ void build_csc(int64_t ncols, const std::vector<int>& rows, const std::vector<in
 
 struct TileLists {
   int tiles_y = 0, tiles_x = 0;
-  std::vector<int> rows, cell, empty;
-  std::vector<int4> items, red;
+  std::vector<int> empty;
+  std::vector<int2> pent;
+  std::vector<int4> jobs, red;
   int slots = 0;
   std::vector<int> prim_rows;
   std::vector<int4> fitems;
 };
 
-// every row under each tile its Ky x Kx window touches, sorted by local cell
+// every row under each patch its Ky x Kx window touches, rows ascending
 TileLists tile_lists(int64_t M, const int32_t* anchor, int Kty, int Ktx, int Ky, int Kx) {
   TileLists T;
   T.tiles_y = Kty / TILE_Y;
   T.tiles_x = Ktx / TILE_X;
-  const int nt = T.tiles_y * T.tiles_x, ncy = TILE_Y + Ky - 1;
+  const int nt = T.tiles_y * T.tiles_x;
+  const int npy = Kty / PATCH, npx = Ktx / PATCH, np = npy * npx;
   auto visit = [&](int a, auto&& f) {
     const int ay = a % Kty, ax = a / Kty;
-    const int ys[2] = {ay / TILE_Y, ((ay + Ky - 1) % Kty) / TILE_Y};
-    const int xs[2] = {ax / TILE_X, ((ax + Kx - 1) % Ktx) / TILE_X};
-    for (int i = 0; i < 2; ++i) {
-      if (i == 1 && xs[1] == xs[0]) break;
-      for (int j = 0; j < 2; ++j) {
-        if (j == 1 && ys[1] == ys[0]) break;
-        const int ty = ys[j], tx = xs[i];
-        const int cyl = ((ay - ty * TILE_Y + Ky - 1) % Kty + Kty) % Kty;
-        const int cxl = ((ax - tx * TILE_X + Kx - 1) % Ktx + Ktx) % Ktx;
-        f(tx * T.tiles_y + ty, cxl * ncy + cyl);
-      }
-    }
+    for (int px = ax / PATCH; px <= (ax + Kx - 1) / PATCH; ++px)
+      for (int py = ay / PATCH; py <= (ay + Ky - 1) / PATCH; ++py)
+        f((px % npx) * npy + py % npy, ay - py * PATCH, ax - px * PATCH);
   };
-  std::vector<int64_t> cnt(nt + 1, 0);
-  for (int64_t m = 0; m < M; ++m) visit(anchor[m], [&](int t, int) { cnt[t + 1]++; });
-  for (int t = 0; t < nt; ++t) cnt[t + 1] += cnt[t];
-  FHS_CHECK(cnt[nt] < (1ll << 31), "gmat_create_separable: tile lists too long");
-  std::vector<std::pair<int, int>> ent(cnt[nt]);   // (cell, row)
-  std::vector<int64_t> pos(cnt.begin(), cnt.end() - 1);
-  for (int64_t m = 0; m < M; ++m)
-    visit(anchor[m], [&](int t, int c) { ent[pos[t]++] = {c, (int)m}; });
-  T.rows.resize(cnt[nt]);
-  T.cell.resize(cnt[nt]);
-  for (int t = 0; t < nt; ++t) std::sort(ent.begin() + cnt[t], ent.begin() + cnt[t + 1]);   // by cell, then row
-  for (size_t e = 0; e < ent.size(); ++e) {
-    T.cell[e] = ent[e].first;
-    T.rows[e] = ent[e].second;
+  std::vector<int64_t> cnt(np + 1, 0);
+  for (int64_t m = 0; m < M; ++m) visit(anchor[m], [&](int p, int, int) { cnt[p + 1]++; });
+  for (int p = 0; p < np; ++p) cnt[p + 1] += cnt[p];
+  FHS_CHECK(cnt[np] < (1ll << 31), "gmat_create_separable: patch lists too long");
+  T.pent.resize(cnt[np]);
+  {
+    std::vector<int64_t> pos(cnt.begin(), cnt.end() - 1);
+    for (int64_t m = 0; m < M; ++m)
+      visit(anchor[m], [&](int p, int dy, int dx) {
+        T.pent[pos[p]++] = make_int2((int)m, (dy & 0xff) | ((dx & 0xff) << 8));
+      });
   }
-  // work items, largest first: whole tiles of at most TILE_ITEM listed rows,
-  // larger tiles cut into TILE_ITEM pieces (partial slots), empty tiles in groups
-  std::vector<int> order(nt);
-  std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(),
-                   [&](int a, int b) { return cnt[a + 1] - cnt[a] > cnt[b + 1] - cnt[b]; });
-  for (int t : order) {
-    const int b = (int)cnt[t], e = (int)cnt[t + 1], n = e - b;
+  // jobs, longest first: patches of at most PATCH_JOB rows whole, larger ones
+  // cut into equal pieces (partial slots), empty ones in groups
+  for (int p = 0; p < np; ++p) {
+    const int b = (int)cnt[p], n = (int)(cnt[p + 1] - cnt[p]);
     if (n == 0) {
-      T.empty.push_back(t);
+      T.empty.push_back(p);
       continue;
     }
-    const int k = (n + TILE_ITEM - 1) / TILE_ITEM;
+    const int k = (n + PATCH_JOB - 1) / PATCH_JOB;
     if (k == 1) {
-      T.items.push_back(make_int4(t, b, e, -1));
+      T.jobs.push_back(make_int4(p, b, n, -1));
       continue;
     }
-    T.red.push_back(make_int4(t, T.slots, k, 0));
-    for (int j = 0; j < k; ++j)
-      T.items.push_back(make_int4(t, b + j * TILE_ITEM, std::min(e, b + (j + 1) * TILE_ITEM), T.slots++));
+    T.red.push_back(make_int4(p, T.slots, k, 0));
+    for (int j = 0; j < k; ++j) {
+      const int e0 = (int)((int64_t)n * j / k), e1 = (int)((int64_t)n * (j + 1) / k);
+      T.jobs.push_back(make_int4(p, b + e0, e1 - e0, T.slots++));
+    }
   }
-  std::stable_sort(T.items.begin(), T.items.end(), [](const int4& a, const int4& b) { return a.z - a.y > b.z - b.y; });
-  for (size_t e = 0; e < T.empty.size(); e += TILE_EMPTY_GROUP)
-    T.items.push_back(make_int4(-1, (int)e, (int)std::min(T.empty.size(), e + TILE_EMPTY_GROUP), -2));
+  std::stable_sort(T.jobs.begin(), T.jobs.end(), [](const int4& a, const int4& b) { return a.z > b.z; });
+  for (size_t e = 0; e < T.empty.size(); e += PATCH_EMPTY_GROUP)
+    T.jobs.push_back(make_int4(-1, (int)e, (int)(std::min(T.empty.size(), e + PATCH_EMPTY_GROUP) - e), -2));
   // forward: every row once, under the tile of its anchor, rows ascending
   std::vector<int64_t> pc(nt + 1, 0);
   auto prim = [&](int a) { return (a / Kty / TILE_X) * T.tiles_y + (a % Kty) / TILE_Y; };
@@ -169,7 +157,7 @@ TileLists tile_lists(int64_t M, const int32_t* anchor, int Kty, int Ktx, int Ky,
 }
 
 __global__ __launch_bounds__(ADJ_THREADS) void k_gmat_adjoint_reduce(GDev g, float2* __restrict__ out) {
-  g_adjoint_tile_reduce(g, blockIdx.x, out);
+  g_adjoint_reduce(g, blockIdx.x, out);
 }
 
 template <int KM>
@@ -191,22 +179,20 @@ __global__ void k_gmat_forward(GDev g, const float2* __restrict__ Fx,
   y[m] = acc;
 }
 
-template <int KM>
+template <int KM, bool LAM>
+__global__ __launch_bounds__(ADJ_THREADS) void k_gmat_adjoint_tiled(GDev g, const float2* __restrict__ y,
+                                                                  const float* __restrict__ lam,
+                                                                  float2* __restrict__ out) {
+  g_adjoint_patches<KM, LAM>(g, blockIdx.x, y, lam, out);
+}
+
 __global__ __launch_bounds__(ADJ_THREADS) void k_gmat_adjoint(GDev g, const float2* __restrict__ y,
                                                                const float* __restrict__ lam,
                                                                float2* __restrict__ out) {
-  extern __shared__ __align__(16) unsigned char lds[];
+  __shared__ float2 prod[ADJ_LDS];
   auto none = [](int) { return make_float2(0.f, 0.f); };
-  auto wl = [&](int r) { return cscale(y[r], lam[r]); };
-  auto wp = [&](int r) { return y[r]; };
-  if (g.tiled) {
-    if (lam) g_adjoint_tile<KM>(g, blockIdx.x, wl, out, lds);
-    else g_adjoint_tile<KM>(g, blockIdx.x, wp, out, lds);
-  } else {
-    float2* prod = reinterpret_cast<float2*>(lds);
-    if (lam) g_adjoint_unit(g, blockIdx.x, wl, none, out, prod);
-    else g_adjoint_unit(g, blockIdx.x, wp, none, out, prod);
-  }
+  if (lam) g_adjoint_unit(g, blockIdx.x, [&](int r) { return cscale(y[r], lam[r]); }, none, out, prod);
+  else g_adjoint_unit(g, blockIdx.x, [&](int r) { return y[r]; }, none, out, prod);
 }
 
 }  // namespace
@@ -410,28 +396,28 @@ int fhs_gmat_create_separable_host(fhs_ctx* ctx, int64_t M, int Kty, int Ktx, in
     d.anchor = (const int*)g->mem[0];
     d.vals = (const float2*)g->mem[1];
     if (tiled) {
-      g->mem[8] = upload(tl.rows);
-      g->mem[9] = upload(tl.cell);
-      g->mem[4] = upload(tl.items);
+      g->mem[8] = upload(tl.pent);
+      g->mem[4] = upload(tl.jobs);
       g->mem[5] = upload(tl.empty);
       g->mem[7] = upload(tl.red);
-      FHS_HIP(hipMalloc(&g->mem[10], std::max<size_t>(1, (size_t)tl.slots * TILE_Y * TILE_X) * sizeof(float2)));
+      FHS_HIP(hipMalloc(&g->mem[10], std::max<size_t>(1, (size_t)tl.slots * PATCH * PATCH) * sizeof(float2)));
       g->mem[11] = upload(tl.prim_rows);
       g->mem[12] = upload(tl.fitems);
       d.tiled = 1;
       d.tiles_y = tl.tiles_y;
       d.tiles_x = tl.tiles_x;
-      d.tile_rows = (const int*)g->mem[8];
-      d.tile_cell = (const int*)g->mem[9];
-      d.items = (const int4*)g->mem[4];
-      d.empty_tiles = (const int*)g->mem[5];
+      d.pent = (const int2*)g->mem[8];
+      d.jobs = (const int4*)g->mem[4];
+      d.njobs = (int)tl.jobs.size();
+      d.patches_y = Kty / PATCH;
+      d.empty = (const int*)g->mem[5];
       d.red = (const int4*)g->mem[7];
       d.nred = (int)tl.red.size();
       d.partial = (float2*)g->mem[10];
       d.prim_rows = (const int*)g->mem[11];
       d.fitems = (const int4*)g->mem[12];
       d.nfitems = (int)tl.fitems.size();
-      d.nunits = (int)tl.items.size();
+      d.nunits = (int)cdiv((long long)tl.jobs.size(), ADJ_THREADS / 64);
     } else {
       g->mem[2] = upload(colptr);
       g->mem[3] = upload(pk);
@@ -486,10 +472,17 @@ int fhs_apply_adjoint_operator(fhs_ctx* ctx, const fhs_gmat* G, const void* y,
   return guard(ctx, [&] {
     FHS_CHECK(G && Fx && y, "apply_adjoint_operator: null argument");
     Scope sc(ctx, "gmat_adjoint");
-    const size_t lds = G->d.tiled ? tile_lds_bytes(G->d.Ky, G->d.Kx) : ADJ_CSC_LDS_BYTES;
-    auto kern = G->d.kmax > 8 ? k_gmat_adjoint<16> : k_gmat_adjoint<8>;
-    allow_dynamic_lds((const void*)kern, lds);
-    kern<<<G->d.nunits, ADJ_THREADS, lds, ctx->stream>>>(G->d, (const float2*)y, Lambda, (float2*)Fx);
+    if (G->d.tiled) {
+      auto go = [&](auto kern) {
+        kern<<<G->d.nunits, ADJ_THREADS, 0, ctx->stream>>>(G->d, (const float2*)y, Lambda, (float2*)Fx);
+      };
+      if (G->d.kmax > 8)
+        Lambda ? go(k_gmat_adjoint_tiled<16, true>) : go(k_gmat_adjoint_tiled<16, false>);
+      else
+        Lambda ? go(k_gmat_adjoint_tiled<8, true>) : go(k_gmat_adjoint_tiled<8, false>);
+    } else {
+      k_gmat_adjoint<<<G->d.nunits, ADJ_THREADS, 0, ctx->stream>>>(G->d, (const float2*)y, Lambda, (float2*)Fx);
+    }
     check_launch();
     if (G->d.tiled && G->d.nred > 0) {
       k_gmat_adjoint_reduce<<<G->d.nred, ADJ_THREADS, 0, ctx->stream>>>(G->d, (float2*)Fx);

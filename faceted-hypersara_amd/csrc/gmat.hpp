@@ -23,6 +23,8 @@
 
 #include <hip/hip_fp16.h>
 
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace fhs {
@@ -50,19 +52,22 @@ struct GDev {
   const int* ucol;      // adjoint work units: unit u = columns [ucol[u], ucol[u+1])
   int nunits;
   const unsigned* csc_pk;  // SEP: (row << 6) | (jx*Ky + jy) per nonzero
-  // SEP on a tiled grid: adjoint by tile gridding (no CSC; nunits = items)
+  // SEP on a tiled grid: adjoint by patches (no CSC; nunits = workgroups of 4 jobs)
   int tiled, tiles_y, tiles_x;
-  const int* tile_rows;    // rows listed under every tile their window touches
-  const int* tile_cell;    // local anchor cell of each listed row
-  // work items {tile, begin, end, slot}, largest first: slot -1 writes the
-  // tile, slot >= 0 writes partial[slot] (a tile split over several items,
-  // summed in slot order by the reduce pass), slot -2 zeroes the empty tiles
-  // empty_tiles[begin, end)
-  const int4* items;
-  const int* empty_tiles;
-  const int4* red;         // {tile, first slot, slot count} of the split tiles
+  // rows listed under every 16 x 16 patch of the grid their window touches:
+  // {row, window origin relative to the patch as two signed bytes (y, x << 8)},
+  // rows ascending inside a patch
+  const int2* pent;
+  // one wave's work each, longest first: {patch, first entry, entries, slot};
+  // slot -1 writes the patch, slot >= 0 writes partial[slot] (a patch split over
+  // several jobs, summed in slot order by the reduce pass), slot -2 zeroes the
+  // empty patches empty[first .. first + entries)
+  const int4* jobs;
+  int njobs, patches_y;
+  const int* empty;
+  const int4* red;         // {patch, first slot, slot count} of the split patches
   int nred;
-  float2* partial;         // [slots][TILE_Y * TILE_X]
+  float2* partial;         // [slots][PATCH * PATCH]
   // forward by tile: rows grouped by the tile of their anchor (ascending row
   // order inside a tile), work items {tile, begin, end, 0} of <= FWD_ITEM rows
   const int* prim_rows;
@@ -266,61 +271,43 @@ __device__ __forceinline__ void g_adjoint_unit(const GDev& g, int u, W&& w, X&& 
   }
 }
 
-// Tile-gridding adjoint of the separable layout.
+// Gridding adjoint of the separable layout, on the matrix cores.
 //
-// The grid is cut into TILE_Y x TILE_X tiles.  At creation every row is
-// listed under each tile its Ky x Kx window touches (1, 2 or 4 tiles), with
-// its anchor cell relative to the tile ("local cell": (TILE_Y + Ky - 1) x
-// (TILE_X + Kx - 1) cells, x-major, the list sorted by it).  One workgroup
-// owns one tile and stages its listed rows in LDS a chunk at a time.  Two
-// forms, chosen by the row width:
-//  - 8-slot rows (7 x 7 windows): a cell-indexed gather.  The chunk is
-//    staged as Q[k][jx] = conj(cx[jx]) w(row), C[k][jy] = conj(cy[jy]);
-//    where each local cell starts in the chunk is found (the first row of
-//    each occupied cell marks it, a block-wide suffix minimum fills the
-//    rest), and every thread sums, for the grid points it owns, the rows of
-//    the Ky consecutive cells of each of the Kx cell columns that reach it.
-//  - 16-slot rows (the w-projected 15 x 15 windows): on the matrix cores.
-//    Restricted to one tile the adjoint is a sum of rank-1 updates,
-//      out[y][x] = sum_rows conj(cy[y - dy]) * (w(row) conj(cx[x - dx])),
-//    (dy, dx) the row's window origin relative to the tile: a GEMM whose
-//    inner dimension runs over the tile's rows.  Each of the 4 waves owns
-//    one 16 x 16 quadrant, accumulated by v_mfma_f32_16x16x4f32 in FP32, two
-//    complex rows per instruction pair (K = 4 real terms, re/im split over
-//    the A/B lanes), over the rows whose window meets its quadrant.  Rows
-//    are staged 32 at a time by all 256 threads (8 per row, coalesced), the
-//    next chunk loaded during this chunk's updates; 32-row chunks keep the
-//    LDS at 17 KB, so eight workgroups fit on a CU (the register limit).  A
-//    7 x 7 window fills under a fifth of such an update, which is why the
-//    narrow rows keep the gather.
-// Every output point is written once, by one thread, after a fixed-order
-// sum: no atomics, deterministic.  The uv density of a tile varies by
-// orders of magnitude (empty corners, a dense centre), so the work is cut
-// into items of at most TILE_ITEM listed rows: a dense tile is spread over
-// several workgroups whose partial tiles a second pass adds in a fixed
-// order, and empty tiles are zeroed in groups.
+// The grid is cut into 16 x 16 patches, and at creation every row is listed
+// under each patch its Ky x Kx window touches (1.9 for a 7 x 7 window on
+// average, 3.5 for 15 x 15), with its window origin (dy, dx) relative to the
+// patch.  Restricted to a patch the adjoint is a sum of rank-1 updates,
+//   out[y][x] = sum_rows conj(cy[y - dy]) * (w(row) conj(cx[x - dx])),
+// a GEMM whose inner dimension runs over the listed rows.  One wave owns one
+// patch and accumulates v_mfma_f32_16x16x4f32 in FP32, two complex rows per
+// instruction pair: lane (i, k) supplies re / im (k even / odd) of row k / 2 of
+// the pair.  The wave stages its rows in LDS of its own, 16 at a time, so there
+// is no barrier and no compaction.  A lane outside a row's window reads the
+// zero slot behind the row (its slot index is clamped).
+//
+// A zero times a non-finite value would still spread NaN over the patch, so
+// a patch with a non-finite sum is summed again tap by tap (patch_exact):
+// only the points a row's window covers see its value.
+//
+// Every output point is written once, by one lane, after a fixed-order sum: no
+// atomics, deterministic.  The uv density varies by orders of magnitude (empty
+// corners, a dense centre), so a patch's list is cut into jobs of at most
+// PATCH_JOB rows whose partial patches a second pass adds in a fixed order, and
+// empty patches are zeroed in groups.  Jobs are sorted by length, so the four
+// waves of a workgroup end together.  256 rows a job: the partial patches add an
+// eighth to the row bytes of a dense patch, and a channel of 65k rows still
+// fills the GPU (SARA 256 x 256: 18 us against 54 us for the earlier gather by
+// 32 x 32 tiles in LDS).  2.6M 7 x 7 rows on 16 grids of 1024 x 1024: 172 us
+// against 268 us for the gather; 1.6M 15 x 15 rows on 4 grids of 4096 x 4096:
+// 318 us, 112 us of it the time to write the grids at the rate of a large copy.
+constexpr int PATCH = 16;
+constexpr int PATCH_JOB = 256;                       // listed rows per job
+constexpr int PATCH_EMPTY_GROUP = 8;                 // empty patches zeroed per job
+// The forward stages windows of 32 x 32 tiles.
 constexpr int TILE_Y = 32, TILE_X = 32;
-constexpr int TILE_PTS = TILE_Y * TILE_X / ADJ_THREADS;
-constexpr int TILE_ITEM = 1024;                      // listed rows per work item
-constexpr int TILE_EMPTY_GROUP = 8;                  // empty tiles zeroed per work item
 constexpr int FWD_ITEM = 1024;                       // rows per forward work item
 template <int KM>
 constexpr int fwd_win() { return (TILE_Y + KM - 1) * (TILE_X + KM - 1); }   // forward window (complex)
-constexpr int TILE_GCH = ADJ_THREADS;                                        // rows staged per chunk (gather)
-template <int KM>
-constexpr int tile_cells_max() { return (TILE_Y + KM - 1) * (TILE_X + KM - 1); }
-
-// LDS of a tile workgroup (dynamic shared memory).  Matrix-core form
-// (16-slot rows): the staged C and B slots of a chunk, then each staged
-// row's window origin.  Gather form (8-slot rows): the staged rows with an
-// odd stride of Kx + Ky + 1 complex values (conj(cx) w, then conj(cy)), so
-// lanes reading consecutive rows hit different banks; their local cells;
-// the cell start offsets.
-__host__ __device__ inline size_t tile_lds_bytes(int Ky, int Kx);
-__host__ __device__ inline size_t tile_lds_bytes_gather(int Ky, int Kx) {
-  return (size_t)TILE_GCH * (Ky + Kx + 1) * 8 + (size_t)(TILE_GCH + ADJ_THREADS / 64) * 4 +
-         ((size_t)(TILE_Y + Ky - 1) * (TILE_X + Kx - 1) + 1) * 4;
-}
 
 // LDS of an adjoint workgroup that may run the CSC unit path (bytes)
 constexpr size_t ADJ_CSC_LDS_BYTES = ADJ_LDS * sizeof(float2);
@@ -331,350 +318,252 @@ inline bool tile_grid_ok(int Kty, int Ktx, int Ky, int Kx) {
 
 typedef float mfma_f4 __attribute__((ext_vector_type(4)));
 
-// Matrix-core tile layout in LDS (16-slot rows).  Staged row i's slots sit
-// at [i * TM_STRIDE + TM_GAP, + 16) of the C and B arrays, with TM_GAP zero
-// slots before the first row and after every row: a lane reading slot
-// jy = qy0 + lane - dy of a row whose window meets its quadrant lands in
-// [-15, 30] around the row's first slot, inside its values or the zero gaps,
-// so the reads need no bounds checks.
-constexpr int TM_GAP = 16, TM_STRIDE = 32;
-template <int CH>
-__host__ __device__ constexpr size_t tile_mfma_lds_bytes() {
-  return 2 * (size_t)(CH * TM_STRIDE + TM_GAP) * 8 + (size_t)CH * 4 + (size_t)4 * (CH + 4) * 4;
-}
-constexpr int TILE_MCH = 32;                          // rows staged per chunk (matrix cores)
-
-__host__ __device__ inline size_t tile_lds_bytes(int Ky, int Kx) {
-  return (Ky > 8 || Kx > 8) ? tile_mfma_lds_bytes<TILE_MCH>() : tile_lds_bytes_gather(Ky, Kx);
+// Pointers that a kernel reads from memory (the members of GDev) are generic
+// to the compiler, whose flat loads wait on the LDS counter too; these casts
+// say that they point to global memory.
+#define FHS_GLOBAL __attribute__((address_space(1)))
+typedef float vec2f __attribute__((ext_vector_type(2)));
+typedef int vec2i __attribute__((ext_vector_type(2)));
+typedef unsigned vec4u __attribute__((ext_vector_type(4)));
+typedef float vec4f __attribute__((ext_vector_type(4)));
+typedef float vec4f_a8 __attribute__((ext_vector_type(4), aligned(8)));   // a caller's complex array is 8-byte aligned
+template <class T>
+__device__ __forceinline__ const FHS_GLOBAL T* as_global(const void* p) {
+  return (const FHS_GLOBAL T*)p;
 }
 
-template <int KM, class W>
-__device__ __forceinline__ void g_adjoint_tile_mfma(const GDev& g, int item, W&& w, float2* __restrict__ out,
-                                                    unsigned char* lds) {
-  static_assert(ADJ_THREADS == 256, "one wave per 16 x 16 quadrant of a 32 x 32 tile");
-  static_assert(KM <= 16 && TM_GAP >= 15 && TM_STRIDE - 16 >= 15, "zero gaps cover a 16-lane read");
-  constexpr int CH = TILE_MCH;
-  constexpr int NSLOT = CH * TM_STRIDE + TM_GAP;
-  float2* C = reinterpret_cast<float2*>(lds);
-  float2* B = C + NSLOT;
-  int* meta = reinterpret_cast<int*>(B + NSLOT);       // [CH] window origin of staged row i
-  int* wl = meta + CH;                                 // [4][CH + 4] this wave's rows, as slot offsets
-  const int4 it = g.items[item];
-  if (it.w == -2) {   // a group of empty tiles: zeros
-    for (int e = it.y; e < it.z; ++e) {
-      const int t = g.empty_tiles[e];
-      const int ty = t % g.tiles_y, tx = t / g.tiles_y;
-#pragma unroll
-      for (int q = 0; q < TILE_PTS; ++q) {
-        const int p = threadIdx.x + q * ADJ_THREADS;
-        out[(size_t)(tx * TILE_X + p / TILE_Y) * g.Kty + ty * TILE_Y + p % TILE_Y] = make_float2(0.f, 0.f);
-      }
-    }
-    return;
-  }
-  const int t = it.x;
-  const int ty = t % g.tiles_y, tx = t / g.tiles_y;
-  const int ncy = TILE_Y + g.Ky - 1;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int li = lane & 15;
-  const bool odd = (lane >> 4) & 1;
-  const int half = lane >> 5;                          // A/B lanes 0-31: first row of a pair, 32-63: second
-  const int qy0 = (wv & 1) * 16, qx0 = (wv >> 1) * 16;
-  int* mine = wl + wv * (CH + 4);
-  // the gaps (and unused slots) are zero for the whole item
-  for (int k = threadIdx.x; k < NSLOT; k += ADJ_THREADS) {
-    C[k] = make_float2(0.f, 0.f);
-    B[k] = make_float2(0.f, 0.f);
-  }
-  mfma_f4 cre = {0.f, 0.f, 0.f, 0.f}, cim = {0.f, 0.f, 0.f, 0.f}, cre2 = cre, cim2 = cim;
-  // staging: TPR = ADJ_THREADS / CH threads per row, thread (row sk, part
-  // sp) loads 16 / TPR contiguous 16-byte words of the row's 2 KM slots
-  // (the first half of the parts cy, the second cx), so a chunk's rows
-  // arrive coalesced by all four waves; the next chunk's loads are issued
-  // before this chunk's matrix-core loop
-  constexpr int TPR = ADJ_THREADS / CH, FPT = 16 / TPR, SPT = 2 * FPT;   // float4 / slots per thread
-  static_assert(ADJ_THREADS % CH == 0 && 16 % TPR == 0 && KM == 16 && TPR >= 2, "row staging split");
-  const int sk = threadIdx.x / TPR, sp = threadIdx.x % TPR;
-  float4 pre[FPT];
-  uint4 preh = make_uint4(0u, 0u, 0u, 0u);   // FP16 rows: the raw word, converted when staged
-  float2 pv = make_float2(0.f, 0.f);
-  int pm = 0;
-  bool pok = false;
-  auto fetch = [&](int c) {
-    pok = sk < min(CH, it.z - c);
-    if (pok) {
-      const int r = g.tile_rows[c + sk];
-      const int cell = g.tile_cell[c + sk];
-      if (sp >= TPR / 2) pv = w(r);
-      if (g.half) {   // the same 4 slots in one 16-byte word of FP16 pairs
-        preh = reinterpret_cast<const uint4*>(reinterpret_cast<const __half2*>(g.vals) + (size_t)r * (2 * KM))[sp];
-      } else {
-        const float4* src = reinterpret_cast<const float4*>(g.vals + (size_t)r * (2 * KM)) + FPT * sp;
-#pragma unroll
-        for (int j = 0; j < FPT; ++j) pre[j] = src[j];
-      }
-      pm = (cell % ncy - (g.Ky - 1) + 32) | ((cell / ncy - (g.Kx - 1) + 32) << 8);
-    }
-  };
-  fetch(it.y);
-  for (int c0 = it.y; c0 < it.z; c0 += CH) {
-    const int n = min(CH, it.z - c0);
-    __syncthreads();   // the previous chunk's reads are done (and the zeroing)
-    if (pok) {
-      if (g.half) {
-        static_assert(FPT == 2, "FP16 rows: 4 slots per thread");
-        const float2 a = h2f(preh.x), b = h2f(preh.y), c = h2f(preh.z), d = h2f(preh.w);
-        pre[0] = make_float4(a.x, a.y, b.x, b.y);
-        pre[1] = make_float4(c.x, c.y, d.x, d.y);
-      }
-      const int s0 = (sp % (TPR / 2)) * SPT;   // first slot of this thread's part
-      if (sp < TPR / 2) {
-        float2* qc = C + sk * TM_STRIDE + TM_GAP + s0;
-#pragma unroll
-        for (int j = 0; j < FPT; ++j) {   // conj(cy)
-          qc[2 * j] = s0 + 2 * j < g.Ky ? make_float2(pre[j].x, -pre[j].y) : make_float2(0.f, 0.f);
-          qc[2 * j + 1] = s0 + 2 * j + 1 < g.Ky ? make_float2(pre[j].z, -pre[j].w) : make_float2(0.f, 0.f);
-        }
-        if (sp == 0) meta[sk] = pm;
-      } else {
-        float2* qb = B + sk * TM_STRIDE + TM_GAP + s0;
-        const float2 v = pv;
-#pragma unroll
-        for (int j = 0; j < FPT; ++j) {   // conj(cx) v
-          qb[2 * j] = s0 + 2 * j < g.Kx ? make_float2(pre[j].x * v.x + pre[j].y * v.y, pre[j].x * v.y - pre[j].y * v.x)
-                                        : make_float2(0.f, 0.f);
-          qb[2 * j + 1] = s0 + 2 * j + 1 < g.Kx
-                              ? make_float2(pre[j].z * v.x + pre[j].w * v.y, pre[j].z * v.y - pre[j].w * v.x)
-                              : make_float2(0.f, 0.f);
-        }
-      }
-    }
-    __syncthreads();
-    // this wave's rows (window meets its quadrant), listed as the slot
-    // offsets of lane 0's reads: C at row + qy0 - dy, B at row + qx0 - dx
-    int nh = 0;
-    for (int b0 = 0; b0 < n; b0 += 64) {
-      const int k = b0 + lane;
-      bool hit = false;
-      int e = 0;
-      if (k < n) {
-        const int m = meta[k];
-        const int dy = (m & 0xff) - 32, dx = ((m >> 8) & 0xff) - 32;
-        hit = dy < qy0 + 16 && dy + g.Ky > qy0 && dx < qx0 + 16 && dx + g.Kx > qx0;
-        const int base = k * TM_STRIDE + TM_GAP;
-        e = (base + qy0 - dy) | ((base + qx0 - dx) << 16);
-      }
-      const unsigned long long mask = __ballot(hit);
-      const int pos = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
-      if (hit) mine[nh + pos] = e;
-      nh += __popcll(mask);
-    }
-    // rows missing from the last group of four read the leading zero gap
-    if (lane < 3) mine[nh + lane] = 0;
-    __syncthreads();
-    if (c0 + CH < it.z) fetch(c0 + CH);
-    // rank-1 updates, two rows per instruction pair and two pairs per step
-    // (their LDS reads issued together): A lane (i, k) holds re / im (k
-    // even / odd) of C at its row's offset + i, B lane (j, k) the matching
-    // re / -im or im / re of B, so cre += Re(C B^T), cim += Im(C B^T)
-    for (int p = 0; p < nh; p += 4) {
-      const int e0 = mine[p + half], e1 = mine[p + 2 + half];
-      const float2 c0 = C[(e0 & 0xffff) + li], b0 = B[(e0 >> 16) + li];
-      const float2 c1 = C[(e1 & 0xffff) + li], b1 = B[(e1 >> 16) + li];
-      cre = __builtin_amdgcn_mfma_f32_16x16x4f32(odd ? c0.y : c0.x, odd ? -b0.y : b0.x, cre, 0, 0, 0);
-      cim = __builtin_amdgcn_mfma_f32_16x16x4f32(odd ? c0.y : c0.x, odd ? b0.x : b0.y, cim, 0, 0, 0);
-      cre2 = __builtin_amdgcn_mfma_f32_16x16x4f32(odd ? c1.y : c1.x, odd ? -b1.y : b1.x, cre2, 0, 0, 0);
-      cim2 = __builtin_amdgcn_mfma_f32_16x16x4f32(odd ? c1.y : c1.x, odd ? b1.x : b1.y, cim2, 0, 0, 0);
-    }
-  }
-  cre += cre2;   // the two pairs' chains (four independent accumulators in the loop)
-  cim += cim2;
-  // lane (j, k) holds rows 4k .. 4k + 3 of column j of the quadrant
-  const int lx = qx0 + li, ly0 = qy0 + 4 * (lane >> 4);
-  if (it.w >= 0) {   // one of several items of this tile: partial sums
-    float2* part = g.partial + (size_t)it.w * (TILE_Y * TILE_X) + lx * TILE_Y + ly0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) part[r] = make_float2(cre[r], cim[r]);
-    return;
-  }
-  float2* o = out + (size_t)(tx * TILE_X + lx) * g.Kty + ty * TILE_Y + ly0;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) o[r] = make_float2(cre[r], cim[r]);
+// value of lane P of this lane's row of 16 (one DPP move, no LDS).  Used in sums
+// only: folded into a subtraction (v_subrev_u32_dpp) it was read from the
+// other operand.
+template <int P>
+__device__ __forceinline__ int row_bcast(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, 0x150 + P, 0xf, 0xf, true);   // row_newbcast:P
 }
 
-// ---- the cell-indexed gather (8-slot rows) ----
-
-struct TileView {
-  float2* qc;
-  int* cell;
-  int* start;
-  int stride;
+// Rows of a patch staged at a time by its wave, in LDS of its own: cy of each
+// slot, and conj(cx) w as the two B operands of re / im (k even: q.re, q.im;
+// k odd: q.im, -q.re), with a zero slot behind each row.
+constexpr int PR = 16;
+template <int KM>
+struct PatchStage {
+  float4 b[PR][KM + 1];
+  float2 a[PR][KM + 1];
 };
 
-__device__ __forceinline__ TileView tile_view(const GDev& g, unsigned char* lds) {
-  TileView v;
-  v.stride = g.Ky + g.Kx + 1;
-  v.qc = reinterpret_cast<float2*>(lds);
-  v.cell = reinterpret_cast<int*>(lds + (size_t)TILE_GCH * v.stride * 8);
-  v.start = v.cell + TILE_GCH + ADJ_THREADS / 64;   // cell[TILE_GCH], scan scratch, start
-  return v;
-}
-
-// a[c] = min(a[c], a[c+1], ..., a[n-1]) for c < n, by the ADJ_THREADS
-// threads of the workgroup (each owns a contiguous segment); wsum: LDS
-// scratch of ADJ_THREADS / 64 ints.  Ends with a barrier.
-template <int KM>
-__device__ __forceinline__ void tile_suffix_min(int* a, int n, int* wsum) {
-  constexpr int PER = (tile_cells_max<KM>() + 1 + ADJ_THREADS - 1) / ADJ_THREADS;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  int v[PER];
-  int m = 0x7fffffff;
-#pragma unroll
-  for (int j = PER - 1; j >= 0; --j) {
-    const int idx = t * PER + j;
-    if (idx < n) m = min(m, a[idx]);
-    v[j] = m;
+// Sums the n listed rows of one job: lane (j, g) gets rows 4g .. 4g + 3
+// of column j.
+// Chunks of PR rows: the row lines come in as 16-byte words (a load of 64
+// scattered slots takes 16 address cycles, three per pair of rows), the next
+// chunk's while this one is multiplied and its entries a chunk earlier.  Lane
+// (i, k) holds the entry of row 2 (i mod 8) + k / 2, so pair p reads its window
+// origins from lane p of its 16 lanes.
+template <int KM, bool HALF, bool LAM>
+__device__ __forceinline__ void patch_mfma(const GDev& g, const int2* __restrict__ entries, int n,
+                                              const float2* __restrict__ wv, const float* __restrict__ lamv,
+                                              PatchStage<KM>& st, mfma_f4& cre, mfma_f4& cim) {
+  constexpr int ROWB = 2 * KM * (HALF ? 4 : 8);   // bytes of a row
+  constexpr int LPR = ROWB / 16, RPI = 64 / LPR;  // lanes per row, rows per load
+  constexpr int NI = PR / RPI;                    // loads per chunk
+  constexpr int SPL = HALF ? 4 : 2;               // slots per lane
+  const int lane = threadIdx.x & 63;
+  const int li = lane & 15, part = (lane >> 4) & 1, half = lane >> 5;
+  const int mine = 2 * (li & 7) + half;
+  const int sub = lane % LPR, rl = lane / LPR, s0 = (sub % (LPR / 2)) * SPL;
+  const bool isb = sub >= LPR / 2;
+  const FHS_GLOBAL char* rows = as_global<char>(g.vals);
+  const FHS_GLOBAL vec2f* w = as_global<vec2f>(wv);
+  const FHS_GLOBAL float* lam = as_global<float>(lamv);
+  const FHS_GLOBAL vec2i* ent = as_global<vec2i>(entries);
+  if (lane < PR) {
+    st.a[lane][KM] = make_float2(0.f, 0.f);
+    st.b[lane][KM] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
-  // inclusive suffix minimum of the segment minima over the lanes of the wave
-  int x = m;
+  // lanes past the end repeat the first row with its window out of reach
+  const int first = ent[0].x;
+  auto entry = [&](int c) {
+    vec2i e = {first, 0xc0c0};   // (dy, dx) = (-64, -64)
+    if (c + mine < n) e = ent[c + mine];
+    return e;
+  };
+  vec4u raw[NI];
+  vec2f v[NI];
+  float lm[NI];
+  auto fetch = [&](int row) {
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_down(x, o, 64);
-    if (lane + o < 64) x = min(x, y);
-  }
-  if (lane == 0) wsum[wv] = x;
-  int ex = __shfl_down(x, 1, 64);
-  if (lane == 63) ex = 0x7fffffff;
-  __syncthreads();
-  for (int u = wv + 1; u < ADJ_THREADS / 64; ++u) ex = min(ex, wsum[u]);
+    for (int t = 0; t < NI; ++t) {
+      const int rr = t * RPI + rl;
+      const int r = __shfl(row, (rr >> 1) + 32 * (rr & 1), 64);
+      raw[t] = *(const FHS_GLOBAL vec4u*)(rows + (size_t)(unsigned)r * ROWB + sub * 16);
+      v[t] = w[r];
+      if constexpr (LAM) lm[t] = lam[r];
+    }
+  };
+  auto stage = [&] {
 #pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    const int idx = t * PER + j;
-    if (idx < n) a[idx] = min(v[j], ex);
-  }
-  __syncthreads();
-}
-
-template <int KM, class W>
-__device__ __forceinline__ void g_adjoint_tile_gather(const GDev& g, int item, W&& w, float2* __restrict__ out,
-                                                      unsigned char* lds) {
-  const TileView s = tile_view(g, lds);
-  const int4 it = g.items[item];
-  if (it.w == -2) {   // a group of empty tiles: zeros
-    for (int e = it.y; e < it.z; ++e) {
-      const int t = g.empty_tiles[e];
-      const int ty = t % g.tiles_y, tx = t / g.tiles_y;
+    for (int t = 0; t < NI; ++t) {
+      const int rr = t * RPI + rl;
+      float2 c[SPL];
+      if constexpr (HALF) {
 #pragma unroll
-      for (int q = 0; q < TILE_PTS; ++q) {
-        const int p = threadIdx.x + q * ADJ_THREADS;
-        out[(size_t)(tx * TILE_X + p / TILE_Y) * g.Kty + ty * TILE_Y + p % TILE_Y] = make_float2(0.f, 0.f);
+        for (int j = 0; j < SPL; ++j) c[j] = h2f(raw[t][j]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < SPL; ++j) c[j] = make_float2(__uint_as_float(raw[t][2 * j]), __uint_as_float(raw[t][2 * j + 1]));
+      }
+      if (isb) {
+        float2 x = make_float2(v[t].x, v[t].y);
+        if constexpr (LAM) x = cscale(x, lm[t]);
+#pragma unroll
+        for (int j = 0; j < SPL; ++j) {
+          const float qx = c[j].x * x.x + c[j].y * x.y, qy = c[j].x * x.y - c[j].y * x.x;
+          st.b[rr][s0 + j] = make_float4(qx, qy, qy, -qx);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < SPL; ++j) st.a[rr][s0 + j] = c[j];
       }
     }
+  };
+  const float* sa = &st.a[half][0].x + part;
+  const float2* sb = reinterpret_cast<const float2*>(&st.b[half][0]) + part;
+  // re += cy.x q.re + cy.y q.im, im += cy.x q.im - cy.y q.re
+  auto pair = [&](auto pc, int ndy, int ndx) {
+    constexpr int P = decltype(pc)::value;
+    const unsigned sy = min((unsigned)(li + row_bcast<P>(ndy)), (unsigned)KM);
+    const unsigned sx = min((unsigned)(li + row_bcast<P>(ndx)), (unsigned)KM);
+    const float a = sa[2 * (P * 2 * (KM + 1) + sy)];
+    const float2 b = sb[2 * (P * 2 * (KM + 1) + sx)];
+    cre = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b.x, cre, 0, 0, 0);
+    cim = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b.y, cim, 0, 0, 0);
+  };
+  vec2i cur = entry(0), nxt = entry(PR);
+  fetch(cur.x);
+  for (int c = 0; c < n; c += PR) {
+    __builtin_amdgcn_wave_barrier();
+    stage();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int ndy = -(int)(signed char)(cur.y & 0xff), ndx = -(int)(signed char)((cur.y >> 8) & 0xff);
+    const int rem = n - c;
+    if (rem > PR) {
+      cur = nxt;
+      fetch(cur.x);
+      nxt = entry(c + 2 * PR);
+    }
+    pair(std::integral_constant<int, 0>{}, ndy, ndx);
+    pair(std::integral_constant<int, 1>{}, ndy, ndx);
+    if (rem <= 4) break;
+    pair(std::integral_constant<int, 2>{}, ndy, ndx);
+    pair(std::integral_constant<int, 3>{}, ndy, ndx);
+    if (rem <= 8) break;
+    pair(std::integral_constant<int, 4>{}, ndy, ndx);
+    pair(std::integral_constant<int, 5>{}, ndy, ndx);
+    if (rem <= 12) break;
+    pair(std::integral_constant<int, 6>{}, ndy, ndx);
+    pair(std::integral_constant<int, 7>{}, ndy, ndx);
+    static_assert(PR == 16, "eight pairs a chunk");
+  }
+}
+
+// The same sums tap by tap (the lane's four points, rows in list order).
+struct PatchSums {
+  mfma_f4 re, im;
+};
+template <int KM, class W>
+__device__ __noinline__ PatchSums patch_exact(const GDev& g, const int2* __restrict__ ent, int n, W w) {
+  const int lane = threadIdx.x & 63, li = lane & 15, y0 = 4 * (lane >> 4);
+  auto slot = [&](int r, int j) {
+    const size_t i = (size_t)r * (2 * KM) + j;
+    return g.half ? h2f(reinterpret_cast<const unsigned*>(g.vals)[i]) : g.vals[i];
+  };
+  mfma_f4 cre = {0.f, 0.f, 0.f, 0.f}, cim = cre;
+  for (int e = 0; e < n; ++e) {
+    const int r = ent[e].x, pk = ent[e].y;
+    const int dy = (int)(signed char)(pk & 0xff), dx = (int)(signed char)((pk >> 8) & 0xff);
+    const int jx = li - dx;
+    if ((unsigned)jx >= (unsigned)g.Kx) continue;
+    const float2 v = w(r), c = slot(r, KM + jx);
+    const float2 q = make_float2(c.x * v.x + c.y * v.y, c.x * v.y - c.y * v.x);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int jy = y0 + i - dy;
+      if ((unsigned)jy < (unsigned)g.Ky) {
+        const float2 a = slot(r, jy);
+        cre[i] += a.x * q.x + a.y * q.y;
+        cim[i] += a.x * q.y - a.y * q.x;
+      }
+    }
+  }
+  return {cre, cim};
+}
+
+// Four jobs, one per wave.
+template <int KM, bool LAM>
+__device__ __forceinline__ void g_adjoint_patches(const GDev& g, int unit, const float2* __restrict__ w,
+                                                  const float* __restrict__ lam, float2* __restrict__ out) {
+  __shared__ PatchStage<KM> stages[ADJ_THREADS / 64];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = unit * (ADJ_THREADS / 64) + wv;
+  if (j >= g.njobs) return;
+  const int4 job = g.jobs[j];
+  const int patch = __builtin_amdgcn_readfirstlane(job.x), e0 = __builtin_amdgcn_readfirstlane(job.y);
+  const int n = __builtin_amdgcn_readfirstlane(job.z), slot = __builtin_amdgcn_readfirstlane(job.w);
+  // a patch leaves as 16-byte words, 8 lanes to a column of 16 points, so whole
+  // 128-byte lines are written
+  auto put = [&](float2* o, size_t stride, vec4f v0, vec4f v1) {
+    FHS_GLOBAL char* q = (FHS_GLOBAL char*)(o + (lane >> 3) * stride + 2 * (lane & 7));
+    *(FHS_GLOBAL vec4f_a8*)q = v0;
+    *(FHS_GLOBAL vec4f_a8*)(q + 8 * stride * sizeof(float2)) = v1;
+  };
+  auto at = [&](int p) {
+    const int py = p % g.patches_y, px = p / g.patches_y;
+    return out + (size_t)(px * PATCH) * g.Kty + py * PATCH;
+  };
+  if (slot == -2) {
+    const vec4f zero = {0.f, 0.f, 0.f, 0.f};
+    for (int e = e0; e < e0 + n; ++e) put(at(g.empty[e]), g.Kty, zero, zero);
     return;
   }
-  const int t = it.x;
-  const int ty = t % g.tiles_y, tx = t / g.tiles_y;
-  const int ncy = TILE_Y + g.Ky - 1, ncx = TILE_X + g.Kx - 1, ncells = ncy * ncx;
-  const int p0 = it.y, p1 = it.z;
-  float2 acc[TILE_PTS];
-#pragma unroll
-  for (int i = 0; i < TILE_PTS; ++i) acc[i] = make_float2(0.f, 0.f);
-  // the next chunk's row index and cell are loaded one chunk ahead, so the
-  // row-indexed loads of a chunk do not wait behind the index load
-  const int i = threadIdx.x;
-  int r_next = 0, cell_next = 0;
-  if (p0 + i < p1) {
-    r_next = g.tile_rows[p0 + i];
-    cell_next = g.tile_cell[p0 + i];
-  }
-  for (int c0 = p0; c0 < p1; c0 += TILE_GCH) {
-    const int n = min(TILE_GCH, p1 - c0);
-    const int r = r_next, rcell = cell_next;
-    if (c0 + TILE_GCH + i < p1) {
-      r_next = g.tile_rows[c0 + TILE_GCH + i];
-      cell_next = g.tile_cell[c0 + TILE_GCH + i];
-    }
-    if (i < n) {
-      const float2 v = w(r);
-      float2 cy[KM], cx[KM];
-      sep_load<KM>(g, r, cy, cx);
-      float2* q = s.qc + (size_t)i * s.stride;
-#pragma unroll
-      for (int j = 0; j < KM; ++j) {
-        if (j < g.Kx) {
-          const float2 c = cx[j];
-          q[j] = make_float2(c.x * v.x + c.y * v.y, c.x * v.y - c.y * v.x);   // conj(c) v
-        }
-        if (j < g.Ky) q[g.Kx + j] = make_float2(cy[j].x, -cy[j].y);
-      }
-      s.cell[i] = rcell;
-    }
-    for (int c = threadIdx.x; c <= ncells; c += ADJ_THREADS) s.start[c] = n;
-    __syncthreads();
-    // start[c] = first staged row with cell >= c: the first row of every
-    // occupied cell marks it, then a block-wide suffix minimum fills the rest
-    if (i < n && (i == 0 || s.cell[i - 1] != s.cell[i])) s.start[s.cell[i]] = i;
-    __syncthreads();
-    tile_suffix_min<KM>(s.start, ncells + 1, s.cell + TILE_GCH);
-    // occupied cell columns of this chunk (cells are sorted, x-major)
-    const int cxmin = s.cell[0] / ncy, cxmax = s.cell[n - 1] / ncy;
-#pragma unroll
-    for (int q = 0; q < TILE_PTS; ++q) {
-      const int p = threadIdx.x + q * ADJ_THREADS;
-      const int ly = p % TILE_Y, lx = p / TILE_Y;
-      float2 a = acc[q];
-      const int jx0 = max(0, lx + g.Kx - 1 - cxmax), jx1 = min(g.Kx - 1, lx + g.Kx - 1 - cxmin);
-      for (int jx = jx0; jx <= jx1; ++jx) {
-        const int base = (lx + g.Kx - 1 - jx) * ncy;
-        const int k0 = s.start[base + ly], k1 = s.start[base + ly + g.Ky];
-        for (int k = k0; k < k1; ++k) {
-          const int jy = ly + g.Ky - 1 - (s.cell[k] - base);
-          const float2* qq = s.qc + (size_t)k * s.stride;
-          const float2 cy = qq[g.Kx + jy], qx = qq[jx];
-          a.x += cy.x * qx.x - cy.y * qx.y;
-          a.y += cy.x * qx.y + cy.y * qx.x;
-        }
-      }
-      acc[q] = a;
-    }
-    __syncthreads();
-  }
-  if (it.w >= 0) {   // one of several items of this tile: partial sums
-    float2* part = g.partial + (size_t)it.w * (TILE_Y * TILE_X);
-#pragma unroll
-    for (int q = 0; q < TILE_PTS; ++q) part[threadIdx.x + q * ADJ_THREADS] = acc[q];
-    return;
-  }
-#pragma unroll
-  for (int q = 0; q < TILE_PTS; ++q) {
-    const int p = threadIdx.x + q * ADJ_THREADS;
-    const int ly = p % TILE_Y, lx = p / TILE_Y;
-    out[(size_t)(tx * TILE_X + lx) * g.Kty + ty * TILE_Y + ly] = acc[q];
-  }
-}
-
-
-template <int KM, class W>
-__device__ __forceinline__ void g_adjoint_tile(const GDev& g, int item, W&& w, float2* __restrict__ out,
-                                               unsigned char* lds) {
-  if constexpr (KM > 8)
-    g_adjoint_tile_mfma<KM>(g, item, w, out, lds);
+  mfma_f4 cre = {0.f, 0.f, 0.f, 0.f}, cim = cre;
+  const int2* __restrict__ ent = g.pent + e0;
+  if (g.half)
+    patch_mfma<KM, true, LAM>(g, ent, n, w, lam, stages[wv], cre, cim);
   else
-    g_adjoint_tile_gather<KM>(g, item, w, out, lds);
+    patch_mfma<KM, false, LAM>(g, ent, n, w, lam, stages[wv], cre, cim);
+  bool bad = false;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) bad = bad || !isfinite(cre[r]) || !isfinite(cim[r]);
+  if (__any(bad)) {
+    auto wr = [=](int r) { return LAM ? cscale(w[r], lam[r]) : w[r]; };
+    const PatchSums e = patch_exact<KM>(g, ent, n, wr);
+    cre = e.re;
+    cim = e.im;
+  }
+  // lane (i, k) holds points 4k .. 4k + 3 of column i: transposed through LDS
+  static_assert(sizeof(PatchStage<KM>) >= PATCH * PATCH * sizeof(float2), "a patch fits the stage");
+  vec4f* t = reinterpret_cast<vec4f*>(&stages[wv]);
+  __builtin_amdgcn_wave_barrier();
+  t[(lane & 15) * 8 + 2 * (lane >> 4)] = vec4f{cre[0], cim[0], cre[1], cim[1]};
+  t[(lane & 15) * 8 + 2 * (lane >> 4) + 1] = vec4f{cre[2], cim[2], cre[3], cim[3]};
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (slot >= 0)
+    put(g.partial + (size_t)slot * (PATCH * PATCH), PATCH, t[lane], t[lane + 64]);
+  else
+    put(at(patch), g.Kty, t[lane], t[lane + 64]);
 }
 
-// sum of the partial tiles of split tile r, in slot order
-__device__ __forceinline__ void g_adjoint_tile_reduce(const GDev& g, int r, float2* __restrict__ out) {
+// sum of the partial patches of split patch r, in slot order (one point per thread)
+__device__ __forceinline__ void g_adjoint_reduce(const GDev& g, int r, float2* __restrict__ out) {
+  static_assert(ADJ_THREADS == PATCH * PATCH, "one point per thread");
   const int4 rd = g.red[r];
-  const int t = rd.x, ty = t % g.tiles_y, tx = t / g.tiles_y;
-#pragma unroll
-  for (int q = 0; q < TILE_PTS; ++q) {
-    const int p = threadIdx.x + q * ADJ_THREADS;
-    float2 a = make_float2(0.f, 0.f);
-    for (int j = 0; j < rd.z; ++j) a = cadd(a, g.partial[(size_t)(rd.y + j) * (TILE_Y * TILE_X) + p]);
-    out[(size_t)(tx * TILE_X + p / TILE_Y) * g.Kty + ty * TILE_Y + p % TILE_Y] = a;
-  }
+  const int py = rd.x % g.patches_y, px = rd.x / g.patches_y, p = threadIdx.x;
+  const float2* part = g.partial + (size_t)rd.y * (PATCH * PATCH) + p;
+  float2 a = make_float2(0.f, 0.f);
+  for (int j = 0; j < rd.z; ++j) a = cadd(a, part[(size_t)j * (PATCH * PATCH)]);
+  out[(size_t)(px * PATCH + p / PATCH) * g.Kty + py * PATCH + p % PATCH] = a;
 }
+
 // Forward (degridding) of one work item: the (TILE_Y + Ky - 1) x (TILE_X +
 // Kx - 1) grid window of the tile is staged in LDS once (all loads issued
 // before the stores), then every row of the item reads its Ky x Kx taps from
