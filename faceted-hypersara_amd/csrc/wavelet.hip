@@ -9,15 +9,8 @@
 // lf): out[k] = sum_j f[j] in[2k + 2 - lf + j], n_out = floor((n + lf - 1)/2).
 // a = lo_y lo_x, h = hi_y lo_x, v = lo_y hi_x, d = hi_y hi_x (y = rows).
 //
-// Kernels work on output tiles (analysis 32 x 16, synthesis 32 x 32): the
-// input window (plus filter halo) is staged in LDS, filtered along x then y
-// (separable, 2 lf FMAs per output).  Analysis runs one workgroup per (tile,
-// basis, channel) at every level; its 32 x 16 tiles keep the LDS at 24 KB,
-// so five workgroups fit on a CU instead of three with 32 x 32 tiles (one
-// workgroup per tile running all the bases from one image window measured
-// slower: the bases then run one after the other).  Synthesis mirrors the analysis,
-// and its finest level sums all bases and the Dirac part in registers so the
-// image is written once.
+// Both directions run one wave per tile on registers and LDS of its own (see
+// k_analysis and k_synthesis); the l21 step is part of the analysis.
 #include <algorithm>
 #include <cmath>
 
@@ -29,8 +22,6 @@ namespace fhs {
 constexpr int WMAX_BASES = 8;
 constexpr int WMAX_LEVELS = 6;
 constexpr int WMAX_LF = 16;
-constexpr int WT = 32;           // output tile edge
-constexpr int WTHREADS = 256;
 
 struct SaraGeom {
   int Ny, Nx, nlevel, nb, dirac;
@@ -44,8 +35,7 @@ struct SaraGeom {
   int64_t scr[WMAX_BASES][WMAX_LEVELS + 1];   // scratch offset of approx level k (per channel)
   int64_t scr_per_chan;
   int64_t s;                             // coefficients per channel
-  float lo[WMAX_BASES][WMAX_LF];
-  float hi[WMAX_BASES][WMAX_LF];
+  float lo[WMAX_BASES][WMAX_LF];         // reconstruction low-pass; high-pass (-1)^j lo[lf - 1 - j]
 };
 
 }  // namespace fhs
@@ -53,190 +43,360 @@ struct SaraGeom {
 struct fhs_sara {
   int device = 0;
   fhs::SaraGeom g{};
+  fhs::SaraGeom* d = nullptr;   // device copy: the kernels' few fields come from L2, not from the 1 KB of arguments
 };
 
 namespace fhs {
 namespace {
 
-// ---- analysis of one T x T output tile from an LDS window -----------------
-// win: window origin at input (wy0, wx0), height WH (column-major: [x][y]);
-// the basis' own window starts at offset o (longest-filter window at level 1).
-struct AnOut {
-  float* v1;          // channel vector (coefficients accumulate here)
-  float* approx;      // scratch for A_k (nullptr at the last level)
-  int64_t a_off;      // offset of A_k in approx (or of A_J in v1 at the last level)
-  int64_t h_off;      // offset of H_k in v1 (V, D follow)
-  int ny, nx;         // output level shape
-  bool last;
+// ---- analysis -----------------------------------------------------------------
+// One wave transforms one tile of AT_Y x AT_X outputs of a level, basis and
+// channel.  Its input window has at most 2 AT_Y + 14 = 126 rows: lane r reads the
+// 2 AT_X + lf - 2 values of rows r and r + 64 along x straight from memory, 64
+// consecutive floats a load, so the x filter runs on registers (an earlier form
+// staged the window in LDS and read every tap of every output from there).  The
+// two x-filtered halves turn through LDS of the wave's own, even and odd rows
+// apart, and lane ky filters along y; its accesses to v1 are again 56
+// consecutive floats.  A workgroup's waves hold the channels of one tile, so the
+// norms of the l21 step over the channels close inside it: analysis, threshold
+// and dual update read and write v1 once, not twice.  One channel a wave, and one
+// column address per array with the columns as lane offsets: four channels a wave
+// and an address per column spilled 200 scalar registers into lanes, which
+// doubled the instructions (level 1 of 16 channels of 1024 x 1024: 508 us, 411 us
+// in this form).  What bounds it there: 1024-thread workgroups of 80 registers, one
+// on a CU, whose load and filter phases do not overlap.
+constexpr int AT_Y = 56, AT_X = 4;
+constexpr int AT_LD = 96;                 // LDS stride of the 63 rows of a parity: even and odd rows in other banks
+constexpr int AT_PAIR = 2;                // columns in the turning tile at a time
+constexpr int AT_LH = 4 * AT_PAIR * AT_LD;   // floats of a wave's turning tile
+constexpr int AN_CHANNELS = 16;           // waves of a workgroup at most
+
+// hi[j] = (-1)^j lo[lf - 1 - j]: one set of taps in scalar registers serves both
+// filters
+template <int LF>
+struct Taps {
+  float f[LF];
+  __device__ __forceinline__ float lo(int j) const { return f[j]; }
+  __device__ __forceinline__ float hi(int j) const { return j & 1 ? -f[LF - 1 - j] : f[LF - 1 - j]; }
 };
-
-// analysis tiles: AY x AX outputs (rows x columns)
-constexpr int AY = 32, AX = 16;
-constexpr int AN_PER = AY * AX / WTHREADS;   // outputs per thread
-
-// old values of the coefficients a tile accumulates into (+=), loaded at
-// kernel start so that their latency overlaps the window load
-struct AnPre {
-  float a[AN_PER], h[AN_PER], v[AN_PER], d[AN_PER];
-};
-
-__device__ __forceinline__ void an_prefetch(int ky0, int kx0, const AnOut& out, AnPre& pre) {
+template <int LF>
+__device__ __forceinline__ Taps<LF> load_taps(const SaraGeom& G, int b) {
+  Taps<LF> t;
 #pragma unroll
-  for (int q = 0; q < AN_PER; ++q) {
-    const int t = threadIdx.x + q * WTHREADS;
-    const int gy = ky0 + t % AY, gx = kx0 + t / AY;
-    pre.a[q] = pre.h[q] = pre.v[q] = pre.d[q] = 0.f;
-    if (gy < out.ny && gx < out.nx) {
-      const int64_t p = gy + (int64_t)out.ny * gx;
-      const int64_t sz = (int64_t)out.ny * out.nx;
-      if (out.last) pre.a[q] = out.v1[out.a_off + p];
-      pre.h[q] = out.v1[out.h_off + p];
-      pre.v[q] = out.v1[out.h_off + sz + p];
-      pre.d[q] = out.v1[out.h_off + 2 * sz + p];
-    }
-  }
+  for (int j = 0; j < LF; ++j) t.f[j] = G.lo[b][j];
+  return t;
+}
+// element `off` bytes behind a wave-uniform base
+__device__ __forceinline__ float& at_bytes(float* base, unsigned off) {
+  return *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + off);
+}
+__device__ __forceinline__ float at_bytes(const float* base, unsigned off) {
+  return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + off);
 }
 
-template <int LF>
-__device__ void an_tile_t(const float* win, int WH, const float* lo, const float* hi, int ky0, int kx0, float* Lx,
-                          float* Hx, const AnOut& out, const AnPre& pre) {
-  constexpr int H = 2 * AY + LF - 2;   // rows of the window
-  float rlo[LF], rhi[LF];
+// what becomes of the coefficients c
+enum AnMode {
+  AN_ADD = 0,      // v1 += c
+  AN_SET = 1,      // v1 = c
+  AN_L21 = 2,      // r = v1 + c over the channels, v1 = r - max(|r| - beta w, 0) / (|r| + eps) r
+  AN_WEIGHT = 3,   // wout = beta / (beta + |c|)
+  AN_NORM = 4      // part[workgroup] = sum of |c|
+};
+
+struct AnArgs {
+  const float* x;        // image cube, the input of level 1
+  float* scr;            // A_1 .. A_{J-1} of the bases and channels
+  float* v1;
+  const float* w;
+  double beta;
+  float* wout;
+  double* part;
+  int L, k;
+};
+
+// the l21 factor of a coefficient with norm sqrt(ss): v1 = r - f r
+__device__ __forceinline__ float l21_factor(double ss, double t) {
+  const double l2 = sqrt(ss);
+  return (float)(fmax(l2 - t, 0.0) / (l2 + 2.220446049250313e-16));
+}
+
+template <int LF, int MODE, bool LAST>
+__device__ __forceinline__ void an_tile(const SaraGeom& G, const AnArgs& A, int b, int ky0, int kx0, float* lds) {
+  constexpr int NS = LAST ? 4 : 3;        // subbands kept as coefficients: h, v, d (and a)
+  constexpr int NQ = NS * AT_X;           // coefficients per lane
+  constexpr int WW = 2 * AT_X + LF - 2;   // window columns
+  constexpr bool NORMS = MODE >= AN_L21;
+  const int lane = threadIdx.x & 63, l = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave = channel
+  const int k = A.k, iny = G.ny[b][k - 1], inx = G.nx[b][k - 1], ny = G.ny[b][k], nx = G.nx[b][k];
+  const int64_t sz = (int64_t)ny * nx;
+  const Taps<LF> T = load_taps<LF>(G, b);
+  const bool live = lane < AT_Y && ky0 + lane < ny;
+  const int ncol = min(AT_X, nx - kx0);
+  // offsets of the kept subbands in a channel vector, of the tile, of this lane
+  const int64_t hoff = G.boff[b] + G.doff[b][k], toff = ky0 + (int64_t)ny * kx0;
+  auto soff = [&](int s) { return s == 3 ? G.boff[b] + G.aoff[b] : hoff + s * sz; };
+  const unsigned loff = (unsigned)lane * sizeof(float), cstep = (unsigned)ny * sizeof(float);
+  float* v1 = A.v1 + (int64_t)l * G.s + toff;
+  // r: old coefficients, then plus the new ones (r[3]: the approximation, a coefficient
+  // only at the last level)
+  float r[4][AT_X];
 #pragma unroll
-  for (int j = 0; j < LF; ++j) {
-    rlo[j] = lo[j];
-    rhi[j] = hi[j];
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int q = 0; q < AT_X; ++q) r[s][q] = 0.f;
+  if ((MODE == AN_ADD || MODE == AN_L21) && live) {
+#pragma unroll
+    for (int q = 0; q < AT_X; ++q)
+      if (q < ncol) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) r[s][q] = at_bytes(v1 + soff(s), loff + q * cstep);
+      }
   }
-  // x pass: Lx[kx][r], Hx[kx][r] for r < H, kx < AX
-  for (int t = threadIdx.x; t < H * AX; t += WTHREADS) {
-    const int r = t % H, kx = t / H;
-    float sl = 0.f, sh = 0.f;
-    const float* col = win + (size_t)(2 * kx) * WH + r;
+  float wc = 1.f;   // the threshold weight of the coefficient this thread finishes below
+  auto coef = [&](int e, int64_t& c) {
+    const int i = e >> 6, ln = e & 63, s = i / AT_X, q = i % AT_X;
+    c = soff(s) + toff + (int64_t)ny * q + ln;
+    return q < ncol && ln < AT_Y && ky0 + ln < ny;
+  };
+  if (MODE == AN_L21 && A.w) {
+    int64_t c;
+    if (threadIdx.x < NQ * 64 && coef(threadIdx.x, c)) wc = A.w[c];
+  }
+  // x filter of rows lane and lane + 64
+  float lw[2][AT_X], hg[2][AT_X];
+  {
+    const int wy0 = 2 * ky0 + 2 - LF, wx0 = 2 * kx0 + 2 - LF;
+    const float* img = (k == 1 ? A.x + (int64_t)l * iny * inx : A.scr + (int64_t)l * G.scr_per_chan + G.scr[b][k - 1]) +
+                       (int64_t)iny * wx0;
+    const float scale = k == 1 ? G.norm : 1.f;
+    const bool inside = wx0 >= 0 && wx0 + WW <= inx;
 #pragma unroll
-    for (int j = 0; j < LF; ++j) {
-      const float w = col[(size_t)j * WH];
-      sl += rlo[j] * w;
-      sh += rhi[j] * w;
+    for (int hh = 0; hh < 2; ++hh) {
+      const int row = lane + 64 * hh, wy = wy0 + row;
+      const unsigned off = (unsigned)wy * sizeof(float), step = (unsigned)iny * sizeof(float);
+      float win[WW];
+#pragma unroll
+      for (int c = 0; c < WW; ++c) win[c] = 0.f;
+      if (wy >= 0 && wy < iny && row < 2 * AT_Y + LF - 2) {
+        if (inside) {
+#pragma unroll
+          for (int c = 0; c < WW; ++c) win[c] = at_bytes(img, off + c * step);
+        } else {
+#pragma unroll
+          for (int c = 0; c < WW; ++c)
+            if (wx0 + c >= 0 && wx0 + c < inx) win[c] = at_bytes(img, off + c * step);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < AT_X; ++q) {
+        float sl = 0.f, sh = 0.f;
+#pragma unroll
+        for (int j = 0; j < LF; ++j) {
+          sl += T.lo(j) * win[2 * q + j];
+          sh += T.hi(j) * win[2 * q + j];
+        }
+        lw[hh][q] = sl * scale;
+        hg[hh][q] = sh * scale;
+      }
     }
-    Lx[kx * H + r] = sl;
-    Hx[kx * H + r] = sh;
   }
-  __syncthreads();
-  // y pass
+  // y filter, AT_PAIR columns at a time: output ky0 + lane from rows 2 lane .. 2 lane + LF - 1
+  float* lh = lds + l * AT_LH;
+  float* dst = lh + (lane & 1) * AT_LD + (lane >> 1);   // row lane; row lane + 64 is 32 further
+  const float* src = lh + min(lane, AT_Y - 1);
 #pragma unroll
-  for (int q = 0; q < AN_PER; ++q) {
-    const int t = threadIdx.x + q * WTHREADS;
-    const int ky = t % AY, kx = t / AY;
-    const int gy = ky0 + ky, gx = kx0 + kx;
-    if (gy < out.ny && gx < out.nx) {
-      const float* lc = Lx + kx * H + 2 * ky;
-      const float* hc = Hx + kx * H + 2 * ky;
+  for (int q0 = 0; q0 < AT_X; q0 += AT_PAIR) {
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < AT_PAIR; ++q)
+#pragma unroll
+      for (int hh = 0; hh < 2; ++hh) {
+        dst[(4 * q) * AT_LD + 32 * hh] = lw[hh][q0 + q];
+        dst[(4 * q + 2) * AT_LD + 32 * hh] = hg[hh][q0 + q];
+      }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < AT_PAIR; ++q) {
       float a = 0.f, h = 0.f, v = 0.f, d = 0.f;
 #pragma unroll
       for (int j = 0; j < LF; ++j) {
-        a += rlo[j] * lc[j];
-        h += rhi[j] * lc[j];
-        v += rlo[j] * hc[j];
-        d += rhi[j] * hc[j];
+        const float xl = src[(4 * q + (j & 1)) * AT_LD + j / 2], xh = src[(4 * q + 2 + (j & 1)) * AT_LD + j / 2];
+        a += T.lo(j) * xl;
+        h += T.hi(j) * xl;
+        v += T.lo(j) * xh;
+        d += T.hi(j) * xh;
       }
-      const int64_t p = gy + (int64_t)out.ny * gx;
-      const int64_t sz = (int64_t)out.ny * out.nx;
-      if (out.last)
-        out.v1[out.a_off + p] = pre.a[q] + a;
-      else
-        out.approx[out.a_off + p] = a;
-      out.v1[out.h_off + p] = pre.h[q] + h;
-      out.v1[out.h_off + sz + p] = pre.v[q] + v;
-      out.v1[out.h_off + 2 * sz + p] = pre.d[q] + d;
+      r[0][q0 + q] += h;
+      r[1][q0 + q] += v;
+      r[2][q0 + q] += d;
+      r[3][q0 + q] += a;
+      // the sums are made here: sunk into the masked stores below, they would keep every
+      // tap's input in registers (and spill)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) asm volatile("" : "+v"(r[s][q0 + q]));
     }
   }
-  __syncthreads();
-}
-
-// filter lengths of db1..db8 are 2, 4, ..., 16: one unrolled instance each
-__device__ void an_tile(const float* win, int WH, int lf, const float* lo, const float* hi, int ky0, int kx0,
-                        float* Lx, float* Hx, const AnOut& out, const AnPre& pre) {
-  switch (lf) {
-    case 2: an_tile_t<2>(win, WH, lo, hi, ky0, kx0, Lx, Hx, out, pre); break;
-    case 4: an_tile_t<4>(win, WH, lo, hi, ky0, kx0, Lx, Hx, out, pre); break;
-    case 6: an_tile_t<6>(win, WH, lo, hi, ky0, kx0, Lx, Hx, out, pre); break;
-    case 8: an_tile_t<8>(win, WH, lo, hi, ky0, kx0, Lx, Hx, out, pre); break;
-    case 10: an_tile_t<10>(win, WH, lo, hi, ky0, kx0, Lx, Hx, out, pre); break;
-    case 12: an_tile_t<12>(win, WH, lo, hi, ky0, kx0, Lx, Hx, out, pre); break;
-    case 14: an_tile_t<14>(win, WH, lo, hi, ky0, kx0, Lx, Hx, out, pre); break;
-    default: an_tile_t<16>(win, WH, lo, hi, ky0, kx0, Lx, Hx, out, pre); break;
-  }
-}
-
-constexpr int WIN_ROWS = 2 * AY + WMAX_LF - 2;   // 78
-constexpr int WIN_COLS = 2 * AX + WMAX_LF - 2;   // 46
-constexpr int WIN_PER_THREAD = (WIN_ROWS * WIN_COLS + WTHREADS - 1) / WTHREADS;
-
-// load window [wy0, wy0+WH) x [wx0, wx0+WW) of a column-major ny x nx image;
-// every load of a thread is issued before the first LDS store, so the
-// window arrives in one memory latency instead of one per element
-__device__ void load_window(float* win, const float* img, int ny, int nx, int wy0, int wx0, int WH,
-                            int WW, float scale) {
-  float v[WIN_PER_THREAD];
-  const int n = WH * WW;
+  if (!LAST && live) {
+    float* ak = A.scr + (int64_t)l * G.scr_per_chan + G.scr[b][k] + toff;
 #pragma unroll
-  for (int i = 0; i < WIN_PER_THREAD; ++i) {
-    const int t = threadIdx.x + i * WTHREADS;
-    v[i] = 0.f;
-    if (t < n) {
-      const int r = t % WH, c = t / WH;
-      const int gy = wy0 + r, gx = wx0 + c;
-      if (gy >= 0 && gy < ny && gx >= 0 && gx < nx) v[i] = img[gy + (int64_t)ny * gx];
+    for (int q = 0; q < AT_X; ++q)
+      if (q < ncol) at_bytes(ak, loff + q * cstep) = r[3][q];
+  }
+  auto put = [&](auto value) {
+    if (live) {
+#pragma unroll
+      for (int q = 0; q < AT_X; ++q)
+        if (q < ncol) {
+#pragma unroll
+          for (int s = 0; s < NS; ++s) at_bytes(v1 + soff(s), loff + q * cstep) = value(s, q);
+        }
+    }
+  };
+  if constexpr (!NORMS) {
+    put([&](int s, int q) { return r[s][q]; });
+  } else {
+    // the channels' values meet in LDS (the turning tiles are done with once every
+    // wave has arrived); thread t finishes coefficients t, t + blockDim, ...
+    const int nw = blockDim.x >> 6;
+    float* vals = lds;                       // [channel][coefficient][lane]
+    float* fac = lds + nw * NQ * 64;
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int q = 0; q < AT_X; ++q) vals[(l * NQ + s * AT_X + q) * 64 + lane] = r[s][q];
+    __syncthreads();
+    double tot[1] = {0.0};
+    for (int e = threadIdx.x; e < NQ * 64; e += blockDim.x) {
+      int64_t c;
+      if (!coef(e, c)) continue;
+      if (MODE == AN_L21 && A.w && e >= (int)blockDim.x) wc = A.w[c];
+      double sq = 0.0;
+      for (int u = 0; u < nw; ++u) {
+        const double t = vals[u * NQ * 64 + e];
+        sq += t * t;
+      }
+      if constexpr (MODE == AN_L21) fac[e] = l21_factor(sq, A.beta * (double)wc);
+      if constexpr (MODE == AN_WEIGHT) A.wout[c] = (float)(A.beta / (A.beta + sqrt(sq)));
+      if constexpr (MODE == AN_NORM) tot[0] += sqrt(sq);
+    }
+    if constexpr (MODE == AN_NORM) {
+      __syncthreads();
+      block_sum<1>(tot, reinterpret_cast<double*>(lds));
+      if (threadIdx.x == 0) A.part[blockIdx.x] = tot[0];
+    }
+    if constexpr (MODE == AN_L21) {
+      __syncthreads();
+      put([&](int s, int q) { return r[s][q] - fac[(s * AT_X + q) * 64 + lane] * r[s][q]; });
     }
   }
-#pragma unroll
-  for (int i = 0; i < WIN_PER_THREAD; ++i) {
-    const int t = threadIdx.x + i * WTHREADS;
-    if (t < n) win[t] = v[i] * scale;
-  }
-  __syncthreads();
 }
 
-__global__ __launch_bounds__(WTHREADS) void k_an_lk(SaraGeom G, int k, const float* __restrict__ x,
-                                                    float* __restrict__ v1, float* __restrict__ scr) {
-  __shared__ float win[WIN_ROWS * WIN_COLS];
-  __shared__ float Lx[AX * WIN_ROWS];
-  __shared__ float Hx[AX * WIN_ROWS];
-  __shared__ float flo[WMAX_LF], fhi[WMAX_LF];
-  const int b = blockIdx.z % G.nb, l = blockIdx.z / G.nb;
-  const int ky0 = blockIdx.x * AY, kx0 = blockIdx.y * AX;
-  if (ky0 >= G.ny[b][k] || kx0 >= G.nx[b][k]) return;
-  const int lf = G.lf[b];
-  if (threadIdx.x < lf) {
-    flo[threadIdx.x] = G.lo[b][threadIdx.x];
-    fhi[threadIdx.x] = G.hi[b][threadIdx.x];
+// Workgroup -> (tile, basis).  The XCDs take contiguous runs of tiles (y
+// fastest), each tile's bases one after the other, so the image window the
+// bases share and the lines two tiles of a column share meet in one L2.
+template <int MODE, bool LAST>
+__global__ __launch_bounds__(64 * AN_CHANNELS) void k_analysis(const SaraGeom* __restrict__ geom, AnArgs A, int ty,
+                                                                int tx) {
+  const SaraGeom& G = *geom;
+  extern __shared__ __align__(16) float an_lds[];
+  const int per = (ty * tx + 7) / 8, s = blockIdx.x / 8;
+  const int tile = (int)(blockIdx.x % 8) * per + s / G.nb, b = s % G.nb;
+  const int ky0 = (tile % ty) * AT_Y, kx0 = (tile / ty) * AT_X;
+  if (s / G.nb >= per || ky0 >= G.ny[b][A.k] || kx0 >= G.nx[b][A.k]) {
+    if (MODE == AN_NORM && threadIdx.x == 0) A.part[blockIdx.x] = 0.0;
+    return;
   }
-  const int WH = 2 * AY + lf - 2, WW = 2 * AX + lf - 2;   // window rows, columns
-  float* sc = scr + (int64_t)l * G.scr_per_chan;
-  AnOut out;
-  out.v1 = v1 + (int64_t)l * G.s;
-  out.last = k == G.nlevel;
-  out.approx = sc;
-  out.a_off = out.last ? G.boff[b] + G.aoff[b] : G.scr[b][k];
-  out.h_off = G.boff[b] + G.doff[b][k];
-  out.ny = G.ny[b][k];
-  out.nx = G.nx[b][k];
-  AnPre pre;
-  an_prefetch(ky0, kx0, out, pre);
-  if (k == 1)   // level 1 reads the image, scaled by 1/sqrt(P)
-    load_window(win, x + (int64_t)l * G.Ny * G.Nx, G.Ny, G.Nx, 2 * ky0 + 2 - lf, 2 * kx0 + 2 - lf, WH, WW,
-                G.norm);
-  else
-    load_window(win, sc + G.scr[b][k - 1], G.ny[b][k - 1], G.nx[b][k - 1], 2 * ky0 + 2 - lf,
-                2 * kx0 + 2 - lf, WH, WW, 1.f);
-  an_tile(win, WH, lf, flo, fhi, ky0, kx0, Lx, Hx, out, pre);
+  switch (G.lf[b]) {   // db1 .. db8: 2, 4, ..., 16 taps
+    case 2: an_tile<2, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
+    case 4: an_tile<4, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
+    case 6: an_tile<6, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
+    case 8: an_tile<8, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
+    case 10: an_tile<10, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
+    case 12: an_tile<12, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
+    case 14: an_tile<14, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
+    default: an_tile<16, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
+  }
+}
+
+// The Dirac block: r_l = v1_l + x_l / sqrt(P) (v1 absent in AN_WEIGHT, AN_NORM and
+// AN_SET), then as the modes say.  VEC consecutive pixels per thread with wide
+// accesses when the block is 16-byte aligned in every channel.
+template <int MODE, int VEC>
+__global__ __launch_bounds__(256) void k_dirac(SaraGeom G, const float* __restrict__ x, float* __restrict__ v1, int L,
+                                               const float* __restrict__ w, double beta, float* __restrict__ wout,
+                                               double* __restrict__ part) {
+  struct alignas(4 * VEC) Vec {
+    float v[VEC];
+  };
+  constexpr bool KEEP = MODE == AN_ADD || MODE == AN_L21;
+  __shared__ double sh[256 / 64];
+  const int64_t N = (int64_t)G.Ny * G.Nx, d0 = G.boff[G.nb];
+  double tot[1] = {0.0};
+  for (int64_t p = VEC * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x); p < N;
+       p += VEC * (int64_t)gridDim.x * blockDim.x) {
+    constexpr int LREG = 16;   // channels kept in registers between the norm and the update
+    Vec r[LREG];
+    double ss[VEC];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) ss[j] = 0.0;
+#pragma unroll
+    for (int l = 0; l < LREG; ++l)
+      if (l < L) {
+        r[l] = *reinterpret_cast<const Vec*>(x + (int64_t)l * N + p);
+        Vec old;
+        if (KEEP) old = *reinterpret_cast<const Vec*>(v1 + (int64_t)l * G.s + d0 + p);
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+          r[l].v[j] = KEEP ? old.v[j] + r[l].v[j] * G.norm : r[l].v[j] * G.norm;
+          ss[j] += (double)r[l].v[j] * r[l].v[j];
+        }
+      }
+    float f[VEC];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      f[j] = 0.f;
+      if (MODE == AN_L21) f[j] = l21_factor(ss[j], beta * (w ? (double)w[d0 + p + j] : 1.0));
+      if (MODE == AN_WEIGHT) wout[d0 + p + j] = (float)(beta / (beta + sqrt(ss[j])));
+      if (MODE == AN_NORM) tot[0] += sqrt(ss[j]);
+    }
+    if (MODE <= AN_L21) {
+#pragma unroll
+      for (int l = 0; l < LREG; ++l)
+        if (l < L) {
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) r[l].v[j] -= f[j] * r[l].v[j];
+          *reinterpret_cast<Vec*>(v1 + (int64_t)l * G.s + d0 + p) = r[l];
+        }
+    }
+  }
+  if (MODE == AN_NORM) {
+    block_sum<1>(tot, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = tot[0];
+  }
 }
 
 // ---- synthesis -------------------------------------------------------------
-// Output tile [iy0, iy0+WT) x [ix0, ix0+WT) of the finer level (shape py x px)
-// from the four subbands of level k (shape ny x nx).  Coefficient rows that
-// reach the tile: k in [ceil((i0-1)/2), floor((i0+WT-1+lf-2)/2)].
-constexpr int CMAX = WT / 2 + WMAX_LF / 2 + 1;   // 25
+// One wave makes one tile of ST_Y x ST_X pixels of the finer level from the four
+// subbands of level k.  Output i takes the lf / 2 coefficients floor(i / 2) + m with
+// filter tap (i & 1) + lf - 2 - 2 m, so both pixels of a parity pair share their
+// coefficients.  Lane r holds coefficient row r of the tile (at most 56 + 7) and
+// reads the 3 + lf / 2 columns of each subband straight from memory, 64 consecutive
+// floats a load; the x filter runs on those registers (finest level of 16 channels
+// of 1024 x 1024: 410 us staged, 201 us).  The two half-filtered images turn through LDS of the wave's own and lane (ix, g) filters along y the
+// 14 rows 14 g .. 14 g + 13 of column ix, keeping the sum over the bases in
+// registers at the finest level (the image is written once).  No barrier: an
+// earlier form staged 32 x 32 tiles in LDS, whose column segments of 18 to 25
+// coefficients used half of the lines they touched.
+constexpr int ST_Y = 112, ST_X = 8;
+constexpr int ST_WAVES = 4;                       // tiles per workgroup
+constexpr int ST_PER = ST_Y * ST_X / 64;          // pixels per lane
+constexpr int ST_LD = 66;
+// A tile's bases run one after the other; below this many tiles x channels the chip
+// is not full and the four waves of a workgroup share a tile's bases instead (finest
+// level of SARA 256 x 256, 96 tiles: 22 us in 32 x 32 tiles, 9 us split).
+constexpr int64_t SYN_SPLIT_BELOW = 2048;
 
 struct SynIn {
   const float* a;   // approx of level k (column-major ny x nx)
@@ -244,359 +404,185 @@ struct SynIn {
   int ny, nx;
 };
 
-// A synthesis tile in three steps, so that a caller can overlap the global
-// loads of the next tile with the arithmetic of the current one:
-//   syn_load_t   issues the loads of the 4 subband tiles (CN x CN) into registers,
-//   syn_store_t  writes them to LDS (cs[s][cx][cy]; a barrier must follow),
-//   syn_compute_t accumulates the tile (WT*WT/WTHREADS values per thread, placed
-//                 as syn_acc_coord says) into acc.
-// Output i takes the LF/2 coefficients k = floor(i/2) + m (m < LF/2) with
-// filter tap j = (i & 1) + LF - 2 - 2m; the staged tile is zero beyond the
-// subband, so no clamping is needed.
-constexpr int CS_MAX = (4 * CMAX * CMAX + WTHREADS - 1) / WTHREADS;   // registers per thread
-
 template <int LF>
-__device__ __forceinline__ void syn_load_t(const SynIn& in, int iy0, int ix0, float* cv) {
-  constexpr int CN = WT / 2 + LF / 2 + 1;
-  constexpr int NCS = 4 * CN * CN;
-  const int cy0 = iy0 / 2, cx0 = ix0 / 2;
-  const int64_t sz = (int64_t)in.ny * in.nx;
+__device__ __forceinline__ void syn_tile(const SaraGeom& G, int b, const SynIn& in, int iy0, int ix0, float* pq,
+                                         float* acc) {
+  constexpr int NC = ST_X / 2 + LF / 2 - 1;
+  const int lane = threadIdx.x & 63;
+  const Taps<LF> T = load_taps<LF>(G, b);
+  const int cy = iy0 / 2 + lane, cx0 = ix0 / 2;
+  const int64_t sz = (int64_t)in.ny * in.nx, toff = (int64_t)in.ny * cx0;
+  const float *ba = in.a + toff, *bh = in.h + toff, *bv = bh + sz, *bd = bv + sz;
+  const unsigned off = (unsigned)cy * sizeof(float), step = (unsigned)in.ny * sizeof(float);
+  float a[NC], h[NC], v[NC], d[NC];
 #pragma unroll
-  for (int i = 0; i < CS_MAX; ++i) {
-    const int t = threadIdx.x + i * WTHREADS;
-    cv[i] = 0.f;
-    if (t < NCS) {
-      const int cyl = t % CN, cxl = (t / CN) % CN, s = t / (CN * CN);
-      const int cy = cy0 + cyl, cx = cx0 + cxl;
-      if (cy < in.ny && cx < in.nx) {
-        const int64_t p = cy + (int64_t)in.ny * cx;
-        cv[i] = s == 0 ? in.a[p] : in.h[(s - 1) * sz + p];
+  for (int c = 0; c < NC; ++c) a[c] = h[c] = v[c] = d[c] = 0.f;
+  if (cy < in.ny && lane < ST_Y / 2 + LF / 2 - 1) {
+    if (cx0 + NC <= in.nx) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        a[c] = at_bytes(ba, off + c * step);
+        h[c] = at_bytes(bh, off + c * step);
+        v[c] = at_bytes(bv, off + c * step);
+        d[c] = at_bytes(bd, off + c * step);
       }
+    } else {
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        if (cx0 + c < in.nx) {
+          a[c] = at_bytes(ba, off + c * step);
+          h[c] = at_bytes(bh, off + c * step);
+          v[c] = at_bytes(bv, off + c * step);
+          d[c] = at_bytes(bd, off + c * step);
+        }
     }
   }
-}
-
-template <int LF>
-__device__ __forceinline__ void syn_store_t(const float* cv, float* cs) {
-  constexpr int CN = WT / 2 + LF / 2 + 1;
-  constexpr int NCS = 4 * CN * CN;
+  // x filter: P = lo a + hi v (low along y), Q = lo h + hi d (high along y)
+  __builtin_amdgcn_wave_barrier();
 #pragma unroll
-  for (int i = 0; i < CS_MAX; ++i) {
-    const int t = threadIdx.x + i * WTHREADS;
-    if (t < NCS) cs[t] = cv[i];
-  }
-}
-
-// Output coordinates of a thread's accumulator entry q of syn_compute_t: the
-// thread makes the column pair ixl = 2c, 2c + 1 of row iyl for the pair
-// items t = threadIdx.x + (q / 2) WTHREADS (c = t / WT, iyl = t % WT).
-__device__ __forceinline__ void syn_acc_coord(int q, int& iyl, int& ixl) {
-  const int t = threadIdx.x + (q >> 1) * WTHREADS;
-  iyl = t % WT;
-  ixl = 2 * (t / WT) + (q & 1);
-}
-
-// expects cs staged and the caller's filter writes visible (after a barrier).
-// The two outputs of a parity pair (2u, 2u + 1) take the same LF/2
-// coefficients with the even and the odd taps, so each item makes both and
-// reads every staged value once for two outputs (half the LDS reads).
-template <int LF>
-__device__ __forceinline__ void syn_compute_t(const float* lo, const float* hi, int iy0, int ix0, int py, int px,
-                                              const float* cs, float* Ly, float* Hy, float* acc) {
-  constexpr int CN = WT / 2 + LF / 2 + 1;
-  float rlo[LF], rhi[LF];
-#pragma unroll
-  for (int j = 0; j < LF; ++j) {
-    rlo[j] = lo[j];
-    rhi[j] = hi[j];
-  }
-  // y pass: Ly[cx][iy] = sum_k lo a[k][cx] + hi h[k][cx];  Hy: v, d
-  // (iy0 is even: output 2u + par takes k = u + m with tap par + LF - 2 - 2m)
-  for (int t = threadIdx.x; t < (WT / 2) * CN; t += WTHREADS) {
-    const int u = t % (WT / 2), cxl = t / (WT / 2);
-    const float* a0 = cs + (0 * CN + cxl) * CN + u;
-    const float* h0 = cs + (1 * CN + cxl) * CN + u;
-    const float* v0 = cs + (2 * CN + cxl) * CN + u;
-    const float* d0 = cs + (3 * CN + cxl) * CN + u;
-    float sl0 = 0.f, sh0 = 0.f, sl1 = 0.f, sh1 = 0.f;
+  for (int u = 0; u < ST_X / 2; ++u) {
+    float pe = 0.f, po = 0.f, qe = 0.f, qo = 0.f;
 #pragma unroll
     for (int m = 0; m < LF / 2; ++m) {
       const int je = LF - 2 - 2 * m, jo = je + 1;
-      const float a = a0[m], h = h0[m], v = v0[m], d = d0[m];
-      sl0 += rlo[je] * a + rhi[je] * h;
-      sh0 += rlo[je] * v + rhi[je] * d;
-      sl1 += rlo[jo] * a + rhi[jo] * h;
-      sh1 += rlo[jo] * v + rhi[jo] * d;
+      pe += T.lo(je) * a[u + m] + T.hi(je) * v[u + m];
+      po += T.lo(jo) * a[u + m] + T.hi(jo) * v[u + m];
+      qe += T.lo(je) * h[u + m] + T.hi(je) * d[u + m];
+      qo += T.lo(jo) * h[u + m] + T.hi(jo) * d[u + m];
     }
-    Ly[cxl * WT + 2 * u] = sl0;
-    Hy[cxl * WT + 2 * u] = sh0;
-    Ly[cxl * WT + 2 * u + 1] = sl1;
-    Hy[cxl * WT + 2 * u + 1] = sh1;
+    pq[(2 * u) * ST_LD + lane] = pe;
+    pq[(2 * u + 1) * ST_LD + lane] = po;
+    pq[(ST_X + 2 * u) * ST_LD + lane] = qe;
+    pq[(ST_X + 2 * u + 1) * ST_LD + lane] = qo;
   }
-  __syncthreads();
-  // x pass: column pair (2c, 2c + 1) of row iyl (ix0 is even)
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  // y filter: the lane's 7 parity pairs
+  const int ix = lane & 7, g = lane >> 3;
+  constexpr int NR = ST_PER / 2 + LF / 2 - 1;
+  const float* P = pq + ix * ST_LD + (ST_PER / 2) * g;
+  const float* Q = P + ST_X * ST_LD;
+  float pr[NR], qr[NR];
 #pragma unroll
-  for (int q2 = 0; q2 < WT * WT / 2 / WTHREADS; ++q2) {
-    const int t = threadIdx.x + q2 * WTHREADS;
-    const int iyl = t % WT, c = t / WT;
-    float s0 = 0.f, s1 = 0.f;
+  for (int t = 0; t < NR; ++t) {
+    pr[t] = P[t];
+    qr[t] = Q[t];
+  }
+#pragma unroll
+  for (int u = 0; u < ST_PER / 2; ++u) {
+    float e = 0.f, o = 0.f;
 #pragma unroll
     for (int m = 0; m < LF / 2; ++m) {
       const int je = LF - 2 - 2 * m, jo = je + 1;
-      const float ly = Ly[(c + m) * WT + iyl], hy = Hy[(c + m) * WT + iyl];
-      s0 += rlo[je] * ly + rhi[je] * hy;
-      s1 += rlo[jo] * ly + rhi[jo] * hy;
+      e += T.lo(je) * pr[u + m] + T.hi(je) * qr[u + m];
+      o += T.lo(jo) * pr[u + m] + T.hi(jo) * qr[u + m];
     }
-    if (iy0 + iyl < py) {
-      if (ix0 + 2 * c < px) acc[2 * q2] += s0;
-      if (ix0 + 2 * c + 1 < px) acc[2 * q2 + 1] += s1;
-    }
-  }
-  __syncthreads();
-}
-
-template <int LF>
-__device__ void syn_tile_t(const SynIn& in, const float* lo, const float* hi, int iy0, int ix0, int py, int px,
-                           float* cs, float* Ly, float* Hy, float* acc) {
-  float cv[CS_MAX];
-  syn_load_t<LF>(in, iy0, ix0, cv);
-  syn_store_t<LF>(cv, cs);
-  __syncthreads();
-  syn_compute_t<LF>(lo, hi, iy0, ix0, py, px, cs, Ly, Hy, acc);
-}
-
-__device__ void syn_tile(const SynIn& in, int lf, const float* lo, const float* hi, int iy0, int ix0, int py,
-                         int px, float* cs, float* Ly, float* Hy, float* acc) {
-  switch (lf) {
-    case 2: syn_tile_t<2>(in, lo, hi, iy0, ix0, py, px, cs, Ly, Hy, acc); break;
-    case 4: syn_tile_t<4>(in, lo, hi, iy0, ix0, py, px, cs, Ly, Hy, acc); break;
-    case 6: syn_tile_t<6>(in, lo, hi, iy0, ix0, py, px, cs, Ly, Hy, acc); break;
-    case 8: syn_tile_t<8>(in, lo, hi, iy0, ix0, py, px, cs, Ly, Hy, acc); break;
-    case 10: syn_tile_t<10>(in, lo, hi, iy0, ix0, py, px, cs, Ly, Hy, acc); break;
-    case 12: syn_tile_t<12>(in, lo, hi, iy0, ix0, py, px, cs, Ly, Hy, acc); break;
-    case 14: syn_tile_t<14>(in, lo, hi, iy0, ix0, py, px, cs, Ly, Hy, acc); break;
-    default: syn_tile_t<16>(in, lo, hi, iy0, ix0, py, px, cs, Ly, Hy, acc); break;
+    acc[2 * u] += e;
+    acc[2 * u + 1] += o;
   }
 }
 
-// runtime filter length version (the finest level, whose basis loop would
-// otherwise hold all eight unrolled instances): accumulates the tile into acc
-__device__ void syn_tile_dyn(const SynIn& in, int lf, const float* lo, const float* hi, int iy0, int ix0,
-                         int py, int px, float* cs, float* Ly, float* Hy, float* acc) {
-  const int cy0 = (iy0 - 1) >= 0 ? (iy0) / 2 : 0;    // ceil((iy0-1)/2) for iy0 >= 0
-  const int cx0 = (ix0 - 1) >= 0 ? (ix0) / 2 : 0;
-  const int CN = WT / 2 + lf / 2 + 1;
-  const int64_t sz = (int64_t)in.ny * in.nx;
-  // load 4 subband tiles CN x CN: cs[s][cx][cy] (all loads issued first)
-  constexpr int CS_PER_THREAD = (4 * CMAX * CMAX + WTHREADS - 1) / WTHREADS;   // 10
-  float cv[CS_PER_THREAD];
-  const int ncs = 4 * CN * CN;
-#pragma unroll
-  for (int i = 0; i < CS_PER_THREAD; ++i) {
-    const int t = threadIdx.x + i * WTHREADS;
-    cv[i] = 0.f;
-    if (t < ncs) {
-      const int cyl = t % CN, cxl = (t / CN) % CN, s = t / (CN * CN);
-      const int cy = cy0 + cyl, cx = cx0 + cxl;
-      if (cy < in.ny && cx < in.nx) {
-        const int64_t p = cy + (int64_t)in.ny * cx;
-        cv[i] = s == 0 ? in.a[p] : in.h[(s - 1) * sz + p];
-      }
-    }
+__device__ __forceinline__ void syn_basis(const SaraGeom& G, int b, const SynIn& in, int iy0, int ix0, float* pq,
+                                          float* acc) {
+  switch (G.lf[b]) {
+    case 2: syn_tile<2>(G, b, in, iy0, ix0, pq, acc); break;
+    case 4: syn_tile<4>(G, b, in, iy0, ix0, pq, acc); break;
+    case 6: syn_tile<6>(G, b, in, iy0, ix0, pq, acc); break;
+    case 8: syn_tile<8>(G, b, in, iy0, ix0, pq, acc); break;
+    case 10: syn_tile<10>(G, b, in, iy0, ix0, pq, acc); break;
+    case 12: syn_tile<12>(G, b, in, iy0, ix0, pq, acc); break;
+    case 14: syn_tile<14>(G, b, in, iy0, ix0, pq, acc); break;
+    default: syn_tile<16>(G, b, in, iy0, ix0, pq, acc); break;
   }
-#pragma unroll
-  for (int i = 0; i < CS_PER_THREAD; ++i) {
-    const int t = threadIdx.x + i * WTHREADS;
-    if (t < ncs) cs[t] = cv[i];
-  }
-  __syncthreads();
-  // y pass: Ly[cx][iy] = sum_k lo[.] a[k][cx] + hi[.] h[k][cx];  Hy: v, d
-  for (int t = threadIdx.x; t < WT * CN; t += WTHREADS) {
-    const int iyl = t % WT, cxl = t / WT;
-    const int i = iy0 + iyl;
-    float sl = 0.f, sh = 0.f;
-    // k with j = i - 2k - 2 + lf in [0, lf)
-    int kmin = (i - 1 + 1) / 2;            // ceil((i-1)/2) for i >= 0
-    int kmax = (i + lf - 2) / 2;
-    kmin = max(kmin, cy0);
-    kmax = min(kmax, cy0 + CN - 1);
-    for (int kk = kmin; kk <= kmax; ++kk) {
-      const int j = i - 2 * kk - 2 + lf;
-      const int cyl = kk - cy0;
-      const float fa = lo[j], fh = hi[j];
-      sl += fa * cs[(0 * CN + cxl) * CN + cyl] + fh * cs[(1 * CN + cxl) * CN + cyl];
-      sh += fa * cs[(2 * CN + cxl) * CN + cyl] + fh * cs[(3 * CN + cxl) * CN + cyl];
-    }
-    Ly[cxl * WT + iyl] = sl;
-    Hy[cxl * WT + iyl] = sh;
-  }
-  __syncthreads();
-  // x pass
-  int q = 0;
-  for (int t = threadIdx.x; t < WT * WT; t += WTHREADS, ++q) {
-    const int iyl = t % WT, ixl = t / WT;
-    const int i = ix0 + ixl;
-    float s = 0.f;
-    int kmin = (i) / 2;
-    int kmax = (i + lf - 2) / 2;
-    kmin = max(kmin, cx0);
-    kmax = min(kmax, cx0 + CN - 1);
-    for (int kk = kmin; kk <= kmax; ++kk) {
-      const int j = i - 2 * kk - 2 + lf;
-      const int cxl = kk - cx0;
-      s += lo[j] * Ly[cxl * WT + iyl] + hi[j] * Hy[cxl * WT + iyl];
-    }
-    if (iy0 + iyl < py && i < px) acc[q] += s;
-  }
-  __syncthreads();
 }
 
-__global__ __launch_bounds__(WTHREADS) void k_syn_lk(SaraGeom G, int k, const float* __restrict__ v1,
-                                                     float* __restrict__ scr) {
-  __shared__ float cs[4 * CMAX * CMAX];
-  __shared__ float Ly[CMAX * WT];
-  __shared__ float Hy[CMAX * WT];
-  __shared__ float flo[WMAX_LF], fhi[WMAX_LF];
-  const int b = blockIdx.z % G.nb, l = blockIdx.z / G.nb;
-  const int iy0 = blockIdx.x * WT, ix0 = blockIdx.y * WT;
-  const int py = G.ny[b][k - 1], px = G.nx[b][k - 1];
-  if (iy0 >= py || ix0 >= px) return;
-  const int lf = G.lf[b];
-  if (threadIdx.x < lf) {
-    flo[threadIdx.x] = G.lo[b][threadIdx.x];
-    fhi[threadIdx.x] = G.hi[b][threadIdx.x];
-  }
+// One level.  FINEST: out = scale * (sum over the bases + Dirac) / sqrt(P), grid over
+// (tiles, channels); otherwise A_{k-1} of one basis, grid over (tiles, bases,
+// channels).  SPLIT (few tiles): the four waves of a workgroup share one tile of
+// the finest level, each taking a pair of bases with the same number of taps in
+// all, and add their sums in wave order.
+template <bool FINEST, bool SPLIT>
+__global__ __launch_bounds__(64 * ST_WAVES) void k_synthesis(const SaraGeom* __restrict__ geom, int k, int ty,
+                                                             int tx, int nz, const float* __restrict__ v1,
+                                                             float* __restrict__ scr, float scale,
+                                                             float* __restrict__ out) {
+  const SaraGeom& G = *geom;
+  __shared__ float lds[ST_WAVES][2 * ST_X * ST_LD];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int txg = SPLIT ? tx : (tx + ST_WAVES - 1) / ST_WAVES;
+  // XCDs take contiguous runs of workgroups, x fastest: neighbours in x share columns
+  const int total = ty * txg * nz, per = (total + 7) / 8;
+  const int s = blockIdx.x / 8, id = (int)(blockIdx.x % 8) * per + s;
+  if (s >= per || id >= total) return;
+  const int z = id / (ty * txg), t = id % (ty * txg);
+  const int iy0 = (t / txg) * ST_Y, ix0 = (SPLIT ? t % txg : (t % txg) * ST_WAVES + wv) * ST_X;
+  const int b0 = FINEST ? 0 : z % G.nb, l = FINEST ? z : z / G.nb;
+  const int py = FINEST ? G.Ny : G.ny[b0][k - 1], px = FINEST ? G.Nx : G.nx[b0][k - 1];
+  if (!SPLIT && (iy0 >= py || ix0 >= px)) return;
   const float* v1l = v1 + (int64_t)l * G.s;
   float* sc = scr + (int64_t)l * G.scr_per_chan;
-  SynIn in;
-  in.a = k == G.nlevel ? v1l + G.boff[b] + G.aoff[b] : sc + G.scr[b][k];
-  in.h = v1l + G.boff[b] + G.doff[b][k];
-  in.ny = G.ny[b][k];
-  in.nx = G.nx[b][k];
-  float acc[WT * WT / WTHREADS];
+  float* pq = lds[wv];
+  float acc[ST_PER];
 #pragma unroll
-  for (int q = 0; q < WT * WT / WTHREADS; ++q) acc[q] = 0.f;
-  syn_tile(in, lf, flo, fhi, iy0, ix0, py, px, cs, Ly, Hy, acc);
-  float* o = sc + G.scr[b][k - 1];
-#pragma unroll
-  for (int q = 0; q < WT * WT / WTHREADS; ++q) {
-    int iyl, ixl;
-    syn_acc_coord(q, iyl, ixl);
-    const int iy = iy0 + iyl, ix = ix0 + ixl;
-    if (iy < py && ix < px) o[iy + (int64_t)py * ix] = acc[q];
-  }
-}
-
-// finest level: all bases + Dirac, out = scale * Psi(v1)
-__global__ __launch_bounds__(WTHREADS) void k_syn_l1(SaraGeom G, const float* __restrict__ v1,
-                                                     const float* __restrict__ scr, float scale,
-                                                     float* __restrict__ out) {
-  __shared__ float cs[4 * CMAX * CMAX];
-  __shared__ float Ly[CMAX * WT];
-  __shared__ float Hy[CMAX * WT];
-  __shared__ float flo[WMAX_LF], fhi[WMAX_LF];
-  const int l = blockIdx.z;
-  const int iy0 = blockIdx.x * WT, ix0 = blockIdx.y * WT;
-  const float* v1l = v1 + (int64_t)l * G.s;
-  const float* sc = scr + (int64_t)l * G.scr_per_chan;
-  float acc[WT * WT / WTHREADS];
-#pragma unroll
-  for (int q = 0; q < WT * WT / WTHREADS; ++q) acc[q] = 0.f;
-  for (int b = 0; b < G.nb; ++b) {
-    const int lf = G.lf[b];
-    if (threadIdx.x < lf) {
-      flo[threadIdx.x] = G.lo[b][threadIdx.x];
-      fhi[threadIdx.x] = G.hi[b][threadIdx.x];
-    }
+  for (int q = 0; q < ST_PER; ++q) acc[q] = 0.f;
+  auto one = [&](int b) {
     SynIn in;
-    in.a = G.nlevel == 1 ? v1l + G.boff[b] + G.aoff[b] : sc + G.scr[b][1];
-    in.h = v1l + G.boff[b] + G.doff[b][1];
-    in.ny = G.ny[b][1];
-    in.nx = G.nx[b][1];
-    syn_tile_dyn(in, lf, flo, fhi, iy0, ix0, G.Ny, G.Nx, cs, Ly, Hy, acc);
-  }
-  const float* dir = v1l + G.boff[G.nb];
-  float* o = out + (int64_t)l * G.Ny * G.Nx;
-  int q = 0;
-  for (int t = threadIdx.x; t < WT * WT; t += WTHREADS, ++q) {
-    const int iy = iy0 + t % WT, ix = ix0 + t / WT;
-    if (iy < G.Ny && ix < G.Nx) {
-      const int64_t p = iy + (int64_t)G.Ny * ix;
-      float s = acc[q] * G.norm;
-      if (G.dirac) s += dir[p] * G.norm;
-      o[p] = scale * s;
+    in.a = k == G.nlevel ? v1l + G.boff[b] + G.aoff[b] : sc + G.scr[b][k];
+    in.h = v1l + G.boff[b] + G.doff[b][k];
+    in.ny = G.ny[b][k];
+    in.nx = G.nx[b][k];
+    syn_basis(G, b, in, iy0, ix0, pq, acc);
+  };
+  if constexpr (!FINEST) {
+    one(b0);
+  } else if constexpr (SPLIT) {
+    for (int b = wv; b < G.nb; b += 2 * ST_WAVES) {
+      one(b);
+      const int c = b - wv + 2 * ST_WAVES - 1 - wv;
+      if (c < G.nb) one(c);
     }
+  } else {
+    for (int b = 0; b < G.nb; ++b) one(b);
   }
-}
-
-// The standard SARA dictionary (db1..db8 in order: filter length 2(b+1)),
-// finest level: the basis loop is unrolled at compile time so every basis
-// runs its fixed-length tile code, and the subband loads of basis B+1 are
-// issued before the arithmetic of basis B (software pipelining).
-__device__ __forceinline__ SynIn syn_l1_in(const SaraGeom& G, const float* v1l, const float* sc, int b) {
-  SynIn in;
-  in.a = G.nlevel == 1 ? v1l + G.boff[b] + G.aoff[b] : sc + G.scr[b][1];
-  in.h = v1l + G.boff[b] + G.doff[b][1];
-  in.ny = G.ny[b][1];
-  in.nx = G.nx[b][1];
-  return in;
-}
-
-template <int B>
-__device__ __forceinline__ void syn_l1_std_bases(const SaraGeom& G, const float* v1l, const float* sc, int iy0,
-                                                 int ix0, float* flo, float* fhi, float* cs, float* Ly, float* Hy,
-                                                 float* cv, float* acc) {
-  constexpr int LF = 2 * (B + 1);
-  if (threadIdx.x < LF) {
-    flo[threadIdx.x] = G.lo[B][threadIdx.x];
-    fhi[threadIdx.x] = G.hi[B][threadIdx.x];
-  }
-  syn_store_t<LF>(cv, cs);   // basis B's subbands, loaded one step ahead
-  __syncthreads();
-  if constexpr (B + 1 < WMAX_BASES) syn_load_t<2 * (B + 2)>(syn_l1_in(G, v1l, sc, B + 1), iy0, ix0, cv);
-  syn_compute_t<LF>(flo, fhi, iy0, ix0, G.Ny, G.Nx, cs, Ly, Hy, acc);
-  if constexpr (B + 1 < WMAX_BASES)
-    syn_l1_std_bases<B + 1>(G, v1l, sc, iy0, ix0, flo, fhi, cs, Ly, Hy, cv, acc);
-}
-
-__global__ __launch_bounds__(WTHREADS) void k_syn_l1_std(SaraGeom G, const float* __restrict__ v1,
-                                                         const float* __restrict__ scr, float scale,
-                                                         float* __restrict__ out) {
-  __shared__ float cs[4 * CMAX * CMAX];
-  __shared__ float Ly[CMAX * WT];
-  __shared__ float Hy[CMAX * WT];
-  __shared__ float flo[WMAX_LF], fhi[WMAX_LF];
-  const int l = blockIdx.z;
-  const int iy0 = blockIdx.x * WT, ix0 = blockIdx.y * WT;
-  const float* v1l = v1 + (int64_t)l * G.s;
-  const float* sc = scr + (int64_t)l * G.scr_per_chan;
-  float acc[WT * WT / WTHREADS] = {0.f, 0.f, 0.f, 0.f};
-  float cv[CS_MAX];
-  syn_load_t<2>(syn_l1_in(G, v1l, sc, 0), iy0, ix0, cv);
-  syn_l1_std_bases<0>(G, v1l, sc, iy0, ix0, flo, fhi, cs, Ly, Hy, cv, acc);
-  const float* dir = v1l + G.boff[G.nb];
-  float* o = out + (int64_t)l * G.Ny * G.Nx;
+  // through LDS into whole columns of ST_Y pixels
+  __builtin_amdgcn_wave_barrier();
+  {
+    float* o = pq + (lane & 7) * ST_Y + ST_PER * (lane >> 3);
 #pragma unroll
-  for (int q = 0; q < WT * WT / WTHREADS; ++q) {
-    int iyl, ixl;
-    syn_acc_coord(q, iyl, ixl);
-    const int iy = iy0 + iyl, ix = ix0 + ixl;
-    if (iy < G.Ny && ix < G.Nx) {
-      const int64_t p = iy + (int64_t)G.Ny * ix;
-      float s = acc[q] * G.norm;
-      if (G.dirac) s += dir[p] * G.norm;
-      o[p] = scale * s;
+    for (int q = 0; q < ST_PER; ++q) o[q] = acc[q];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  float* dst = FINEST ? out + (int64_t)l * G.Ny * G.Nx : sc + G.scr[b0][k - 1];
+  const float* dir = v1l + G.boff[G.nb];
+  auto store = [&](int e, float v) {
+    const int iy = iy0 + e % ST_Y, ix = ix0 + e / ST_Y;
+    if (iy >= py || ix >= px) return;
+    const int64_t p = iy + (int64_t)py * ix;
+    if (FINEST) {
+      v *= G.norm;
+      if (G.dirac) v += dir[p] * G.norm;
+      v *= scale;
     }
+    dst[p] = v;
+  };
+  if constexpr (SPLIT) {
+    __syncthreads();
+    for (int e = threadIdx.x; e < ST_Y * ST_X; e += 64 * ST_WAVES)
+      store(e, ((lds[0][e] + lds[1][e]) + lds[2][e]) + lds[3][e]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < ST_PER; ++q) store(q * 64 + lane, pq[q * 64 + lane]);
   }
 }
 
-// ---- l21 dual step, Dirac analysis fused ------------------------------------
-// r_l = v1_l (+ xhat_l(p)/sqrt(P) on the Dirac block); l2 = ||r||_2 over l;
-// v1 <- r - max(l2 - beta w, 0)/(l2 + eps) r.   mode 1: only sum l2 (prior).
+// ---- more than 16 channels ---------------------------------------------------
+// The same modes from stored coefficients (mode 0: l21 step, 1: sum of the
+// norms, 2: weights), Dirac analysis fused.
 __global__ __launch_bounds__(256) void k_l21(SaraGeom G, float* __restrict__ v1,
                                              const float* __restrict__ xhat, int L,
                                              const float* __restrict__ w, double beta, int mode,
-                                             double* __restrict__ partial) {
+                                             float* __restrict__ wout, double* __restrict__ partial) {
   __shared__ double sh[256 / 64];
   double tot[1] = {0.0};
   const int64_t s = G.s;
@@ -627,7 +613,7 @@ __global__ __launch_bounds__(256) void k_l21(SaraGeom G, float* __restrict__ v1,
       continue;
     }
     if (mode == 2) {   // reweighting: w = upsilon / (upsilon + l2), beta = upsilon
-      partial[c] = beta / (beta + l2);
+      wout[c] = (float)(beta / (beta + l2));
       continue;
     }
     const double t = beta * (w ? (double)w[c] : 1.0);
@@ -647,65 +633,6 @@ __global__ __launch_bounds__(256) void k_l21(SaraGeom G, float* __restrict__ v1,
   }
 }
 
-// The same dual step (mode 0) four consecutive coefficients per thread with
-// 16-byte loads and stores: every channel's vector load of a step is issued
-// before the norms need them.  For s, the Dirac offset and Ny*Nx multiples of
-// 4 (a group of four is then wholly Dirac or wholly wavelet).
-__global__ __launch_bounds__(256) void k_l21_v4(SaraGeom G, float* __restrict__ v1,
-                                                const float* __restrict__ xhat, int L,
-                                                const float* __restrict__ w, double beta) {
-  constexpr int LREG = 16;
-  const int64_t s4 = G.s / 4;
-  const int64_t dstart = G.boff[G.nb];
-  const int64_t npix = (int64_t)G.Ny * G.Nx;
-  float4* __restrict__ v = reinterpret_cast<float4*>(v1);
-  for (int64_t c4 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c4 < s4;
-       c4 += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t c = 4 * c4;
-    const bool dir = G.dirac && c >= dstart && xhat;
-    float4 rv[LREG];
-    double ss[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int l = 0; l < LREG; ++l) {
-      if (l < L) {
-        float4 r = v[(int64_t)l * s4 + c4];
-        if (dir) {
-          const float4 xv = *reinterpret_cast<const float4*>(xhat + (int64_t)l * npix + (c - dstart));
-          r.x += xv.x * G.norm;
-          r.y += xv.y * G.norm;
-          r.z += xv.z * G.norm;
-          r.w += xv.w * G.norm;
-        }
-        rv[l] = r;
-        ss[0] += (double)r.x * r.x;
-        ss[1] += (double)r.y * r.y;
-        ss[2] += (double)r.z * r.z;
-        ss[3] += (double)r.w * r.w;
-      }
-    }
-    float4 wv = make_float4(1.f, 1.f, 1.f, 1.f);
-    if (w) wv = *reinterpret_cast<const float4*>(w + c);
-    const float wa[4] = {wv.x, wv.y, wv.z, wv.w};
-    float f[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const double l2 = sqrt(ss[j]);
-      f[j] = (float)(fmax(l2 - beta * (double)wa[j], 0.0) / (l2 + 2.220446049250313e-16));
-    }
-#pragma unroll
-    for (int l = 0; l < LREG; ++l)
-      if (l < L) {
-        const float4 r = rv[l];
-        v[(int64_t)l * s4 + c4] = make_float4(r.x - f[0] * r.x, r.y - f[1] * r.y, r.z - f[2] * r.z, r.w - f[3] * r.w);
-      }
-  }
-}
-
-__global__ void k_f64_to_f32(const double* __restrict__ a, int64_t n, float* __restrict__ b) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    b[i] = (float)a[i];
-}
-
 __global__ void k_sum_l(const double* __restrict__ partial, int n, double* out) {
   __shared__ double sh[4];
   double s[1] = {0.0};
@@ -714,66 +641,96 @@ __global__ void k_sum_l(const double* __restrict__ partial, int n, double* out) 
   if (threadIdx.x == 0) *out = s[0];
 }
 
-// v1 := Psit(x) on the Dirac block when no l21 step follows (plain analysis)
-__global__ void k_dirac_copy(SaraGeom G, const float* __restrict__ x, int L, float* __restrict__ v1,
-                             int accumulate) {
-  const int64_t N = (int64_t)G.Ny * G.Nx;
-  const int64_t dstart = G.boff[G.nb];
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < N * L;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int l = (int)(i / N);
-    const int64_t p = i - (int64_t)l * N;
-    float* d = v1 + (int64_t)l * G.s + dstart + p;
-    const float v = x[i] * G.norm;
-    *d = accumulate ? *d + v : v;
+unsigned analysis_grid(const SaraGeom& G, int k, int& ty, int& tx) {
+  int ny = 0, nx = 0;
+  for (int b = 0; b < G.nb; ++b) {
+    ny = std::max(ny, G.ny[b][k]);
+    nx = std::max(nx, G.nx[b][k]);
   }
+  ty = (int)cdiv(ny, AT_Y);
+  tx = (int)cdiv(nx, AT_X);
+  return 8 * cdiv((long long)ty * tx, 8) * G.nb;
+}
+
+template <int MODE>
+void launch_analysis(fhs_ctx* ctx, const fhs_sara* S, const AnArgs& A, unsigned grid, int ty, int tx) {
+  // LDS: the turning tiles, or every channel's coefficients and the factors
+  const bool last = A.k == S->g.nlevel;
+  const size_t nq = (last ? 4 : 3) * AT_X * 64;
+  const size_t lds = std::max<size_t>(A.L * AT_LH, MODE >= AN_L21 ? (A.L + 1) * nq : 0) * sizeof(float);
+  auto go = [&](auto kern) {
+    allow_dynamic_lds((const void*)kern, lds);
+    kern<<<grid, 64 * A.L, lds, ctx->stream>>>(S->d, A, ty, tx);
+    check_launch();
+  };
+  last ? go(k_analysis<MODE, true>) : go(k_analysis<MODE, false>);
+}
+
+// All levels and the Dirac block in one mode; at most AN_CHANNELS channels for
+// the modes over the channels.  Returns the number of workgroup sums (AN_NORM).
+template <int MODE>
+unsigned sara_analyse(fhs_ctx* ctx, const fhs_sara* S, const float* x, int L, float* v1, const float* w, double beta,
+                      float* wout, double* part) {
+  const SaraGeom& G = S->g;
+  float* scr = (float*)ctx->ws.get("sara_scratch", std::max<int64_t>(1, G.scr_per_chan * L) * sizeof(float));
+  const int64_t N = (int64_t)G.Ny * G.Nx;
+  unsigned nsum = 0;
+  for (int l0 = 0; l0 < L; l0 += AN_CHANNELS) {
+    AnArgs A;
+    A.L = std::min(AN_CHANNELS, L - l0);
+    A.x = x + (int64_t)l0 * N;
+    A.scr = scr + (int64_t)l0 * G.scr_per_chan;
+    A.v1 = v1 ? v1 + (int64_t)l0 * G.s : nullptr;
+    A.w = w;
+    A.beta = beta;
+    A.wout = wout;
+    for (int k = 1; k <= G.nlevel && G.nb > 0; ++k) {
+      int ty, tx;
+      const unsigned grid = analysis_grid(G, k, ty, tx);
+      A.k = k;
+      A.part = part ? part + nsum : nullptr;
+      launch_analysis<MODE>(ctx, S, A, grid, ty, tx);
+      nsum += grid;
+    }
+    if (G.dirac) {
+      const bool vec = N % 4 == 0 && (uintptr_t)A.x % 16 == 0 &&
+                       (MODE > AN_L21 || (G.s % 4 == 0 && G.boff[G.nb] % 4 == 0 && (uintptr_t)A.v1 % 16 == 0));
+      const unsigned grid = std::min<unsigned>(2048, cdiv(vec ? N / 4 : N, 256));
+      (vec ? k_dirac<MODE, 4> : k_dirac<MODE, 1>)<<<grid, 256, 0, ctx->stream>>>(G, A.x, A.v1, A.L, w, beta, wout,
+                                                                                 part ? part + nsum : nullptr);
+      check_launch();
+      nsum += grid;
+    }
+  }
+  return nsum;
 }
 
 }  // namespace
-
-// coefficients (+)= Psit(x) for the wavelet bases (Dirac block untouched)
-void sara_analysis_wavelets(fhs_ctx* ctx, const fhs_sara* S, const float* x, int L, float* v1) {
-  const SaraGeom& G = S->g;
-  float* scr = (float*)ctx->ws.get("sara_scratch", std::max<int64_t>(1, G.scr_per_chan * L) * sizeof(float));
-  int my = 0, mx = 0;
-  for (int b = 0; b < G.nb; ++b) {
-    my = std::max(my, G.ny[b][1]);
-    mx = std::max(mx, G.nx[b][1]);
-  }
-  Scope sc(ctx, "wavelet_analysis");
-  (void)my;
-  (void)mx;
-  for (int k = 1; k <= G.nlevel; ++k) {
-    int ny = 0, nx = 0;
-    for (int b = 0; b < G.nb; ++b) {
-      ny = std::max(ny, G.ny[b][k]);
-      nx = std::max(nx, G.nx[b][k]);
-    }
-    k_an_lk<<<dim3(cdiv(ny, AY), cdiv(nx, AX), G.nb * L), WTHREADS, 0, ctx->stream>>>(G, k, x, v1, scr);
-    check_launch();
-  }
-}
 
 // out = scale * Psi(v1) (wavelets + Dirac)
 void sara_synthesis(fhs_ctx* ctx, const fhs_sara* S, const float* v1, int L, float scale, float* out) {
   const SaraGeom& G = S->g;
   float* scr = (float*)ctx->ws.get("sara_scratch", std::max<int64_t>(1, G.scr_per_chan * L) * sizeof(float));
   Scope sc(ctx, "wavelet_synthesis");
+  auto grid = [](int ty, int txg, int z) { return dim3(8 * cdiv((long long)ty * txg * z, 8), 1, 1); };
   for (int k = G.nlevel; k >= 2 && G.nb > 0; --k) {
     int py = 0, px = 0;
     for (int b = 0; b < G.nb; ++b) {
       py = std::max(py, G.ny[b][k - 1]);
       px = std::max(px, G.nx[b][k - 1]);
     }
-    k_syn_lk<<<dim3(cdiv(py, WT), cdiv(px, WT), G.nb * L), WTHREADS, 0, ctx->stream>>>(G, k, v1, scr);
+    const int ty = (int)cdiv(py, ST_Y), tx = (int)cdiv(px, ST_X);
+    k_synthesis<false, false><<<grid(ty, (int)cdiv(tx, ST_WAVES), G.nb * L), 64 * ST_WAVES, 0, ctx->stream>>>(
+        S->d, k, ty, tx, G.nb * L, v1, scr, scale, out);
     check_launch();
   }
-  bool std_dict = G.nb == WMAX_BASES;
-  for (int b = 0; b < G.nb && std_dict; ++b) std_dict = G.lf[b] == 2 * (b + 1);
-  if (std_dict)
-    k_syn_l1_std<<<dim3(cdiv(G.Ny, WT), cdiv(G.Nx, WT), L), WTHREADS, 0, ctx->stream>>>(G, v1, scr, scale, out);
+  const int ty = (int)cdiv(G.Ny, ST_Y), tx = (int)cdiv(G.Nx, ST_X);
+  if ((int64_t)ty * tx * L < SYN_SPLIT_BELOW)
+    k_synthesis<true, true><<<grid(ty, tx, L), 64 * ST_WAVES, 0, ctx->stream>>>(S->d, 1, ty, tx, L, v1, scr, scale,
+                                                                                       out);
   else
-    k_syn_l1<<<dim3(cdiv(G.Ny, WT), cdiv(G.Nx, WT), L), WTHREADS, 0, ctx->stream>>>(G, v1, scr, scale, out);
+    k_synthesis<true, false><<<grid(ty, (int)cdiv(tx, ST_WAVES), L), 64 * ST_WAVES, 0, ctx->stream>>>(
+        S->d, 1, ty, tx, L, v1, scr, scale, out);
   check_launch();
 }
 
@@ -781,17 +738,16 @@ void sara_synthesis(fhs_ctx* ctx, const fhs_sara* S, const float* v1, int L, flo
 void sara_dual_step(fhs_ctx* ctx, const fhs_sara* S, float* v1, const float* xhat, int L,
                     const float* w, double beta, float sigma1, float* g1) {
   const SaraGeom& G = S->g;
-  if (G.nb) sara_analysis_wavelets(ctx, S, xhat, L, v1);
   {
-    Scope sc(ctx, "l21_threshold");
-    const bool v4 = L <= 16 && G.s % 4 == 0 && G.boff[G.nb] % 4 == 0 && ((int64_t)G.Ny * G.Nx) % 4 == 0 &&
-                    (((uintptr_t)v1 | (uintptr_t)xhat | (uintptr_t)w) % 16) == 0;
-    if (v4)
-      k_l21_v4<<<std::min<int64_t>(cdiv(G.s / 4, 256), 2048), 256, 0, ctx->stream>>>(G, v1, xhat, L, w, beta);
-    else
-      k_l21<<<cdiv(G.s, 256) < 2048 ? cdiv(G.s, 256) : 2048, 256, 0, ctx->stream>>>(G, v1, xhat, L, w, beta, 0,
-                                                                                     nullptr);
-    check_launch();
+    Scope sc(ctx, "wavelet_l21");
+    if (L <= AN_CHANNELS) {
+      sara_analyse<AN_L21>(ctx, S, xhat, L, v1, w, beta, nullptr, nullptr);
+    } else {
+      sara_analyse<AN_ADD>(ctx, S, xhat, L, v1, nullptr, 0.0, nullptr, nullptr);
+      k_l21<<<std::min<unsigned>(2048, cdiv(G.s, 256)), 256, 0, ctx->stream>>>(G, v1, nullptr, L, w, beta, 0, nullptr,
+                                                                               nullptr);
+      check_launch();
+    }
   }
   sara_synthesis(ctx, S, v1, L, sigma1, g1);
 }
@@ -830,7 +786,6 @@ int fhs_sara_create_host(fhs_ctx* ctx, int Ny, int Nx, int nlevel, int nbases,
       G.lf[b] = lf;
       for (int j = 0; j < lf; ++j) {
         G.lo[b][j] = (float)f[j];
-        G.hi[b][j] = (float)((j % 2 ? -1.0 : 1.0) * f[lf - 1 - j]);
       }
       f += lf;
       G.ny[b][0] = Ny;
@@ -856,11 +811,18 @@ int fhs_sara_create_host(fhs_ctx* ctx, int Ny, int Nx, int nlevel, int nbases,
     G.boff[nbases] = off;
     G.s = off + (G.dirac ? (int64_t)Ny * Nx : 0);
     G.scr_per_chan = soff;
+    FHS_HIP(hipSetDevice(ctx->device));
+    FHS_HIP(hipMalloc(&S->d, sizeof(SaraGeom)));
+    FHS_HIP(hipMemcpy(S->d, &G, sizeof(SaraGeom), hipMemcpyHostToDevice));
     *out = S;
   });
 }
 
 int fhs_sara_destroy(fhs_sara* S) {
+  if (S && S->d) {
+    (void)hipSetDevice(S->device);
+    (void)hipFree(S->d);
+  }
   delete S;
   return FHS_OK;
 }
@@ -876,13 +838,11 @@ int fhs_sara_analysis(fhs_ctx* ctx, const fhs_sara* S, const float* x, int L, fl
   if (!ctx) return FHS_ERR_ARG;
   return guard(ctx, [&] {
     FHS_CHECK(S && x && coefs && L >= 1 && L * std::max(1, S->g.nb) <= 65535, "sara_analysis: bad argument");
-    if (!accumulate)
-      FHS_HIP(hipMemsetAsync(coefs, 0, (size_t)S->g.s * L * sizeof(float), ctx->stream));
-    if (S->g.nb) sara_analysis_wavelets(ctx, S, x, L, coefs);
-    if (S->g.dirac) {
-      k_dirac_copy<<<1024, 256, 0, ctx->stream>>>(S->g, x, L, coefs, 1);
-      check_launch();
-    }
+    Scope sc(ctx, "wavelet_analysis");
+    if (accumulate)
+      sara_analyse<AN_ADD>(ctx, S, x, L, coefs, nullptr, 0.0, nullptr, nullptr);
+    else
+      sara_analyse<AN_SET>(ctx, S, x, L, coefs, nullptr, 0.0, nullptr, nullptr);
   });
 }
 
@@ -911,14 +871,14 @@ int fhs_sara_update_weights(fhs_ctx* ctx, const fhs_sara* S, const float* x, int
     FHS_CHECK(S && x && weights1 && L >= 1 && L * std::max(1, S->g.nb) <= 65535,
               "sara_update_weights: bad argument");
     const SaraGeom& G = S->g;
+    if (L <= AN_CHANNELS) {   // the coefficients are never stored
+      sara_analyse<AN_WEIGHT>(ctx, S, x, L, nullptr, nullptr, upsilon, weights1, nullptr);
+      return;
+    }
     float* c = (float*)ctx->ws.get("sara_prior_coefs", (size_t)G.s * L * sizeof(float));
-    FHS_HIP(hipMemsetAsync(c, 0, (size_t)G.s * L * sizeof(float), ctx->stream));
-    if (G.nb) sara_analysis_wavelets(ctx, S, x, L, c);
-    double* w = (double*)ctx->ws.get("sara_weights_f64", (size_t)G.s * sizeof(double));
-    const unsigned nbk = cdiv(G.s, 256) < 2048 ? cdiv(G.s, 256) : 2048;
-    k_l21<<<nbk, 256, 0, ctx->stream>>>(G, c, G.dirac ? x : nullptr, L, nullptr, upsilon, 2, w);
-    check_launch();
-    k_f64_to_f32<<<nbk, 256, 0, ctx->stream>>>(w, G.s, weights1);
+    sara_analyse<AN_SET>(ctx, S, x, L, c, nullptr, 0.0, nullptr, nullptr);
+    k_l21<<<std::min<unsigned>(2048, cdiv(G.s, 256)), 256, 0, ctx->stream>>>(G, c, nullptr, L, nullptr, upsilon, 2,
+                                                                             weights1, nullptr);
     check_launch();
   });
 }
@@ -928,16 +888,25 @@ int fhs_compute_sara_prior(fhs_ctx* ctx, const fhs_sara* S, const float* x, int 
   return guard(ctx, [&] {
     FHS_CHECK(S && x && out && L >= 1 && L * std::max(1, S->g.nb) <= 65535, "compute_sara_prior: bad argument");
     const SaraGeom& G = S->g;
-    float* c = (float*)ctx->ws.get("sara_prior_coefs", (size_t)G.s * L * sizeof(float));
-    FHS_HIP(hipMemsetAsync(c, 0, (size_t)G.s * L * sizeof(float), ctx->stream));
-    if (G.nb) sara_analysis_wavelets(ctx, S, x, L, c);
-    const unsigned nbk = cdiv(G.s, 256) < 2048 ? cdiv(G.s, 256) : 2048;
-    double* part = (double*)ctx->ws.get("sara_prior_partial", (nbk + 1) * sizeof(double));
-    k_l21<<<nbk, 256, 0, ctx->stream>>>(G, c, G.dirac ? x : nullptr, L, nullptr, 0.0, 1, part);
+    unsigned n = 2048;   // workgroup sums
+    for (int k = 1; k <= G.nlevel && G.nb > 0; ++k) {
+      int ty, tx;
+      n += analysis_grid(G, k, ty, tx);
+    }
+    double* part = (double*)ctx->ws.get("sara_prior_partial", (n + 1) * sizeof(double));
+    unsigned nsum = 0;
+    if (L <= AN_CHANNELS) {
+      nsum = sara_analyse<AN_NORM>(ctx, S, x, L, nullptr, nullptr, 0.0, nullptr, part);
+    } else {
+      float* c = (float*)ctx->ws.get("sara_prior_coefs", (size_t)G.s * L * sizeof(float));
+      sara_analyse<AN_SET>(ctx, S, x, L, c, nullptr, 0.0, nullptr, nullptr);
+      nsum = std::min<unsigned>(2048, cdiv(G.s, 256));
+      k_l21<<<nsum, 256, 0, ctx->stream>>>(G, c, nullptr, L, nullptr, 0.0, 1, nullptr, part);
+      check_launch();
+    }
+    k_sum_l<<<1, 256, 0, ctx->stream>>>(part, (int)nsum, part + n);
     check_launch();
-    k_sum_l<<<1, 256, 0, ctx->stream>>>(part, nbk, part + nbk);
-    check_launch();
-    FHS_HIP(hipMemcpyAsync(out, part + nbk, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    FHS_HIP(hipMemcpyAsync(out, part + n, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
     FHS_HIP(hipStreamSynchronize(ctx->stream));
   });
 }

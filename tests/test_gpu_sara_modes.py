@@ -1,0 +1,52 @@
+"""Every use of the analysis (set, accumulate, l21 step, weights, prior) and the
+synthesis at the edges of their tiles (56 x 4 coefficients, 112 x 8 pixels),
+for channel counts that fill a workgroup, do not, and exceed it; against the
+FP64 oracle at the 1e-5 of the FP32 transforms."""
+import numpy as np
+import pytest
+import torch
+
+from oracle.wavelets import SaraDictionary as SaraRef
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5
+
+
+def rel(a, b):
+    return np.linalg.norm(np.asarray(a, dtype=np.float64) - b) / np.linalg.norm(b)
+
+
+@pytest.mark.parametrize('Ny,Nx,L,nlevel', [(5, 3, 1, 2), (112, 8, 2, 1), (113, 9, 5, 4), (30, 250, 4, 4),
+                                            (98, 64, 16, 4), (40, 33, 17, 3)])
+def test_modes(ctx, Ny, Nx, L, nlevel):
+    import fhs
+    rng = np.random.default_rng(Ny + Nx + L)
+    S = fhs.SaraDictionary(ctx, Ny, Nx, nlevel=nlevel)
+    ref = SaraRef(Ny, Nx, nlevel=nlevel)
+    x = rng.random((L, Nx, Ny)).astype(np.float32)
+    xd = torch.from_numpy(x).cuda()
+    c = np.stack([ref.psit(x[l].T.astype(np.float64)) for l in range(L)])
+    out = torch.full((L, S.s), float('nan'), device='cuda')
+    S.psit(xd, out=out)
+    assert rel(out.cpu().numpy(), c) < TOL
+    v1 = rng.standard_normal((L, S.s)).astype(np.float32)
+    w = rng.random(S.s).astype(np.float32)
+    acc = torch.from_numpy(v1).cuda()
+    S.psit(xd, out=acc, accumulate=True)
+    assert rel(acc.cpu().numpy(), v1 + c) < TOL
+    for weights in (w, None):
+        vd = torch.from_numpy(v1).cuda()
+        vd, g1 = fhs.hs_update_dual_sparsity_distributed(
+            vd, S, S, xd, None if weights is None else torch.from_numpy(weights).cuda(), 0.8, 0.3)
+        r = v1.astype(np.float64) + c
+        n = np.linalg.norm(r, axis=0)
+        thr = 0.8 * (1.0 if weights is None else weights.astype(np.float64))
+        vr = r - np.maximum(n - thr, 0) / (n + np.finfo(float).eps) * r
+        assert rel(vd.cpu().numpy(), vr) < TOL
+        gr = np.stack([0.3 * ref.psi(vr[l]).T for l in range(L)])
+        assert rel(g1.cpu().numpy(), gr) < TOL
+    wd = torch.full((S.s,), float('nan'), device='cuda')
+    ctx.check(fhs.lib().fhs_sara_update_weights(ctx.h, S.h, xd.data_ptr(), L, 0.1, wd.data_ptr()), 'weights')
+    n = np.linalg.norm(c, axis=0)
+    assert rel(wd.cpu().numpy(), 0.1 / (0.1 + n)) < TOL
+    assert abs(fhs.compute_sara_prior(xd, S) / n.sum() - 1) < TOL
