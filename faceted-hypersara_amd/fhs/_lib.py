@@ -127,6 +127,9 @@ PROTOTYPES = {
     'fhs_sara_update_weights': [c_void_p, c_void_p, c_void_p, c_int, c_double, c_void_p],
     'fhs_nn_gemm': [c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_void_p, c_int,
                     C.c_float, C.c_float, c_void_p, c_int],
+    'fhs_nn_conv3x3': [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p],
+    'fhs_nn_conv3x3_backward': [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p,
+                                c_void_p, c_void_p, c_void_p],
     'fhs_nn_im2col3': [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     'fhs_nn_col2im3': [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     'fhs_nn_relu_bwd': [c_void_p, c_void_p, c_void_p, c_i64],

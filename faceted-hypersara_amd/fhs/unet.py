@@ -3,8 +3,8 @@ FP32 accumulation) mapping back-projected dirty facet tiles to an initial
 cube, trained and run with this project's own kernels (``fhs_nn_*``).
 
 Activations are FP32 tensors in [C][N][H][W] order; every 3x3 convolution
-is im2col + one BF16 matrix-core GEMM (``fhs_nn_gemm``), its gradients one
-GEMM each plus a col2im gather.  torch only owns the buffers (and
+and its gradients are BF16 matrix-core kernels (``fhs_nn_conv3x3``,
+``fhs_nn_conv3x3_backward``).  torch only owns the buffers (and
 concatenates skip connections).
 
 The warm start plugs into the reference's hook for an initial cube
@@ -42,34 +42,21 @@ class Conv3x3:
 
     def forward(self, x, NB, H, W, keep=True):
         ctx = self.ctx
-        Q = NB * H * W
-        col = torch.empty((self.cin * 9, Q), dtype=torch.float32, device=ctx.device)
-        ctx.check(lib().fhs_nn_im2col3(ctx.h, _f(x), self.cin, NB, H, W, _f(col)), 'nn_im2col3')
-        y = torch.empty((self.cout, Q), dtype=torch.float32, device=ctx.device)
-        ctx.check(lib().fhs_nn_gemm(ctx.h, self.cout, Q, self.cin * 9, _f(self.W), self.cin * 9, 0, _f(col), Q, 0,
-                                    _f(y), Q, 1.0, 0.0, _f(self.b), int(self.relu)), 'nn_gemm')
-        self.cache = (col, y, NB, H, W) if keep else None
+        y = torch.empty((self.cout, NB * H * W), dtype=torch.float32, device=ctx.device)
+        ctx.check(lib().fhs_nn_conv3x3(ctx.h, _f(x), self.cin, NB, H, W, _f(self.W), self.cout, _f(self.b),
+                                       int(self.relu), _f(y)), 'nn_conv3x3')
+        self.cache = (x, y, NB, H, W) if keep else None
         return y
 
     def backward(self, gy):
-        """gy: gradient w.r.t. the output (masked in place by the ReLU);
-        accumulates dW, db; returns the gradient w.r.t. the input."""
+        """gy: gradient w.r.t. the output; accumulates dW, db; returns the
+        gradient w.r.t. the input."""
         ctx = self.ctx
-        col, y, NB, H, W = self.cache
-        Q = NB * H * W
-        if self.relu:
-            ctx.check(lib().fhs_nn_relu_bwd(ctx.h, _f(y), _f(gy), gy.numel()), 'nn_relu_bwd')
-        K = self.cin * 9
-        ctx.check(lib().fhs_nn_gemm(ctx.h, self.cout, K, Q, _f(gy), Q, 0, _f(col), Q, 1,
-                                    _f(self.dW), K, 1.0, 1.0, None, 0), 'nn_gemm dW')
-        db = torch.empty_like(self.db)
-        ctx.check(lib().fhs_nn_bias_grad(ctx.h, _f(gy), self.cout, Q, _f(db)), 'nn_bias_grad')
-        self.db += db
-        dcol = torch.empty((K, Q), dtype=torch.float32, device=ctx.device)
-        ctx.check(lib().fhs_nn_gemm(ctx.h, K, Q, self.cout, _f(self.W), K, 1, _f(gy), Q, 0,
-                                    _f(dcol), Q, 1.0, 0.0, None, 0), 'nn_gemm dcol')
-        dx = torch.empty((self.cin, Q), dtype=torch.float32, device=ctx.device)
-        ctx.check(lib().fhs_nn_col2im3(ctx.h, _f(dcol), self.cin, NB, H, W, _f(dx)), 'nn_col2im3')
+        x, y, NB, H, W = self.cache
+        dx = torch.empty((self.cin, NB * H * W), dtype=torch.float32, device=ctx.device)
+        ctx.check(lib().fhs_nn_conv3x3_backward(ctx.h, _f(x), self.cin, NB, H, W, _f(self.W), self.cout,
+                                                _f(y) if self.relu else None, _f(gy), _f(self.dW), _f(self.db),
+                                                _f(dx)), 'nn_conv3x3_backward')
         self.cache = None
         return dx
 
@@ -93,6 +80,18 @@ class UNet:
             self.dec.append((Conv3x3(ctx, w[i + 1], w[i], True, rng), Conv3x3(ctx, 2 * w[i], w[i], True, rng),
                              Conv3x3(ctx, w[i], w[i], True, rng)))
         self.head = Conv3x3(ctx, w[0], cout, False, rng)
+        # parameters, gradients and moments of all layers each in one buffer the
+        # layers' tensors are views of: one fill and one Adam launch a step
+        names = [(layer, four) for layer in self.layers()
+                 for four in (('W', 'dW', 'mW', 'vW'), ('b', 'db', 'mb', 'vb'))]
+        values = torch.cat([getattr(layer, four[0]).reshape(-1) for layer, four in names])
+        self._flat = [values] + [torch.zeros_like(values) for _ in range(3)]
+        at = 0
+        for layer, four in names:
+            t = getattr(layer, four[0])
+            for flat, name in zip(self._flat, four):
+                setattr(layer, name, flat[at:at + t.numel()].view(t.shape))
+            at += t.numel()
         self.step_count = 0
         self._skips = None
 
@@ -131,6 +130,8 @@ class UNet:
         """x: (cin, NB*H*W) float32 ([C][N][H][W]) -> (cout, NB*H*W).
         H and W must be divisible by 2^(levels-1)."""
         h, Hc, Wc = x.contiguous(), H, W
+        if keep and h.data_ptr() == x.data_ptr():
+            h = h.clone()        # backward reads it again: the caller may reuse x meanwhile
         skips = []
         for i, (a, b) in enumerate(self.enc):
             h = b.forward(a.forward(h, NB, Hc, Wc, keep), NB, Hc, Wc, keep)
@@ -169,17 +170,30 @@ class UNet:
         self._skips = None
         return g
 
+    def _whole(self):
+        """The layers' tensors still tile the flat buffers (none was replaced)."""
+        at = 0
+        for layer in self.layers():
+            for four in layer.params():
+                if any(t.data_ptr() != f.data_ptr() + 4 * at for t, f in zip(four, self._flat)):
+                    return False
+                at += four[0].numel()
+        return True
+
     def zero_grad(self):
+        if self._whole():
+            self._flat[1].zero_()
+            return
         for layer in self.layers():
             layer.dW.zero_()
             layer.db.zero_()
 
     def adam(self, lr=1e-3, beta1=0.9, beta2=0.999, eps=1e-8):
         self.step_count += 1
-        for layer in self.layers():
-            for p, g, m, v in layer.params():
-                self.ctx.check(lib().fhs_nn_adam(self.ctx.h, _f(p), _f(g), _f(m), _f(v), p.numel(), lr, beta1,
-                                                 beta2, eps, self.step_count), 'nn_adam')
+        groups = [self._flat] if self._whole() else [p for layer in self.layers() for p in layer.params()]
+        for p, g, m, v in groups:
+            self.ctx.check(lib().fhs_nn_adam(self.ctx.h, _f(p), _f(g), _f(m), _f(v), p.numel(), lr, beta1,
+                                             beta2, eps, self.step_count), 'nn_adam')
 
     def mse(self, pred, target, grad=True):
         """mean squared error and its gradient (2/n)(pred - target)."""

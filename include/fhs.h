@@ -499,6 +499,16 @@ int fhs_pdfb_stream(fhs_pdfb* p, void** stream);
  * trans_a (A stored K x M, leading dim lda), op(B) = B^T when trans_b. */
 int fhs_nn_gemm(fhs_ctx* ctx, int M, int N, int K, const float* A, int lda, int trans_a, const float* B,
                 int ldb, int trans_b, float* C, int ldc, float alpha, float beta, const float* bias, int relu);
+/* out = conv3x3(in; w) + bias (ReLU), zero padding 1: in float[cin][NB][H][W],
+ * w float[cout][cin*9] (k = c*9 + ky*3 + kx), bias float[cout] or NULL, out
+ * float[cout][NB][H][W]; operands rounded to BF16, FP32 sums. */
+int fhs_nn_conv3x3(fhs_ctx* ctx, const float* in, int cin, int NB, int H, int W, const float* w, int cout,
+                   const float* bias, int relu, float* out);
+/* Its gradients from gout float[cout][NB][H][W], which counts where out_relu (the
+ * layer's output; NULL without ReLU) is not <= 0: dw float[cout][cin*9] and db
+ * float[cout] are added to, gin float[cin][NB][H][W] is written (NULL: not wanted). */
+int fhs_nn_conv3x3_backward(fhs_ctx* ctx, const float* in, int cin, int NB, int H, int W, const float* w, int cout,
+                            const float* out_relu, const float* gout, float* dw, float* db, float* gin);
 /* col[(c*9 + ky*3 + kx)][n,y,x] = in[c][n][y+ky-1][x+kx-1] (zero padding) */
 int fhs_nn_im2col3(fhs_ctx* ctx, const float* in, int C, int NB, int H, int W, float* col);
 /* adjoint of im2col3 (gather form, no atomics) */

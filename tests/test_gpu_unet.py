@@ -115,3 +115,46 @@ def test_unet_training_reduces_loss(ctx):
         net.backward(g, NB, H, W)
         net.adam(lr=2e-3)
     assert loss < 0.1 * first
+
+
+@pytest.mark.parametrize('cin,cout,NB,H,W', [(8, 16, 1, 8, 32), (5, 3, 2, 9, 33), (16, 16, 1, 3, 7), (17, 40, 1, 20, 45),
+                                             (64, 32, 2, 16, 64), (128, 128, 1, 8, 8), (24, 20, 3, 70, 38)])
+@pytest.mark.parametrize('relu', [True, False])
+def test_conv3x3(ctx, cin, cout, NB, H, W, relu):
+    """The convolution and its gradients at the edges of their pixel tiles and
+    channel groups, against the FP64 products of the BF16-rounded operands
+    (1e-5: FP32 sums), and the bits of im2col, GEMM and col2im."""
+    from fhs._lib import lib
+    from fhs.core import _ptr
+    rng = np.random.default_rng(cin + cout + W)
+    Q = NB * H * W
+    x, w, b, gy = (rng.normal(size=s).astype(np.float32) for s in ((cin, Q), (cout, cin * 9), (cout,), (cout, Q)))
+    xd, wd, bd, gd = dev(x), dev(w), dev(b), dev(gy)
+    y = torch.full((cout, Q), float('nan'), device='cuda')
+    ctx.check(lib().fhs_nn_conv3x3(ctx.h, _ptr(xd), cin, NB, H, W, _ptr(wd), cout, _ptr(bd), int(relu), _ptr(y)), 'conv')
+    col = im2col3(bf16(x), NB, H, W)
+    ref = bf16(w) @ col + b[:, None].astype(np.float64)
+    ref = np.maximum(ref, 0) if relu else ref
+    assert rel(y.cpu().numpy(), ref) < 1e-5
+    cd, yg = torch.empty((cin * 9, Q), device='cuda'), torch.empty_like(y)
+    ctx.check(lib().fhs_nn_im2col3(ctx.h, _ptr(xd), cin, NB, H, W, _ptr(cd)), 'im2col')
+    ctx.check(lib().fhs_nn_gemm(ctx.h, cout, Q, cin * 9, _ptr(wd), cin * 9, 0, _ptr(cd), Q, 0, _ptr(yg), Q, 1.0, 0.0,
+                                _ptr(bd), int(relu)), 'gemm')
+    assert torch.equal(y, yg)
+    dw, db = dev(np.ones_like(w)), dev(np.ones_like(b))
+    dx = torch.full((cin, Q), float('nan'), device='cuda')
+    ctx.check(lib().fhs_nn_conv3x3_backward(ctx.h, _ptr(xd), cin, NB, H, W, _ptr(wd), cout, _ptr(y) if relu else None,
+                                            _ptr(gd), _ptr(dw), _ptr(db), _ptr(dx)), 'conv backward')
+    g = np.where(y.cpu().numpy() > 0, gy, 0) if relu else gy
+    assert rel(dw.cpu().numpy() - 1.0, bf16(g) @ col.T) < 1e-5
+    assert rel(db.cpu().numpy() - 1.0, g.astype(np.float64).sum(1)) < 1e-5
+    assert rel(dx.cpu().numpy(), col2im3(bf16(w).T @ bf16(g), cin, NB, H, W)) < 1e-5
+    gm, xg = dev(g.astype(np.float32)), torch.empty_like(dx)
+    wg = dev(np.ones_like(w))
+    ctx.check(lib().fhs_nn_gemm(ctx.h, cout, cin * 9, Q, _ptr(gm), Q, 0, _ptr(cd), Q, 1, _ptr(wg), cin * 9, 1.0, 1.0,
+                                None, 0), 'gemm')
+    assert torch.equal(dw, wg)
+    ctx.check(lib().fhs_nn_gemm(ctx.h, cin * 9, Q, cout, _ptr(wd), cin * 9, 1, _ptr(gm), Q, 0, _ptr(cd), Q, 1.0, 0.0,
+                                None, 0), 'gemm')
+    ctx.check(lib().fhs_nn_col2im3(ctx.h, _ptr(cd), cin, NB, H, W, _ptr(xg)), 'col2im')
+    assert torch.equal(dx, xg)
