@@ -155,13 +155,12 @@ def algorithmic_bytes(meas, sara_s, lowrank=None):
     return {
         'data_adjoint': adj,
         'data_forward': fwd,
-        'fft_fwd_y': 4 * N * L + 8 * (No // 2) * L,          # read image, write half-grid
-        'fft_fwd_x': 8 * (No // 2) * L + 8 * No * L,
-        'fft_adj_x': 8 * No * L + 8 * (No // 2) * L,
-        'fft_adj_y': 8 * (No // 2) * L + 4 * N * L,
-        'wavelet_analysis': 4 * L * N + 8 * L * sara_s,
+        'fft_fwd_y': 4 * N * L + 8 * (No // 4) * L,          # read image, write column pairs
+        'fft_fwd_x': 8 * (No // 4) * L + 8 * No * L,
+        'fft_adj_x': 8 * No * L + 8 * (No // 4) * L,
+        'fft_adj_y': 8 * (No // 4) * L + 4 * N * L,
+        'wavelet_l21': 4 * L * N + 8 * L * sara_s + 4 * sara_s,
         'wavelet_synthesis': 4 * L * sara_s + 4 * L * N,
-        'l21_threshold': 8 * L * sara_s + 4 * L * N + 4 * sara_s,
         'primal': 4 * L * N * 6,
         'fb_dual': 44 * sum(M),
         **lowrank_bytes(lowrank, L, N),

@@ -2,14 +2,23 @@
 // adjoint, batched over channels.
 //
 // The grid is Kty x Ktx (column-major, y contiguous); the image Ny x Nx sits
-// in its top-left corner.  Each transform is two passes through HBM:
-//   forward : (1) y-pass: one workgroup per image column, scale by sn, zero
-//                 pad to Kty and FFT -> T (Kty x Nx, only Nx columns exist,
-//                 the rest are zero);
-//             (2) x-pass: one workgroup per B consecutive grid rows, FFT of
-//                 length Ktx over the Nx non-zero columns of T -> Fx.
-//   adjoint : (1') x-pass inverse keeping the first Nx outputs -> T;
-//             (2') y-pass inverse, keep Ny outputs, * sn, real part, * scale.
+// in its top-left corner.  The image is real, so two of its columns make one
+// complex y transform, and the adjoint needs the rows ky <= Kty / 2 of the grid's
+// Hermitian part only.  Each transform is two passes through HBM:
+//   forward : (1) y-pass: one workgroup per two image columns a, b: scale by sn
+//                 and 1/2, zero pad to Kty, FFT of a + i b -> Z (Kty x Nx / 2);
+//             (2) x-pass: one workgroup per B consecutive grid rows: the columns'
+//                 rows from Z[ky] and Z[-ky], FFT of length Ktx -> Fx.
+//   adjoint : (1') x-pass: the real part of the image comes from the Hermitian
+//                 part g[ky][kx] + conj g[-ky][-kx]; inverse FFT of its rows
+//                 ky <= Kty / 2, first Nx outputs -> U (half of Kty, x Nx);
+//             (2') y-pass of U[a] + i U[b]: real and imaginary part are the two
+//                 columns, keep Ny outputs, * sn / 2 * scale.
+// Against one transform per column and per row, us of (1) (2) (1') (2'): 16 grids of
+// 1024^2 30 48 51 25 -> 20 51 42 18, 8 of 2048^2 61 119 132 52 -> 36 116 97 35, 4 of
+// 4096^2 141 414 323 122 -> 79 377 277 77; the bytes of the full grid bound the x-passes.
+// (Rows ky <= Kty / 2 in (2) too, each writing its mirror: 56 and 158 us at 1024 and
+// 2048, since mirrored row groups are never aligned and write parts of lines.)
 // The y-passes use a register-resident radix-16 Stockham FFT whose first
 // stage reads the column from global memory and whose last stage writes it
 // (two LDS round trips at 4096 points).  The x-passes read and write B
@@ -266,7 +275,7 @@ constexpr int fft_threads() { return B * n / 16 < 64 ? 64 : (B * n / 16 > 1024 ?
 // workgroups per CU), 4 from N = 2048 (64 KB of rows plus the twiddles, two
 // workgroups per CU; 128 KB and one per CU at N = 4096, where 2 rows, 16-byte
 // segments, measured slower).  Segments below 128 bytes are merged in one
-// XCD's L2 by xpass_row0.
+// XCD's L2 (xpass_row0).
 template <int N>
 constexpr int b_strided() { return N >= 2048 ? 4 : (N >= 1024 ? 8 : 16); }
 template <int N, int B>
@@ -274,12 +283,11 @@ constexpr int nt_strided() {
   return B * N / 4 > 1024 ? 1024 : (B * N / 4 < 64 ? 64 : B * N / 4);
 }
 
-// x-pass workgroup -> first grid row.  Workgroups are dispatched to the 8
-// XCDs round-robin (linear id mod 8; gridDim.x is a multiple of 8 here, so
-// blockIdx.x mod 8).  When B rows are fewer than a 128-byte line (G = 16 / B
-// workgroups share each line of every grid column), workgroups b, b + 8, ...,
-// b + 8 (G - 1) take G adjacent row groups, so the line is fetched into one
-// XCD's L2 instead of G.
+// x-pass workgroup -> first of its B grid rows.  Workgroups are dispatched to the 8
+// XCDs round-robin (linear id mod 8; gridDim.x is a multiple of 8, so blockIdx.x mod
+// 8).  Forward: when B rows are fewer than a 128-byte line (G = 16 / B workgroups
+// share each line of every grid column), workgroups b, b + 8, ..., b + 8 (G - 1)
+// take G adjacent row groups, so the line is put together in one XCD's L2.
 template <int B>
 __device__ __forceinline__ int xpass_row0() {
   constexpr int G = 16 / B;
@@ -291,59 +299,113 @@ __device__ __forceinline__ int xpass_row0() {
     return ((b / (8 * G)) * (8 * G) + (b % 8) * G + (b / 8) % G) * B;
   }
 }
+// Runtime lengths and the adjoint, whose groups read their mirror too, which is not aligned: an XCD takes a
+// contiguous eighth of the rows in turn (60 -> 54 us at 16 x 1024 x 1024).
+__device__ __forceinline__ int xpass_eighth_row0(int B) {
+  return ((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8) * B;
+}
+inline unsigned xpass_eighth_grid(int rows, int B) { return (cdiv(rows, B) + 7) / 8 * 8; }
+
+// ---- rows of a real image's transform ---------------------------------------
+// An adjoint x-pass of the fixed sizes runs rows 0 .. half_rows(Kty) - 1: with Kty even
+// rows 0 and Kty / 2, both Hermitian in kx (real outputs), share slot 0 as real and
+// imaginary part, so that Kty / 2 transforms fill the grid exactly.
+__host__ __device__ inline int half_rows(int Kty) { return Kty % 2 ? Kty / 2 + 1 : Kty / 2; }
+// stride of a column of U (rows 0 .. Kty / 2), whole 128-byte lines
+__host__ __device__ inline int half_stride(int Kty) { return (Kty / 2 + 1 + 15) / 16 * 16; }
+
+// Row ky of columns 2 p and 2 p + 1 from z = Z[p][ky], m = Z[p][-ky] (1/2 is in Z)
+__device__ __forceinline__ void split_pair(float2 z, float2 m, float2& a, float2& b) {
+  a = make_float2(z.x + m.x, z.y - m.y);
+  b = make_float2(z.y + m.y, m.x - z.x);
+}
+
+// The rows of an adjoint x-pass thread: its own, its mirror, and the second row of the
+// shared slot.  A thread beyond the last row idles on row 0.
+struct HalfRow {
+  int ky, mirror, second;
+  bool valid, shared;
+  __device__ __forceinline__ HalfRow(int k, int Kty) {
+    valid = k < half_rows(Kty);
+    ky = valid ? k : 0;
+    mirror = ky ? Kty - ky : 0;
+    shared = ky == 0 && Kty % 2 == 0;
+    second = Kty / 2;
+  }
+};
+
+// an adjoint x-pass output: the shared slot holds row 0 and row Kty / 2, both real
+__device__ __forceinline__ void adj_store(float2* __restrict__ col, const HalfRow& row, float2 u) {
+  col[row.ky] = row.shared ? make_float2(u.x, 0.f) : u;
+  if (row.shared) col[row.second] = make_float2(u.y, 0.f);
+}
+
+// twice the Hermitian part of the grid at (ky, kx)
+__device__ __forceinline__ float2 hermitian(float2 v, float2 m) { return make_float2(v.x + m.x, v.y - m.y); }
 
 // threads of a y-pass workgroup of an N-point grid
 template <int N>
 constexpr int nt_y() { return fft_threads<N, 1>(); }
 
-// (1) forward y-pass: one workgroup per image column, scaled by sn, zero
+// (1) forward y-pass: one workgroup per two image columns, scaled by sn, zero
 // padded to N = Kty
 template <int N>
 __global__ __launch_bounds__(nt_y<N>()) void k_fwd_y(const float* __restrict__ x,
                                                               const float* __restrict__ sy,
                                                               const float* __restrict__ sx, int Ny, int Nx,
                                                               const float2* __restrict__ tw,
-                                                              float2* __restrict__ T) {
+                                                              float2* __restrict__ Z) {
   constexpr int NT = fft_threads<N, 1>();
   __shared__ float2 s[fft_lds_slots<N, 1>()];
-  const int ix = blockIdx.x, l = blockIdx.y;
-  const float* __restrict__ xc = x + ((size_t)l * Nx + ix) * Ny;
-  const float scx = sx[ix];
-  float2* __restrict__ out = T + ((size_t)l * Nx + ix) * N;
+  const int ix = 2 * blockIdx.x, l = blockIdx.y, two = ix + 1 < Nx;
+  const float* __restrict__ xa = x + ((size_t)l * Nx + ix) * Ny;
+  const float* __restrict__ xb = xa + (two ? Ny : 0);
+  const float sa = 0.5f * sx[ix], sb = two ? 0.5f * sx[ix + 1] : 0.f;
+  float2* __restrict__ out = Z + ((size_t)l * gridDim.x + blockIdx.x) * N;
   auto load = [&](int, int, int, int n) {
-    return n < Ny ? make_float2(xc[n] * sy[n] * scx, 0.f) : make_float2(0.f, 0.f);
+    return n < Ny ? make_float2(xa[n] * sy[n] * sa, two ? xb[n] * sy[n] * sb : 0.f) : make_float2(0.f, 0.f);
   };
   auto store = [&](int, int, int, int n, float2 v) { out[n] = v; };
   fft_reg<N, 1, NT, false>(s, tw, 1, load, store);
 }
 
-// (2) forward x-pass: N = Ktx
+// (2) forward x-pass: N = Ktx.  A thread's LDS slots are two neighbouring columns of
+// one row: slots(j) = ((2 p) B + b, (2 p + 1) B + b) for pair p B + b = threadIdx.x + j NT.
 template <int N, int B>
-__global__ __launch_bounds__((nt_strided<N, B>())) void k_fwd_x(const float2* __restrict__ T, int Kty,
+__global__ __launch_bounds__((nt_strided<N, B>())) void k_fwd_x(const float2* __restrict__ Z, int Kty,
                                                           int Nx, const float2* __restrict__ tw,
                                                           float2* __restrict__ Fx) {
   constexpr int NT = nt_strided<N, B>();
+  static_assert(NT % B == 0 && N * B / 2 % NT == 0, "a thread keeps its row");
   __shared__ float2 s[N * B];
   __shared__ float2 tws[TW_LDS<N>];
-  const int ky0 = xpass_row0<B>(), l = blockIdx.y;
+  const int b = threadIdx.x % B, p0 = threadIdx.x / B, l = blockIdx.y, row = xpass_row0<B>() + b;
+  const bool valid = row < Kty;
+  const int ky = valid ? row : 0, mk = ky ? Kty - ky : 0;
   const float2* twp = stage_twiddles<N, NT, TW_LDS<N>>(tw, tws);
-  const float2* Tl = T + (size_t)l * Nx * Kty;
-  constexpr int PER = N * B / NT;   // every load issued before the first LDS store
-  float2 v[PER];
+  const float2* Zl = Z + (size_t)l * ((Nx + 1) / 2) * Kty;
+  constexpr int PER = N * B / 2 / NT;   // every load issued before the first LDS store
+  float2 z[PER], m[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int t = threadIdx.x + j * NT;
-    const int b = t % B, i = t / B;
-    v[j] = i < Nx ? Tl[(size_t)i * Kty + ky0 + b] : make_float2(0.f, 0.f);
+    const int p = p0 + j * (NT / B);
+    const bool in = 2 * p < Nx;
+    z[j] = in ? Zl[(size_t)p * Kty + ky] : make_float2(0.f, 0.f);
+    m[j] = in ? Zl[(size_t)p * Kty + mk] : make_float2(0.f, 0.f);
   }
 #pragma unroll
-  for (int j = 0; j < PER; ++j) s[threadIdx.x + j * NT] = v[j];
+  for (int j = 0; j < PER; ++j) {
+    const int p = p0 + j * (NT / B);
+    float2 a, c;
+    split_pair(z[j], m[j], a, c);
+    s[2 * p * B + b] = a;
+    s[(2 * p + 1) * B + b] = 2 * p + 1 < Nx ? c : make_float2(0.f, 0.f);
+  }
   __syncthreads();
   fft_lds<N, B, NT, false>(s, twp);
   float2* F = Fx + (size_t)l * N * Kty;
   for (int t = threadIdx.x; t < N * B; t += NT) {
-    const int b = t % B, k = t / B;
-    F[(size_t)k * Kty + ky0 + b] = s[t];
+    if (valid) F[(size_t)(t / B) * Kty + ky] = s[t];
   }
 }
 
@@ -351,29 +413,40 @@ __global__ __launch_bounds__((nt_strided<N, B>())) void k_fwd_x(const float2* __
 template <int N, int B>
 __global__ __launch_bounds__((nt_strided<N, B>())) void k_adj_x(const float2* __restrict__ g, int Kty,
                                                           int Nx, const float2* __restrict__ tw,
-                                                          float2* __restrict__ T) {
+                                                          float2* __restrict__ U) {
   constexpr int NT = nt_strided<N, B>();
   __shared__ float2 s[N * B];
   __shared__ float2 tws[TW_LDS<N>];
-  const int ky0 = xpass_row0<B>(), l = blockIdx.y;
+  const int b = threadIdx.x % B, l = blockIdx.y, ky0 = xpass_eighth_row0(B);
+  if (ky0 >= half_rows(Kty)) return;
+  const HalfRow row(ky0 + b, Kty);
   const float2* twp = stage_twiddles<N, NT, TW_LDS<N>>(tw, tws);
   const float2* gl = g + (size_t)l * N * Kty;
   constexpr int PER = N * B / NT;   // every load issued before the first LDS store
-  float2 v[PER];
+  float2 v[PER], m[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int t = threadIdx.x + j * NT;
-    v[j] = gl[(size_t)(t / B) * Kty + ky0 + t % B];
+    const int k = (threadIdx.x + j * NT) / B;
+    v[j] = gl[(size_t)k * Kty + row.ky];
+    m[j] = gl[(size_t)((N - k) % N) * Kty + row.mirror];
   }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) v[j] = hermitian(v[j], m[j]);
+  if (row.shared)
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int k = (threadIdx.x + j * NT) / B;
+      const float2 h = hermitian(gl[(size_t)k * Kty + row.second], gl[(size_t)((N - k) % N) * Kty + row.second]);
+      v[j] = make_float2(v[j].x - h.y, v[j].y + h.x);
+    }
 #pragma unroll
   for (int j = 0; j < PER; ++j) s[threadIdx.x + j * NT] = v[j];
   __syncthreads();
   fft_lds<N, B, NT, true>(s, twp);
-  float2* Tl = T + (size_t)l * Nx * Kty;
-  for (int t = threadIdx.x; t < Nx * B; t += NT) {
-    const int b = t % B, i = t / B;
-    Tl[(size_t)i * Kty + ky0 + b] = s[t];
-  }
+  const int hs = half_stride(Kty);
+  float2* Ul = U + (size_t)l * Nx * hs;
+  if (row.valid)
+    for (int t = threadIdx.x; t < Nx * B; t += NT) adj_store(Ul + (size_t)(t / B) * hs, row, s[t]);
 }
 
 // Split x-passes for N >= X_SPLIT_MIN when the image holds at most half the
@@ -386,80 +459,111 @@ __global__ __launch_bounds__((nt_strided<N, B>())) void k_adj_x(const float2* __
 // The two H-point transforms run one after the other in the same H x B
 // rows of LDS (64 KB at N = 4096 instead of 128 KB: two workgroups per CU),
 // the H-point twiddles being every other entry of the N-point table.
+// 64 registers, for those two workgroups of 1024 threads: a few spilled values cost less
+// than one workgroup a CU (adjoint 332 -> 277 us, 4 grids of 4096^2).
 constexpr int X_SPLIT_MIN = 4096;
 
 template <int N, int B>
-__global__ __launch_bounds__((nt_strided<N, B>())) void k_fwd_x_split(const float2* __restrict__ T, int Kty,
+__global__ __launch_bounds__((nt_strided<N, B>()), B == 8 ? 4 : 8) void k_fwd_x_split(const float2* __restrict__ Z, int Kty,
                                                                 int Nx, const float2* __restrict__ tw,
                                                                 float2* __restrict__ Fx) {
   constexpr int H = N / 2;
   constexpr int NT = nt_strided<N, B>();
-  static_assert(H * B % NT == 0, "split x-pass: whole rows per thread");
+  static_assert(H * B / 2 % NT == 0 && NT % B == 0, "split x-pass: whole rows per thread");
   __shared__ float2 s[H * B];
   __shared__ float2 tws[3 * H / 4];
-  const int ky0 = xpass_row0<B>(), l = blockIdx.y;
+  const int b = threadIdx.x % B, p0 = threadIdx.x / B, l = blockIdx.y, row = xpass_row0<B>() + b;
+  const bool valid = row < Kty;
+  const int ky = valid ? row : 0, mk = ky ? Kty - ky : 0;
   for (int i = threadIdx.x; i < 3 * H / 4; i += NT) tws[i] = tw[2 * i];
-  const float2* Tl = T + (size_t)l * Nx * Kty;
-  constexpr int PER = H * B / NT;
-  float2 v[PER];
+  const float2* Zl = Z + (size_t)l * ((Nx + 1) / 2) * Kty;
+  constexpr int PER = H * B / 2 / NT;
+  float2 v[PER], w[PER];          // columns 2 p and 2 p + 1
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int t = threadIdx.x + j * NT;
-    const int b = t % B, i = t / B;
-    v[j] = i < Nx ? Tl[(size_t)i * Kty + ky0 + b] : make_float2(0.f, 0.f);
+    const int p = p0 + j * (NT / B);
+    const bool in = 2 * p < Nx;
+    v[j] = in ? Zl[(size_t)p * Kty + ky] : make_float2(0.f, 0.f);
+    w[j] = in ? Zl[(size_t)p * Kty + mk] : make_float2(0.f, 0.f);
   }
 #pragma unroll
-  for (int j = 0; j < PER; ++j) s[threadIdx.x + j * NT] = v[j];
+  for (int j = 0; j < PER; ++j) {
+    const int p = p0 + j * (NT / B);
+    float2 a, c;
+    split_pair(v[j], w[j], a, c);
+    v[j] = a;
+    w[j] = 2 * p + 1 < Nx ? c : make_float2(0.f, 0.f);
+    s[2 * p * B + b] = v[j];
+    s[(2 * p + 1) * B + b] = w[j];
+  }
   __syncthreads();
   fft_lds<H, B, NT, false>(s, tws);
   float2* F = Fx + (size_t)l * N * Kty;
-  // each thread reads back, then overwrites, only its own LDS slots
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int k = 2 * (p0 + j * (NT / B)) + i;
+      if (valid) F[(size_t)(2 * k) * Kty + ky] = s[k * B + b];
+    }
+  // each thread read back, and now overwrites, only its own LDS slots
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int t = threadIdx.x + j * NT;
-    const int b = t % B, k = t / B;
-    F[(size_t)(2 * k) * Kty + ky0 + b] = s[t];
-    s[t] = cmul(v[j], tw[k]);
+    const int k = 2 * (p0 + j * (NT / B));
+    s[k * B + b] = cmul(v[j], tw[k]);
+    s[(k + 1) * B + b] = cmul(w[j], tw[k + 1]);
   }
   __syncthreads();
   fft_lds<H, B, NT, false>(s, tws);
 #pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    const int t = threadIdx.x + j * NT;
-    const int b = t % B, k = t / B;
-    F[(size_t)(2 * k + 1) * Kty + ky0 + b] = s[t];
-  }
+  for (int j = 0; j < PER; ++j)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int k = 2 * (p0 + j * (NT / B)) + i;
+      if (valid) F[(size_t)(2 * k + 1) * Kty + ky] = s[k * B + b];
+    }
 }
 
 template <int N, int B>
-__global__ __launch_bounds__((nt_strided<N, B>())) void k_adj_x_split(const float2* __restrict__ g, int Kty,
+__global__ __launch_bounds__((nt_strided<N, B>()), B == 8 ? 4 : 8) void k_adj_x_split(const float2* __restrict__ g, int Kty,
                                                                 int Nx, const float2* __restrict__ tw,
-                                                                float2* __restrict__ T) {
+                                                                float2* __restrict__ U) {
   constexpr int H = N / 2;
   constexpr int NT = nt_strided<N, B>();
-  static_assert(H * B % NT == 0, "split x-pass: whole rows per thread");
+  static_assert(H * B % NT == 0 && NT % B == 0, "split x-pass: whole rows per thread");
   __shared__ float2 s[H * B];
   __shared__ float2 tws[3 * H / 4];
-  const int ky0 = xpass_row0<B>(), l = blockIdx.y;
+  const int b = threadIdx.x % B, l = blockIdx.y, ky0 = xpass_eighth_row0(B);
+  if (ky0 >= half_rows(Kty)) return;
+  const HalfRow row(ky0 + b, Kty);
   for (int i = threadIdx.x; i < 3 * H / 4; i += NT) tws[i] = tw[2 * i];
   const float2* gl = g + (size_t)l * N * Kty;
   constexpr int PER = H * B / NT;
   float2 v[PER], e[PER];
+  auto load = [&](int odd) {
+    float2 m[PER];
 #pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    const int t = threadIdx.x + j * NT;
-    v[j] = gl[(size_t)(2 * (t / B)) * Kty + ky0 + t % B];
-  }
+    for (int j = 0; j < PER; ++j) {
+      const int k = 2 * ((threadIdx.x + j * NT) / B) + odd;
+      v[j] = gl[(size_t)k * Kty + row.ky];
+      m[j] = gl[(size_t)((N - k) % N) * Kty + row.mirror];
+    }
+#pragma unroll
+    for (int j = 0; j < PER; ++j) v[j] = hermitian(v[j], m[j]);
+    if (row.shared)
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        const int k = 2 * ((threadIdx.x + j * NT) / B) + odd;
+        const float2 h = hermitian(gl[(size_t)k * Kty + row.second], gl[(size_t)((N - k) % N) * Kty + row.second]);
+        v[j] = make_float2(v[j].x - h.y, v[j].y + h.x);
+      }
+  };
+  load(0);
 #pragma unroll
   for (int j = 0; j < PER; ++j) s[threadIdx.x + j * NT] = v[j];
-  // the odd rows are loaded while the even half is transformed
-#pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    const int t = threadIdx.x + j * NT;
-    v[j] = gl[(size_t)(2 * (t / B) + 1) * Kty + ky0 + t % B];
-  }
   __syncthreads();
   fft_lds<H, B, NT, true>(s, tws);
+  load(1);
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int t = threadIdx.x + j * NT;
@@ -468,22 +572,30 @@ __global__ __launch_bounds__((nt_strided<N, B>())) void k_adj_x_split(const floa
   }
   __syncthreads();
   fft_lds<H, B, NT, true>(s, tws);
-  float2* Tl = T + (size_t)l * Nx * Kty;
+  const int hs = half_stride(Kty);
+  float2* Ul = U + (size_t)l * Nx * hs;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    const int t = threadIdx.x + j * NT;
-    const int b = t % B, n = t / B;
-    if (n < Nx) {
+    const int t = threadIdx.x + j * NT, n = t / B;
+    if (n < Nx && row.valid) {
       float2 w = tw[n];
       w.y = -w.y;
-      Tl[(size_t)n * Kty + ky0 + b] = cadd(e[j], cmul(s[t], w));
+      adj_store(Ul + (size_t)n * hs, row, cadd(e[j], cmul(s[t], w)));
     }
   }
 }
 
-// (2') adjoint y-pass: N = Kty, keep Ny outputs, real part, scale
+// element n of U[a] + i U[b], both Hermitian with rows 0 .. N / 2 stored
+__device__ __forceinline__ float2 join_pair(const float2* __restrict__ ua, const float2* __restrict__ ub, int N, int n) {
+  const bool mirror = 2 * n > N;
+  const int k = mirror ? N - n : n;
+  const float2 a = ua[k], c = ub ? ub[k] : make_float2(0.f, 0.f);
+  return mirror ? make_float2(a.x + c.y, c.x - a.y) : make_float2(a.x - c.y, a.y + c.x);
+}
+
+// (2') adjoint y-pass: N = Kty, two columns, keep Ny outputs, scale
 template <int N>
-__global__ __launch_bounds__(nt_y<N>()) void k_adj_y(const float2* __restrict__ T,
+__global__ __launch_bounds__(nt_y<N>()) void k_adj_y(const float2* __restrict__ U,
                                                               const float* __restrict__ sy,
                                                               const float* __restrict__ sx, int Ny, int Nx,
                                                               const float2* __restrict__ tw,
@@ -491,13 +603,18 @@ __global__ __launch_bounds__(nt_y<N>()) void k_adj_y(const float2* __restrict__ 
                                                               float* __restrict__ out) {
   constexpr int NT = fft_threads<N, 1>();
   __shared__ float2 s[fft_lds_slots<N, 1>()];
-  const int ix = blockIdx.x, l = blockIdx.y;
-  const float2* __restrict__ Tc = T + ((size_t)l * Nx + ix) * N;
-  const float sc = (scale ? scale[l] : 1.f) * sx[ix];
+  const int ix = 2 * blockIdx.x, l = blockIdx.y, hs = half_stride(N);
+  const bool two = ix + 1 < Nx;
+  const float2* __restrict__ ua = U + ((size_t)l * Nx + ix) * hs;
+  const float2* __restrict__ ub = two ? ua + hs : nullptr;
+  const float sc = 0.5f * (scale ? scale[l] : 1.f), sa = sc * sx[ix], sb = two ? sc * sx[ix + 1] : 0.f;
   float* __restrict__ o = out + ((size_t)l * Nx + ix) * Ny;
-  auto load = [&](int, int, int, int n) { return Tc[n]; };
+  auto load = [&](int, int, int, int n) { return join_pair(ua, ub, N, n); };
   auto store = [&](int, int, int, int n, float2 v) {
-    if (n < Ny) o[n] = sc * sy[n] * v.x;
+    if (n < Ny) {
+      o[n] = sa * sy[n] * v.x;
+      if (two) o[Ny + n] = sb * sy[n] * v.y;
+    }
   };
   fft_reg<N, 1, NT, true>(s, tw, 1, load, store);
 }
@@ -520,7 +637,7 @@ void dispatch_pow2(int n, Args&&... args) {
 template <int N>
 struct RunFwdY {
   static void run(hipStream_t st, int Nx, int L, const float* x, const fhs_nufft* p, float2* T) {
-    k_fwd_y<N><<<dim3(Nx, L), nt_y<N>(), 0, st>>>(x, p->sy, p->sx, p->Ny, p->Nx, p->twy, T);
+    k_fwd_y<N><<<dim3((Nx + 1) / 2, L), nt_y<N>(), 0, st>>>(x, p->sy, p->sx, p->Ny, p->Nx, p->twy, T);
   }
 };
 // Rows per x-pass workgroup: the default first, then the autotuner's other
@@ -572,10 +689,10 @@ struct RunFwdX {
                     with_rows<N, SP>(c, [&](auto b_c) {
                       constexpr int B = decltype(b_c)::value;
                       if constexpr (SP)
-                        k_fwd_x_split<N, B><<<dim3(Kty / B, L), nt_strided<N, B>(), 0, ctx->stream>>>(T, Kty, p->Nx,
+                        k_fwd_x_split<N, B><<<dim3(cdiv(Kty, B), L), nt_strided<N, B>(), 0, ctx->stream>>>(T, Kty, p->Nx,
                                                                                                     p->twx, F);
                       else
-                        k_fwd_x<N, B><<<dim3(Kty / B, L), nt_strided<N, B>(), 0, ctx->stream>>>(T, Kty, p->Nx,
+                        k_fwd_x<N, B><<<dim3(cdiv(Kty, B), L), nt_strided<N, B>(), 0, ctx->stream>>>(T, Kty, p->Nx,
                                                                                               p->twx, F);
                       check_launch();
                     });
@@ -601,10 +718,10 @@ struct RunAdjX {
                     with_rows<N, SP>(c, [&](auto b_c) {
                       constexpr int B = decltype(b_c)::value;
                       if constexpr (SP)
-                        k_adj_x_split<N, B><<<dim3(Kty / B, L), nt_strided<N, B>(), 0, ctx->stream>>>(g, Kty, p->Nx,
+                        k_adj_x_split<N, B><<<dim3(xpass_eighth_grid(half_rows(Kty), B), L), nt_strided<N, B>(), 0, ctx->stream>>>(g, Kty, p->Nx,
                                                                                                     p->twx, T);
                       else
-                        k_adj_x<N, B><<<dim3(Kty / B, L), nt_strided<N, B>(), 0, ctx->stream>>>(g, Kty, p->Nx,
+                        k_adj_x<N, B><<<dim3(xpass_eighth_grid(half_rows(Kty), B), L), nt_strided<N, B>(), 0, ctx->stream>>>(g, Kty, p->Nx,
                                                                                               p->twx, T);
                       check_launch();
                     });
@@ -623,7 +740,7 @@ template <int N>
 struct RunAdjY {
   static void run(hipStream_t st, int Nx, int L, const float2* T, const fhs_nufft* p,
                   const float* scale, float* out) {
-    k_adj_y<N><<<dim3(Nx, L), nt_y<N>(), 0, st>>>(T, p->sy, p->sx, p->Ny, p->Nx, p->twy, scale, out);
+    k_adj_y<N><<<dim3((Nx + 1) / 2, L), nt_y<N>(), 0, st>>>(T, p->sy, p->sx, p->Ny, p->Nx, p->twy, scale, out);
   }
 };
 
@@ -644,7 +761,7 @@ float2* twiddles(int n) {
 // 16 16 4 5) run the same register Stockham stages with the length known at
 // run time: radix 16 while N/NS divides by 16, then the remaining power of
 // two, then radix 5 and 3 stages (dft3 / dft5 below).  Each thread holds up
-// to ceil(16 / R) butterflies of a radix-R stage; the x-passes use the same
+// to ceil(PT / R) butterflies of a radix-R stage; the x-passes use the same
 // core on B rows per workgroup (no split form).
 __device__ __forceinline__ int fft_radix_rt(int rem) {
   if (rem % 16 == 0) return 16;
@@ -696,10 +813,10 @@ __device__ __forceinline__ void dft_any(float2* v) {
     dft_reg<R, INV>(v);
 }
 
-template <int R, bool INV, class Load, class Store>
+template <int PT, int R, bool INV, class Load, class Store>
 __device__ __forceinline__ void fft_stage_rt(float2* s, const float2* __restrict__ tw, int N, int NS, int B, int NT,
                                              bool first, bool last, Load& load, Store& store) {
-  constexpr int PMAX = (16 + R - 1) / R;   // butterflies per thread (NT >= B N / 16)
+  constexpr int PMAX = (PT + R - 1) / R;   // butterflies per thread (NT >= B N / PT)
   const int NBF = B * N / R;
   const int TS = N / (NS * R);
   float2 v[PMAX][R];
@@ -746,95 +863,135 @@ __device__ __forceinline__ void fft_stage_rt(float2* s, const float2* __restrict
   if (!last) __syncthreads();
 }
 
-template <bool INV, class Load, class Store>
-__device__ void fft_rt(float2* s, const float2* __restrict__ tw, int N, int B, int NT, Load& load, Store& store) {
+template <int PT, bool INV, class Load, class Store>
+__device__ __forceinline__ void fft_rt(float2* s, const float2* __restrict__ tw, int N, int B, int NT, Load& load, Store& store) {
   int ns = 1;
   bool first = true;
   while (ns < N) {
     const int R = fft_radix_rt(N / ns);
     const bool last = ns * R == N;
     switch (R) {
-      case 16: fft_stage_rt<16, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
-      case 8: fft_stage_rt<8, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
-      case 4: fft_stage_rt<4, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
-      case 2: fft_stage_rt<2, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
-      case 5: fft_stage_rt<5, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
-      default: fft_stage_rt<3, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
+      case 16: fft_stage_rt<PT, 16, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
+      case 8: fft_stage_rt<PT, 8, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
+      case 4: fft_stage_rt<PT, 4, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
+      case 2: fft_stage_rt<PT, 2, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
+      case 5: fft_stage_rt<PT, 5, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
+      default: fft_stage_rt<PT, 3, INV>(s, tw, N, ns, B, NT, first, last, load, store); break;
     }
     ns *= R;
     first = false;
   }
 }
 
-// threads and LDS bytes of a runtime-length workgroup of B transforms
+// Values per thread of a runtime-length workgroup of B transforms, its threads and LDS
+// bytes.  As few values as 1024 threads allow: the stages are a chain of
+// latencies, which more threads shorten (one 1000 x 1440 grid: y-passes 36 -> 24 and 36 ->
+// 20 us, x-passes 50 -> 36, with the column pairs and mirrored rows).
+inline int fft_rt_values(int N, int B) { return B * N <= 4096 ? 4 : B * N <= 8192 ? 8 : 16; }
 inline int fft_rt_threads(int N, int B) {
-  const int t = (B * N + 15) / 16;
+  const int t = (int)cdiv(B * N, fft_rt_values(N, B));
   return std::max(64, (t + 63) / 64 * 64);
 }
 inline size_t fft_rt_lds(int N, int B) { return ((size_t)fft_pad(N) * B + B) * sizeof(float2); }
-// rows per runtime x-pass workgroup: 4, 2 or 1, dividing the other axis, with
-// one radix-16 butterfly per thread (B N <= 16384) and the rows in LDS
-inline int fft_rt_rows(int N, int other) {
-  for (int B : {4, 2, 1})
-    if (other % B == 0 && B * N <= 16384 && fft_rt_lds(N, B) <= 150 * 1024) return B;
+template <class F>
+void with_values(int v, F&& f) {
+  if (v == 4)
+    f(std::integral_constant<int, 4>{});
+  else if (v == 8)
+    f(std::integral_constant<int, 8>{});
+  else
+    f(std::integral_constant<int, 16>{});
+}
+// rows per runtime x-pass workgroup: 4, 2 or 1, with one radix-16 butterfly per
+// thread (B N <= 16384) and the rows in LDS, fewer while CUs would stay idle.
+inline int fft_rt_rows(int N, int rows, int L) {
+  for (int B : {4, 2})
+    if (B * N <= 16384 && fft_rt_lds(N, B) <= 150 * 1024 && (int64_t)cdiv(rows, B) * L >= 256) return B;
   return 1;
 }
 
+template <int PT>
 __global__ __launch_bounds__(1024) void k_fwd_y_rt(const float* __restrict__ x, const float* __restrict__ sy,
                                                    const float* __restrict__ sx, int Ny, int Nx, int N,
-                                                   const float2* __restrict__ tw, float2* __restrict__ T) {
+                                                   const float2* __restrict__ tw, float2* __restrict__ Z) {
   extern __shared__ __align__(16) float2 s_rt[];
-  const int ix = blockIdx.x, l = blockIdx.y;
-  const float* __restrict__ xc = x + ((size_t)l * Nx + ix) * Ny;
-  const float scx = sx[ix];
-  float2* __restrict__ out = T + ((size_t)l * Nx + ix) * N;
+  const int ix = 2 * blockIdx.x, l = blockIdx.y, two = ix + 1 < Nx;
+  const float* __restrict__ xa = x + ((size_t)l * Nx + ix) * Ny;
+  const float* __restrict__ xb = xa + (two ? Ny : 0);
+  const float sa = 0.5f * sx[ix], sb = two ? 0.5f * sx[ix + 1] : 0.f;
+  float2* __restrict__ out = Z + ((size_t)l * gridDim.x + blockIdx.x) * N;
   auto load = [&](int, int, int, int n) {
-    return n < Ny ? make_float2(xc[n] * sy[n] * scx, 0.f) : make_float2(0.f, 0.f);
+    return n < Ny ? make_float2(xa[n] * sy[n] * sa, two ? xb[n] * sy[n] * sb : 0.f) : make_float2(0.f, 0.f);
   };
   auto store = [&](int, int, int, int n, float2 v) { out[n] = v; };
-  fft_rt<false>(s_rt, tw, N, 1, blockDim.x, load, store);
+  fft_rt<PT, false>(s_rt, tw, N, 1, blockDim.x, load, store);
 }
 
-__global__ __launch_bounds__(1024) void k_adj_y_rt(const float2* __restrict__ T, const float* __restrict__ sy,
+template <int PT>
+__global__ __launch_bounds__(1024) void k_adj_y_rt(const float2* __restrict__ U, const float* __restrict__ sy,
                                                    const float* __restrict__ sx, int Ny, int Nx, int N,
                                                    const float2* __restrict__ tw, const float* __restrict__ scale,
                                                    float* __restrict__ out) {
   extern __shared__ __align__(16) float2 s_rt[];
-  const int ix = blockIdx.x, l = blockIdx.y;
-  const float2* __restrict__ Tc = T + ((size_t)l * Nx + ix) * N;
-  const float sc = (scale ? scale[l] : 1.f) * sx[ix];
+  const int ix = 2 * blockIdx.x, l = blockIdx.y, hs = half_stride(N);
+  const bool two = ix + 1 < Nx;
+  const float2* __restrict__ ua = U + ((size_t)l * Nx + ix) * hs;
+  const float2* __restrict__ ub = two ? ua + hs : nullptr;
+  const float sc = 0.5f * (scale ? scale[l] : 1.f), sa = sc * sx[ix], sb = two ? sc * sx[ix + 1] : 0.f;
   float* __restrict__ o = out + ((size_t)l * Nx + ix) * Ny;
-  auto load = [&](int, int, int, int n) { return Tc[n]; };
+  auto load = [&](int, int, int, int n) { return join_pair(ua, ub, N, n); };
   auto store = [&](int, int, int, int n, float2 v) {
-    if (n < Ny) o[n] = sc * sy[n] * v.x;
+    if (n < Ny) {
+      o[n] = sa * sy[n] * v.x;
+      if (two) o[Ny + n] = sb * sy[n] * v.y;
+    }
   };
-  fft_rt<true>(s_rt, tw, N, 1, blockDim.x, load, store);
+  fft_rt<PT, true>(s_rt, tw, N, 1, blockDim.x, load, store);
 }
 
-__global__ __launch_bounds__(1024) void k_fwd_x_rt(const float2* __restrict__ T, int Kty, int Nx, int N, int B,
+template <int PT>
+__global__ __launch_bounds__(1024) void k_fwd_x_rt(const float2* __restrict__ Z, int Kty, int Nx, int N, int B,
                                                    const float2* __restrict__ tw, float2* __restrict__ Fx) {
   extern __shared__ __align__(16) float2 s_rt[];
-  const int ky0 = blockIdx.x * B, l = blockIdx.y;
-  const float2* __restrict__ Tl = T + (size_t)l * Nx * Kty;
+  const int ky0 = xpass_eighth_row0(B), l = blockIdx.y;
+  if (2 * ky0 > Kty) return;
+  const float2* __restrict__ Zl = Z + (size_t)l * ((Nx + 1) / 2) * Kty;
   float2* __restrict__ F = Fx + (size_t)l * N * Kty;
   auto load = [&](int, int, int b, int n) {
-    return n < Nx ? Tl[(size_t)n * Kty + ky0 + b] : make_float2(0.f, 0.f);
+    const int ky = ky0 + b;
+    if (n >= Nx || 2 * ky > Kty) return make_float2(0.f, 0.f);
+    const float2* __restrict__ zp = Zl + (size_t)(n >> 1) * Kty;
+    float2 a, c;
+    split_pair(zp[ky], zp[ky ? Kty - ky : 0], a, c);
+    return n & 1 ? c : a;
   };
-  auto store = [&](int, int, int b, int n, float2 v) { F[(size_t)n * Kty + ky0 + b] = v; };
-  fft_rt<false>(s_rt, tw, N, B, blockDim.x, load, store);
+  auto store = [&](int, int, int b, int n, float2 v) {
+    const int ky = ky0 + b;
+    if (2 * ky > Kty) return;
+    F[(size_t)n * Kty + ky] = v;
+    if (ky && 2 * ky < Kty) F[(size_t)(n ? N - n : 0) * Kty + Kty - ky] = make_float2(v.x, -v.y);
+  };
+  fft_rt<PT, false>(s_rt, tw, N, B, blockDim.x, load, store);
 }
 
+template <int PT>
 __global__ __launch_bounds__(1024) void k_adj_x_rt(const float2* __restrict__ g, int Kty, int Nx, int N, int B,
-                                                   const float2* __restrict__ tw, float2* __restrict__ T) {
+                                                   const float2* __restrict__ tw, float2* __restrict__ U) {
   extern __shared__ __align__(16) float2 s_rt[];
-  const int ky0 = blockIdx.x * B, l = blockIdx.y;
+  const int ky0 = xpass_eighth_row0(B), l = blockIdx.y, hs = half_stride(Kty);
+  if (2 * ky0 > Kty) return;
   const float2* __restrict__ gl = g + (size_t)l * N * Kty;
-  float2* __restrict__ Tl = T + (size_t)l * Nx * Kty;
-  auto load = [&](int, int, int b, int n) { return gl[(size_t)n * Kty + ky0 + b]; };
-  auto store = [&](int, int, int b, int n, float2 v) {
-    if (n < Nx) Tl[(size_t)n * Kty + ky0 + b] = v;
+  float2* __restrict__ Ul = U + (size_t)l * Nx * hs;
+  auto load = [&](int, int, int b, int n) {
+    const int ky = ky0 + b;
+    if (2 * ky > Kty) return make_float2(0.f, 0.f);
+    return hermitian(gl[(size_t)n * Kty + ky], gl[(size_t)(n ? N - n : 0) * Kty + (ky ? Kty - ky : 0)]);
   };
-  fft_rt<true>(s_rt, tw, N, B, blockDim.x, load, store);
+  auto store = [&](int, int, int b, int n, float2 v) {
+    const int ky = ky0 + b;
+    if (n < Nx && 2 * ky <= Kty) Ul[(size_t)n * hs + ky] = v;
+  };
+  fft_rt<PT, true>(s_rt, tw, N, B, blockDim.x, load, store);
 }
 
 inline bool is_pow2_grid(int n) { return n >= 16 && n <= 4096 && (n & (n - 1)) == 0; }
@@ -844,10 +1001,13 @@ void fwd_y_any(fhs_ctx* ctx, const fhs_nufft* p, int L, const float* x, float2* 
     dispatch_pow2<RunFwdY>(p->Kty, ctx->stream, p->Nx, L, x, p, T);
     return;
   }
-  const int nt = fft_rt_threads(p->Kty, 1);
   const size_t lds = fft_rt_lds(p->Kty, 1);
-  allow_dynamic_lds((const void*)k_fwd_y_rt, lds);
-  k_fwd_y_rt<<<dim3(p->Nx, L), nt, lds, ctx->stream>>>(x, p->sy, p->sx, p->Ny, p->Nx, p->Kty, p->twy, T);
+  with_values(fft_rt_values(p->Kty, 1), [&](auto v) {
+    constexpr int PT = decltype(v)::value;
+    allow_dynamic_lds((const void*)k_fwd_y_rt<PT>, lds);
+    k_fwd_y_rt<PT><<<dim3((p->Nx + 1) / 2, L), fft_rt_threads(p->Kty, 1), lds, ctx->stream>>>(
+        x, p->sy, p->sx, p->Ny, p->Nx, p->Kty, p->twy, T);
+  });
 }
 
 void adj_y_any(fhs_ctx* ctx, const fhs_nufft* p, int L, const float2* T, const float* scale, float* out) {
@@ -855,10 +1015,13 @@ void adj_y_any(fhs_ctx* ctx, const fhs_nufft* p, int L, const float2* T, const f
     dispatch_pow2<RunAdjY>(p->Kty, ctx->stream, p->Nx, L, T, p, scale, out);
     return;
   }
-  const int nt = fft_rt_threads(p->Kty, 1);
   const size_t lds = fft_rt_lds(p->Kty, 1);
-  allow_dynamic_lds((const void*)k_adj_y_rt, lds);
-  k_adj_y_rt<<<dim3(p->Nx, L), nt, lds, ctx->stream>>>(T, p->sy, p->sx, p->Ny, p->Nx, p->Kty, p->twy, scale, out);
+  with_values(fft_rt_values(p->Kty, 1), [&](auto v) {
+    constexpr int PT = decltype(v)::value;
+    allow_dynamic_lds((const void*)k_adj_y_rt<PT>, lds);
+    k_adj_y_rt<PT><<<dim3((p->Nx + 1) / 2, L), fft_rt_threads(p->Kty, 1), lds, ctx->stream>>>(
+        T, p->sy, p->sx, p->Ny, p->Nx, p->Kty, p->twy, scale, out);
+  });
 }
 
 void fwd_x_any(fhs_ctx* ctx, const fhs_nufft* p, int L, const float2* T, float2* F) {
@@ -866,11 +1029,14 @@ void fwd_x_any(fhs_ctx* ctx, const fhs_nufft* p, int L, const float2* T, float2*
     dispatch_pow2<RunFwdX>(p->Ktx, ctx, p->Kty, L, T, p, F);
     return;
   }
-  const int B = fft_rt_rows(p->Ktx, p->Kty);
-  const int nt = fft_rt_threads(p->Ktx, B);
+  const int B = fft_rt_rows(p->Ktx, p->Kty / 2 + 1, L);
   const size_t lds = fft_rt_lds(p->Ktx, B);
-  allow_dynamic_lds((const void*)k_fwd_x_rt, lds);
-  k_fwd_x_rt<<<dim3(p->Kty / B, L), nt, lds, ctx->stream>>>(T, p->Kty, p->Nx, p->Ktx, B, p->twx, F);
+  with_values(fft_rt_values(p->Ktx, B), [&](auto v) {
+    constexpr int PT = decltype(v)::value;
+    allow_dynamic_lds((const void*)k_fwd_x_rt<PT>, lds);
+    k_fwd_x_rt<PT><<<dim3(xpass_eighth_grid(p->Kty / 2 + 1, B), L), fft_rt_threads(p->Ktx, B), lds, ctx->stream>>>(
+        T, p->Kty, p->Nx, p->Ktx, B, p->twx, F);
+  });
 }
 
 void adj_x_any(fhs_ctx* ctx, const fhs_nufft* p, int L, const float2* g, float2* T) {
@@ -878,18 +1044,27 @@ void adj_x_any(fhs_ctx* ctx, const fhs_nufft* p, int L, const float2* g, float2*
     dispatch_pow2<RunAdjX>(p->Ktx, ctx, p->Kty, L, g, p, T);
     return;
   }
-  const int B = fft_rt_rows(p->Ktx, p->Kty);
-  const int nt = fft_rt_threads(p->Ktx, B);
+  const int B = fft_rt_rows(p->Ktx, p->Kty / 2 + 1, L);
   const size_t lds = fft_rt_lds(p->Ktx, B);
-  allow_dynamic_lds((const void*)k_adj_x_rt, lds);
-  k_adj_x_rt<<<dim3(p->Kty / B, L), nt, lds, ctx->stream>>>(g, p->Kty, p->Nx, p->Ktx, B, p->twx, T);
+  with_values(fft_rt_values(p->Ktx, B), [&](auto v) {
+    constexpr int PT = decltype(v)::value;
+    allow_dynamic_lds((const void*)k_adj_x_rt<PT>, lds);
+    k_adj_x_rt<PT><<<dim3(xpass_eighth_grid(p->Kty / 2 + 1, B), L), fft_rt_threads(p->Ktx, B), lds, ctx->stream>>>(
+        g, p->Kty, p->Nx, p->Ktx, B, p->twx, T);
+  });
+}
+
+// Z of the forward, U of the adjoint transform
+float2* nufft_workspace(fhs_ctx* ctx, const fhs_nufft* p, int L) {
+  const size_t z = (size_t)((p->Nx + 1) / 2) * p->Kty, u = (size_t)p->Nx * half_stride(p->Kty);
+  return (float2*)ctx->ws.get("nufft_T", L * std::max(z, u) * sizeof(float2));
 }
 
 }  // namespace
 
 // Used by the fused data-fidelity step.
 void nufft_forward(fhs_ctx* ctx, const fhs_nufft* p, const float* x, int L, float2* Fx) {
-  float2* T = (float2*)ctx->ws.get("nufft_T", (size_t)L * p->Nx * p->Kty * sizeof(float2));
+  float2* T = nufft_workspace(ctx, p, L);
   {
     Scope sc(ctx, "fft_fwd_y");
     fwd_y_any(ctx, p, L, x, T);
@@ -904,7 +1079,7 @@ void nufft_forward(fhs_ctx* ctx, const fhs_nufft* p, const float* x, int L, floa
 
 void nufft_adjoint(fhs_ctx* ctx, const fhs_nufft* p, const float2* g, int L, const float* scale_dev,
                    float* out) {
-  float2* T = (float2*)ctx->ws.get("nufft_T", (size_t)L * p->Nx * p->Kty * sizeof(float2));
+  float2* T = nufft_workspace(ctx, p, L);
   {
     Scope sc(ctx, "fft_adj_x");
     adj_x_any(ctx, p, L, g, T);
