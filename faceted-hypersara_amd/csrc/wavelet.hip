@@ -366,7 +366,8 @@ __global__ __launch_bounds__(256) void k_dirac(SaraGeom G, const float* __restri
       for (int l = 0; l < LREG; ++l)
         if (l < L) {
 #pragma unroll
-          for (int j = 0; j < VEC; ++j) r[l].v[j] -= f[j] * r[l].v[j];
+          for (int j = 0; j < VEC; ++j)
+            if (MODE == AN_L21) r[l].v[j] -= f[j] * r[l].v[j];
           *reinterpret_cast<Vec*>(v1 + (int64_t)l * G.s + d0 + p) = r[l];
         }
     }

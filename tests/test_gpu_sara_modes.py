@@ -50,3 +50,20 @@ def test_modes(ctx, Ny, Nx, L, nlevel):
     n = np.linalg.norm(c, axis=0)
     assert rel(wd.cpu().numpy(), 0.1 / (0.1 + n)) < TOL
     assert abs(fhs.compute_sara_prior(xd, S) / n.sum() - 1) < TOL
+
+
+@pytest.mark.parametrize('Ny,Nx', [(16, 12), (7, 5)])       # four pixels a thread, one
+def test_dirac_block_keeps_infinities(ctx, Ny, Nx):
+    """Without a threshold the Dirac coefficients are the scaled pixels, infinite
+    ones too: no product with a zero factor turns them into NaN."""
+    import fhs
+    for bases in (('db2', 'db8', 'self'), ('self',)):
+        S = fhs.SaraDictionary(ctx, Ny, Nx, bases=bases, nlevel=1)
+        x = torch.ones((2, Nx, Ny), device='cuda')
+        x[0, 1, 2], x[1, 3, 4] = float('inf'), -float('inf')
+        want = x.reshape(2, -1) * np.float32(1 / np.sqrt(len(bases)))
+        c = S.psit(x)[:, -Nx * Ny:]
+        assert torch.equal(c, want)
+        out = torch.full((2, S.s), 0.5, device='cuda')
+        S.psit(x, out=out, accumulate=True)
+        assert torch.allclose(out[:, -Nx * Ny:], want + 0.5)
