@@ -465,29 +465,34 @@ __device__ __forceinline__ void patch_mfma(const GDev& g, const int2* __restrict
   }
 }
 
-// The same sums tap by tap (the lane's four points, rows in list order).
+// The same sums tap by tap (the lane's four points, rows in list order).  Called,
+// not inlined, so it takes the members it needs by value: a reference to a matrix
+// that is a kernel argument would copy the whole of it, 240 bytes, to scratch in
+// every lane (500k rows of 15 x 15 taps on a 4096 x 4096 grid: 230 us, 100 without;
+// 1M of 7 x 7 on 2048 x 2048: 111 and 64).
 struct PatchSums {
   mfma_f4 re, im;
 };
 template <int KM, class W>
-__device__ __noinline__ PatchSums patch_exact(const GDev& g, const int2* __restrict__ ent, int n, W w) {
+__device__ __noinline__ PatchSums patch_exact(const float2* __restrict__ vals, int half, int Ky, int Kx,
+                                              const int2* __restrict__ ent, int n, W w) {
   const int lane = threadIdx.x & 63, li = lane & 15, y0 = 4 * (lane >> 4);
   auto slot = [&](int r, int j) {
     const size_t i = (size_t)r * (2 * KM) + j;
-    return g.half ? h2f(reinterpret_cast<const unsigned*>(g.vals)[i]) : g.vals[i];
+    return half ? h2f(reinterpret_cast<const unsigned*>(vals)[i]) : vals[i];
   };
   mfma_f4 cre = {0.f, 0.f, 0.f, 0.f}, cim = cre;
   for (int e = 0; e < n; ++e) {
     const int r = ent[e].x, pk = ent[e].y;
     const int dy = (int)(signed char)(pk & 0xff), dx = (int)(signed char)((pk >> 8) & 0xff);
     const int jx = li - dx;
-    if ((unsigned)jx >= (unsigned)g.Kx) continue;
+    if ((unsigned)jx >= (unsigned)Kx) continue;
     const float2 v = w(r), c = slot(r, KM + jx);
     const float2 q = make_float2(c.x * v.x + c.y * v.y, c.x * v.y - c.y * v.x);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int jy = y0 + i - dy;
-      if ((unsigned)jy < (unsigned)g.Ky) {
+      if ((unsigned)jy < (unsigned)Ky) {
         const float2 a = slot(r, jy);
         cre[i] += a.x * q.x + a.y * q.y;
         cim[i] += a.x * q.y - a.y * q.x;
@@ -535,7 +540,7 @@ __device__ __forceinline__ void g_adjoint_patches(const GDev& g, int unit, const
   for (int r = 0; r < 4; ++r) bad = bad || !isfinite(cre[r]) || !isfinite(cim[r]);
   if (__any(bad)) {
     auto wr = [=](int r) { return LAM ? cscale(w[r], lam[r]) : w[r]; };
-    const PatchSums e = patch_exact<KM>(g, ent, n, wr);
+    const PatchSums e = patch_exact<KM>(g.vals, g.half, g.Ky, g.Kx, ent, n, wr);
     cre = e.re;
     cim = e.im;
   }
