@@ -41,6 +41,12 @@ class Conv3x3:
         return [(self.W, self.dW, self.mW, self.vW), (self.b, self.db, self.mb, self.vb)]
 
     def forward(self, x, NB, H, W, keep=True):
+        """x: (cin, NB*H*W) float32; with keep, backward may follow, also after
+        the caller has reused x (it reads a copy)."""
+        return self._forward(x.clone() if keep else x, NB, H, W, keep)
+
+    def _forward(self, x, NB, H, W, keep):
+        """forward of an x that nobody writes to before backward."""
         ctx = self.ctx
         y = torch.empty((self.cout, NB * H * W), dtype=torch.float32, device=ctx.device)
         ctx.check(lib().fhs_nn_conv3x3(ctx.h, _f(x), self.cin, NB, H, W, _f(self.W), self.cout, _f(self.b),
@@ -134,7 +140,7 @@ class UNet:
             h = h.clone()        # backward reads it again: the caller may reuse x meanwhile
         skips = []
         for i, (a, b) in enumerate(self.enc):
-            h = b.forward(a.forward(h, NB, Hc, Wc, keep), NB, Hc, Wc, keep)
+            h = b._forward(a._forward(h, NB, Hc, Wc, keep), NB, Hc, Wc, keep)
             if i < len(self.enc) - 1:
                 skips.append(h)
                 h = self._pool(h, self.widths[i], NB, Hc, Wc)
@@ -143,11 +149,11 @@ class UNet:
             i = len(self.widths) - 2 - j
             hu = self._up(h, self.widths[i + 1], NB, Hc, Wc)
             Hc, Wc = Hc * 2, Wc * 2
-            hu = u.forward(hu, NB, Hc, Wc, keep)
+            hu = u._forward(hu, NB, Hc, Wc, keep)
             cat = torch.cat([hu, skips[i]], dim=0)
-            h = b.forward(a.forward(cat, NB, Hc, Wc, keep), NB, Hc, Wc, keep)
+            h = b._forward(a._forward(cat, NB, Hc, Wc, keep), NB, Hc, Wc, keep)
         self._skips = skips if keep else None
-        return self.head.forward(h, NB, Hc, Wc, keep)
+        return self.head._forward(h, NB, Hc, Wc, keep)
 
     def backward(self, g, NB, H, W):
         """g: gradient of the loss w.r.t. the output; accumulates the

@@ -158,3 +158,25 @@ def test_conv3x3(ctx, cin, cout, NB, H, W, relu):
                                 None, 0), 'gemm')
     ctx.check(lib().fhs_nn_col2im3(ctx.h, _ptr(cd), cin, NB, H, W, _ptr(xg)), 'col2im')
     assert torch.equal(dx, xg)
+
+
+@pytest.mark.parametrize('net', [False, True])
+def test_backward_after_the_input_was_reused(ctx, net):
+    """A layer's, and the network's, gradients are those of the input that forward
+    saw: writing to that tensor before backward changes none of them."""
+    from fhs.unet import Conv3x3, UNet
+    NB, H, W = 1, 8, 16
+    rng = np.random.default_rng(11)
+    x, gy = (dev(rng.normal(size=(8, NB * H * W))) for _ in range(2))
+    grads = []
+    for reuse in (False, True):
+        m = UNet(ctx, 8, 8, widths=(8, 8), seed=2) if net else Conv3x3(ctx, 8, 8, True, np.random.default_rng(2))
+        xin = x.clone()
+        m.forward(xin, NB, H, W)
+        if reuse:
+            xin.zero_()
+        dx = m.backward(gy.clone(), NB, H, W) if net else m.backward(gy.clone())
+        layers = m.layers() if net else [m]
+        grads.append([dx] + [t.clone() for p in layers for t in (p.dW, p.db)])
+    assert all(torch.equal(a, b) for a, b in zip(*grads))
+    assert all(float(g.abs().max()) > 0 for g in grads[0])
