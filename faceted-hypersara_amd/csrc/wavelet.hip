@@ -13,6 +13,7 @@
 // k_analysis and k_synthesis); the l21 step is part of the analysis.
 #include <algorithm>
 #include <cmath>
+#include <memory>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -38,12 +39,60 @@ struct SaraGeom {
   float lo[WMAX_BASES][WMAX_LF];         // reconstruction low-pass; high-pass (-1)^j lo[lf - 1 - j]
 };
 
+// What a launch on one level reads of it, by value: a launch or a captured graph
+// then needs the dictionary no more.  A workgroup's share is the few fields in
+// front and the 120 bytes of its basis, two or three lines of the arguments: as
+// fast as a copy in device memory (dual step of 128 x 128 67 us, 1024 x 1024 x 16
+// 925 against 940), where the whole geometry by value, 2 KB with every field of a
+// basis in another line, took 1.2 us more a launch (73 us).
+struct SaraLevel {
+  int lf;                 // taps
+  int ny, nx, py, px;     // shapes of levels k and k - 1
+  int64_t hoff;           // H_k (V_k, D_k follow) in a channel's coefficients
+  int64_t aoff;           // A_J
+  int64_t fine, coarse;   // scratch offsets of the approximations of levels k - 1 and k
+  float lo[WMAX_LF];
+};
+struct SaraArgs {
+  int Ny, Nx, nlevel, nb, dirac, k;
+  float norm;
+  int64_t s, scr_per_chan, dstart;
+  SaraLevel b[WMAX_BASES];
+};
+
+SaraArgs level_args(const SaraGeom& G, int k) {
+  SaraArgs A{};
+  A.Ny = G.Ny;
+  A.Nx = G.Nx;
+  A.nlevel = G.nlevel;
+  A.nb = G.nb;
+  A.dirac = G.dirac;
+  A.k = k;
+  A.norm = G.norm;
+  A.s = G.s;
+  A.scr_per_chan = G.scr_per_chan;
+  A.dstart = G.boff[G.nb];
+  for (int b = 0; b < G.nb; ++b) {
+    SaraLevel& B = A.b[b];
+    B.lf = G.lf[b];
+    B.ny = G.ny[b][k];
+    B.nx = G.nx[b][k];
+    B.py = G.ny[b][k - 1];
+    B.px = G.nx[b][k - 1];
+    B.hoff = G.boff[b] + G.doff[b][k];
+    B.aoff = G.boff[b] + G.aoff[b];
+    B.fine = G.scr[b][k - 1];
+    B.coarse = G.scr[b][k];
+    for (int j = 0; j < B.lf; ++j) B.lo[j] = G.lo[b][j];
+  }
+  return A;
+}
+
 }  // namespace fhs
 
 struct fhs_sara {
-  int device = 0;
   fhs::SaraGeom g{};
-  fhs::SaraGeom* d = nullptr;   // device copy: the kernels' few fields come from L2, not from the 1 KB of arguments
+  fhs::SaraArgs level[fhs::WMAX_LEVELS + 1];   // [k], k = 1 .. nlevel
 };
 
 namespace fhs {
@@ -80,10 +129,10 @@ struct Taps {
   __device__ __forceinline__ float hi(int j) const { return j & 1 ? -f[LF - 1 - j] : f[LF - 1 - j]; }
 };
 template <int LF>
-__device__ __forceinline__ Taps<LF> load_taps(const SaraGeom& G, int b) {
+__device__ __forceinline__ Taps<LF> load_taps(const SaraLevel& G) {
   Taps<LF> t;
 #pragma unroll
-  for (int j = 0; j < LF; ++j) t.f[j] = G.lo[b][j];
+  for (int j = 0; j < LF; ++j) t.f[j] = G.lo[j];
   return t;
 }
 // element `off` bytes behind a wave-uniform base
@@ -111,7 +160,7 @@ struct AnArgs {
   double beta;
   float* wout;
   double* part;
-  int L, k;
+  int L;
 };
 
 // the l21 factor of a coefficient with norm sqrt(ss): v1 = r - f r
@@ -121,20 +170,20 @@ __device__ __forceinline__ float l21_factor(double ss, double t) {
 }
 
 template <int LF, int MODE, bool LAST>
-__device__ __forceinline__ void an_tile(const SaraGeom& G, const AnArgs& A, int b, int ky0, int kx0, float* lds) {
+__device__ __forceinline__ void an_tile(const SaraArgs& G, const SaraLevel& B, const AnArgs& A, int ky0, int kx0, float* lds) {
   constexpr int NS = LAST ? 4 : 3;        // subbands kept as coefficients: h, v, d (and a)
   constexpr int NQ = NS * AT_X;           // coefficients per lane
   constexpr int WW = 2 * AT_X + LF - 2;   // window columns
   constexpr bool NORMS = MODE >= AN_L21;
   const int lane = threadIdx.x & 63, l = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave = channel
-  const int k = A.k, iny = G.ny[b][k - 1], inx = G.nx[b][k - 1], ny = G.ny[b][k], nx = G.nx[b][k];
+  const int k = G.k, iny = B.py, inx = B.px, ny = B.ny, nx = B.nx;
   const int64_t sz = (int64_t)ny * nx;
-  const Taps<LF> T = load_taps<LF>(G, b);
+  const Taps<LF> T = load_taps<LF>(B);
   const bool live = lane < AT_Y && ky0 + lane < ny;
   const int ncol = min(AT_X, nx - kx0);
   // offsets of the kept subbands in a channel vector, of the tile, of this lane
-  const int64_t hoff = G.boff[b] + G.doff[b][k], toff = ky0 + (int64_t)ny * kx0;
-  auto soff = [&](int s) { return s == 3 ? G.boff[b] + G.aoff[b] : hoff + s * sz; };
+  const int64_t hoff = B.hoff, toff = ky0 + (int64_t)ny * kx0;
+  auto soff = [&](int s) { return s == 3 ? B.aoff : hoff + s * sz; };
   const unsigned loff = (unsigned)lane * sizeof(float), cstep = (unsigned)ny * sizeof(float);
   float* v1 = A.v1 + (int64_t)l * G.s + toff;
   // r: old coefficients, then plus the new ones (r[3]: the approximation, a coefficient
@@ -166,7 +215,7 @@ __device__ __forceinline__ void an_tile(const SaraGeom& G, const AnArgs& A, int 
   float lw[2][AT_X], hg[2][AT_X];
   {
     const int wy0 = 2 * ky0 + 2 - LF, wx0 = 2 * kx0 + 2 - LF;
-    const float* img = (k == 1 ? A.x + (int64_t)l * iny * inx : A.scr + (int64_t)l * G.scr_per_chan + G.scr[b][k - 1]) +
+    const float* img = (k == 1 ? A.x + (int64_t)l * iny * inx : A.scr + (int64_t)l * G.scr_per_chan + B.fine) +
                        (int64_t)iny * wx0;
     const float scale = k == 1 ? G.norm : 1.f;
     const bool inside = wx0 >= 0 && wx0 + WW <= inx;
@@ -238,7 +287,7 @@ __device__ __forceinline__ void an_tile(const SaraGeom& G, const AnArgs& A, int 
     }
   }
   if (!LAST && live) {
-    float* ak = A.scr + (int64_t)l * G.scr_per_chan + G.scr[b][k] + toff;
+    float* ak = A.scr + (int64_t)l * G.scr_per_chan + B.coarse + toff;
 #pragma unroll
     for (int q = 0; q < AT_X; ++q)
       if (q < ncol) at_bytes(ak, loff + q * cstep) = r[3][q];
@@ -297,26 +346,24 @@ __device__ __forceinline__ void an_tile(const SaraGeom& G, const AnArgs& A, int 
 // fastest), each tile's bases one after the other, so the image window the
 // bases share and the lines two tiles of a column share meet in one L2.
 template <int MODE, bool LAST>
-__global__ __launch_bounds__(64 * AN_CHANNELS) void k_analysis(const SaraGeom* __restrict__ geom, AnArgs A, int ty,
-                                                                int tx) {
-  const SaraGeom& G = *geom;
+__global__ __launch_bounds__(64 * AN_CHANNELS) void k_analysis(SaraArgs G, AnArgs A, int ty, int tx) {
   extern __shared__ __align__(16) float an_lds[];
   const int per = (ty * tx + 7) / 8, s = blockIdx.x / 8;
   const int tile = (int)(blockIdx.x % 8) * per + s / G.nb, b = s % G.nb;
   const int ky0 = (tile % ty) * AT_Y, kx0 = (tile / ty) * AT_X;
-  if (s / G.nb >= per || ky0 >= G.ny[b][A.k] || kx0 >= G.nx[b][A.k]) {
+  if (s / G.nb >= per || ky0 >= G.b[b].ny || kx0 >= G.b[b].nx) {
     if (MODE == AN_NORM && threadIdx.x == 0) A.part[blockIdx.x] = 0.0;
     return;
   }
-  switch (G.lf[b]) {   // db1 .. db8: 2, 4, ..., 16 taps
-    case 2: an_tile<2, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
-    case 4: an_tile<4, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
-    case 6: an_tile<6, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
-    case 8: an_tile<8, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
-    case 10: an_tile<10, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
-    case 12: an_tile<12, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
-    case 14: an_tile<14, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
-    default: an_tile<16, MODE, LAST>(G, A, b, ky0, kx0, an_lds); break;
+  switch (G.b[b].lf) {   // db1 .. db8: 2, 4, ..., 16 taps
+    case 2: an_tile<2, MODE, LAST>(G, G.b[b], A, ky0, kx0, an_lds); break;
+    case 4: an_tile<4, MODE, LAST>(G, G.b[b], A, ky0, kx0, an_lds); break;
+    case 6: an_tile<6, MODE, LAST>(G, G.b[b], A, ky0, kx0, an_lds); break;
+    case 8: an_tile<8, MODE, LAST>(G, G.b[b], A, ky0, kx0, an_lds); break;
+    case 10: an_tile<10, MODE, LAST>(G, G.b[b], A, ky0, kx0, an_lds); break;
+    case 12: an_tile<12, MODE, LAST>(G, G.b[b], A, ky0, kx0, an_lds); break;
+    case 14: an_tile<14, MODE, LAST>(G, G.b[b], A, ky0, kx0, an_lds); break;
+    default: an_tile<16, MODE, LAST>(G, G.b[b], A, ky0, kx0, an_lds); break;
   }
 }
 
@@ -406,11 +453,11 @@ struct SynIn {
 };
 
 template <int LF>
-__device__ __forceinline__ void syn_tile(const SaraGeom& G, int b, const SynIn& in, int iy0, int ix0, float* pq,
+__device__ __forceinline__ void syn_tile(const SaraLevel& B, const SynIn& in, int iy0, int ix0, float* pq,
                                          float* acc) {
   constexpr int NC = ST_X / 2 + LF / 2 - 1;
   const int lane = threadIdx.x & 63;
-  const Taps<LF> T = load_taps<LF>(G, b);
+  const Taps<LF> T = load_taps<LF>(B);
   const int cy = iy0 / 2 + lane, cx0 = ix0 / 2;
   const int64_t sz = (int64_t)in.ny * in.nx, toff = (int64_t)in.ny * cx0;
   const float *ba = in.a + toff, *bh = in.h + toff, *bv = bh + sz, *bd = bv + sz;
@@ -483,17 +530,17 @@ __device__ __forceinline__ void syn_tile(const SaraGeom& G, int b, const SynIn& 
   }
 }
 
-__device__ __forceinline__ void syn_basis(const SaraGeom& G, int b, const SynIn& in, int iy0, int ix0, float* pq,
+__device__ __forceinline__ void syn_basis(const SaraLevel& B, const SynIn& in, int iy0, int ix0, float* pq,
                                           float* acc) {
-  switch (G.lf[b]) {
-    case 2: syn_tile<2>(G, b, in, iy0, ix0, pq, acc); break;
-    case 4: syn_tile<4>(G, b, in, iy0, ix0, pq, acc); break;
-    case 6: syn_tile<6>(G, b, in, iy0, ix0, pq, acc); break;
-    case 8: syn_tile<8>(G, b, in, iy0, ix0, pq, acc); break;
-    case 10: syn_tile<10>(G, b, in, iy0, ix0, pq, acc); break;
-    case 12: syn_tile<12>(G, b, in, iy0, ix0, pq, acc); break;
-    case 14: syn_tile<14>(G, b, in, iy0, ix0, pq, acc); break;
-    default: syn_tile<16>(G, b, in, iy0, ix0, pq, acc); break;
+  switch (B.lf) {
+    case 2: syn_tile<2>(B, in, iy0, ix0, pq, acc); break;
+    case 4: syn_tile<4>(B, in, iy0, ix0, pq, acc); break;
+    case 6: syn_tile<6>(B, in, iy0, ix0, pq, acc); break;
+    case 8: syn_tile<8>(B, in, iy0, ix0, pq, acc); break;
+    case 10: syn_tile<10>(B, in, iy0, ix0, pq, acc); break;
+    case 12: syn_tile<12>(B, in, iy0, ix0, pq, acc); break;
+    case 14: syn_tile<14>(B, in, iy0, ix0, pq, acc); break;
+    default: syn_tile<16>(B, in, iy0, ix0, pq, acc); break;
   }
 }
 
@@ -503,11 +550,9 @@ __device__ __forceinline__ void syn_basis(const SaraGeom& G, int b, const SynIn&
 // the finest level, each taking a pair of bases with the same number of taps in
 // all, and add their sums in wave order.
 template <bool FINEST, bool SPLIT>
-__global__ __launch_bounds__(64 * ST_WAVES) void k_synthesis(const SaraGeom* __restrict__ geom, int k, int ty,
-                                                             int tx, int nz, const float* __restrict__ v1,
-                                                             float* __restrict__ scr, float scale,
-                                                             float* __restrict__ out) {
-  const SaraGeom& G = *geom;
+__global__ __launch_bounds__(64 * ST_WAVES) void k_synthesis(SaraArgs G, int ty, int tx, int nz,
+                                                             const float* __restrict__ v1, float* __restrict__ scr,
+                                                             float scale, float* __restrict__ out) {
   __shared__ float lds[ST_WAVES][2 * ST_X * ST_LD];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int txg = SPLIT ? tx : (tx + ST_WAVES - 1) / ST_WAVES;
@@ -518,7 +563,7 @@ __global__ __launch_bounds__(64 * ST_WAVES) void k_synthesis(const SaraGeom* __r
   const int z = id / (ty * txg), t = id % (ty * txg);
   const int iy0 = (t / txg) * ST_Y, ix0 = (SPLIT ? t % txg : (t % txg) * ST_WAVES + wv) * ST_X;
   const int b0 = FINEST ? 0 : z % G.nb, l = FINEST ? z : z / G.nb;
-  const int py = FINEST ? G.Ny : G.ny[b0][k - 1], px = FINEST ? G.Nx : G.nx[b0][k - 1];
+  const int py = FINEST ? G.Ny : G.b[b0].py, px = FINEST ? G.Nx : G.b[b0].px;
   if (!SPLIT && (iy0 >= py || ix0 >= px)) return;
   const float* v1l = v1 + (int64_t)l * G.s;
   float* sc = scr + (int64_t)l * G.scr_per_chan;
@@ -528,11 +573,12 @@ __global__ __launch_bounds__(64 * ST_WAVES) void k_synthesis(const SaraGeom* __r
   for (int q = 0; q < ST_PER; ++q) acc[q] = 0.f;
   auto one = [&](int b) {
     SynIn in;
-    in.a = k == G.nlevel ? v1l + G.boff[b] + G.aoff[b] : sc + G.scr[b][k];
-    in.h = v1l + G.boff[b] + G.doff[b][k];
-    in.ny = G.ny[b][k];
-    in.nx = G.nx[b][k];
-    syn_basis(G, b, in, iy0, ix0, pq, acc);
+    const SaraLevel& B = G.b[b];
+    in.a = G.k == G.nlevel ? v1l + B.aoff : sc + B.coarse;
+    in.h = v1l + B.hoff;
+    in.ny = B.ny;
+    in.nx = B.nx;
+    syn_basis(B, in, iy0, ix0, pq, acc);
   };
   if constexpr (!FINEST) {
     one(b0);
@@ -554,8 +600,8 @@ __global__ __launch_bounds__(64 * ST_WAVES) void k_synthesis(const SaraGeom* __r
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
-  float* dst = FINEST ? out + (int64_t)l * G.Ny * G.Nx : sc + G.scr[b0][k - 1];
-  const float* dir = v1l + G.boff[G.nb];
+  float* dst = FINEST ? out + (int64_t)l * G.Ny * G.Nx : sc + G.b[b0].fine;
+  const float* dir = v1l + G.dstart;
   auto store = [&](int e, float v) {
     const int iy = iy0 + e % ST_Y, ix = ix0 + e / ST_Y;
     if (iy >= py || ix >= px) return;
@@ -654,14 +700,14 @@ unsigned analysis_grid(const SaraGeom& G, int k, int& ty, int& tx) {
 }
 
 template <int MODE>
-void launch_analysis(fhs_ctx* ctx, const fhs_sara* S, const AnArgs& A, unsigned grid, int ty, int tx) {
+void launch_analysis(fhs_ctx* ctx, const fhs_sara* S, int k, const AnArgs& A, unsigned grid, int ty, int tx) {
   // LDS: the turning tiles, or every channel's coefficients and the factors
-  const bool last = A.k == S->g.nlevel;
+  const bool last = k == S->g.nlevel;
   const size_t nq = (last ? 4 : 3) * AT_X * 64;
   const size_t lds = std::max<size_t>(A.L * AT_LH, MODE >= AN_L21 ? (A.L + 1) * nq : 0) * sizeof(float);
   auto go = [&](auto kern) {
     allow_dynamic_lds((const void*)kern, lds);
-    kern<<<grid, 64 * A.L, lds, ctx->stream>>>(S->d, A, ty, tx);
+    kern<<<grid, 64 * A.L, lds, ctx->stream>>>(S->level[k], A, ty, tx);
     check_launch();
   };
   last ? go(k_analysis<MODE, true>) : go(k_analysis<MODE, false>);
@@ -688,9 +734,8 @@ unsigned sara_analyse(fhs_ctx* ctx, const fhs_sara* S, const float* x, int L, fl
     for (int k = 1; k <= G.nlevel && G.nb > 0; ++k) {
       int ty, tx;
       const unsigned grid = analysis_grid(G, k, ty, tx);
-      A.k = k;
       A.part = part ? part + nsum : nullptr;
-      launch_analysis<MODE>(ctx, S, A, grid, ty, tx);
+      launch_analysis<MODE>(ctx, S, k, A, grid, ty, tx);
       nsum += grid;
     }
     if (G.dirac) {
@@ -722,16 +767,16 @@ void sara_synthesis(fhs_ctx* ctx, const fhs_sara* S, const float* v1, int L, flo
     }
     const int ty = (int)cdiv(py, ST_Y), tx = (int)cdiv(px, ST_X);
     k_synthesis<false, false><<<grid(ty, (int)cdiv(tx, ST_WAVES), G.nb * L), 64 * ST_WAVES, 0, ctx->stream>>>(
-        S->d, k, ty, tx, G.nb * L, v1, scr, scale, out);
+        S->level[k], ty, tx, G.nb * L, v1, scr, scale, out);
     check_launch();
   }
   const int ty = (int)cdiv(G.Ny, ST_Y), tx = (int)cdiv(G.Nx, ST_X);
   if ((int64_t)ty * tx * L < SYN_SPLIT_BELOW)
-    k_synthesis<true, true><<<grid(ty, tx, L), 64 * ST_WAVES, 0, ctx->stream>>>(S->d, 1, ty, tx, L, v1, scr, scale,
+    k_synthesis<true, true><<<grid(ty, tx, L), 64 * ST_WAVES, 0, ctx->stream>>>(S->level[1], ty, tx, L, v1, scr, scale,
                                                                                        out);
   else
     k_synthesis<true, false><<<grid(ty, (int)cdiv(tx, ST_WAVES), L), 64 * ST_WAVES, 0, ctx->stream>>>(
-        S->d, 1, ty, tx, L, v1, scr, scale, out);
+        S->level[1], ty, tx, L, v1, scr, scale, out);
   check_launch();
 }
 
@@ -770,8 +815,7 @@ int fhs_sara_create_host(fhs_ctx* ctx, int Ny, int Nx, int nlevel, int nbases,
     FHS_CHECK(nlevel >= 1 && nlevel <= WMAX_LEVELS, "sara_create: nlevel must be in [1, 6]");
     FHS_CHECK(nbases >= 0 && nbases <= WMAX_BASES, "sara_create: at most 8 wavelet bases");
     FHS_CHECK(nbases + (with_dirac ? 1 : 0) >= 1, "sara_create: empty dictionary");
-    fhs_sara* S = new fhs_sara();
-    S->device = ctx->device;
+    auto S = std::make_unique<fhs_sara>();
     SaraGeom& G = S->g;
     G.Ny = Ny;
     G.Nx = Nx;
@@ -812,18 +856,12 @@ int fhs_sara_create_host(fhs_ctx* ctx, int Ny, int Nx, int nlevel, int nbases,
     G.boff[nbases] = off;
     G.s = off + (G.dirac ? (int64_t)Ny * Nx : 0);
     G.scr_per_chan = soff;
-    FHS_HIP(hipSetDevice(ctx->device));
-    FHS_HIP(hipMalloc(&S->d, sizeof(SaraGeom)));
-    FHS_HIP(hipMemcpy(S->d, &G, sizeof(SaraGeom), hipMemcpyHostToDevice));
-    *out = S;
+    for (int k = 1; k <= nlevel; ++k) S->level[k] = level_args(G, k);
+    *out = S.release();
   });
 }
 
 int fhs_sara_destroy(fhs_sara* S) {
-  if (S && S->d) {
-    (void)hipSetDevice(S->device);
-    (void)hipFree(S->d);
-  }
   delete S;
   return FHS_OK;
 }

@@ -67,3 +67,39 @@ def test_dirac_block_keeps_infinities(ctx, Ny, Nx):
         out = torch.full((2, S.s), 0.5, device='cuda')
         S.psit(x, out=out, accumulate=True)
         assert torch.allclose(out[:, -Nx * Ny:], want + 0.5)
+
+
+@pytest.mark.parametrize('L', [3, 17])
+def test_captured_step_outlives_its_dictionary(L):
+    """A captured dual step needs its dictionary no more, which may also be created
+    and dropped while the capture runs: replays give the eager step."""
+    import gc
+    import fhs
+    ctx = fhs.Context(0)
+    Ny, Nx = 60, 41
+    rng = np.random.default_rng(L)
+    x = torch.from_numpy(rng.random((L, Nx, Ny)).astype(np.float32)).cuda()
+    S = fhs.SaraDictionary(ctx, Ny, Nx, nlevel=2)
+    v0 = torch.from_numpy(rng.standard_normal((L, S.s)).astype(np.float32)).cuda()
+
+    def step(S, v):
+        return fhs.hs_update_dual_sparsity_distributed(v, S, S, x, None, 0.8, 0.3)
+
+    want = [t.clone() for t in step(S, v0.clone())]      # also sizes the context's workspace
+    v = v0.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ctx.bind_stream()
+        D = fhs.SaraDictionary(ctx, Ny, Nx, nlevel=2)
+        got = step(D, v)
+        del D
+        gc.collect()
+    ctx.bind_stream()
+    for seed in range(4):
+        v.copy_(v0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+        again = step(S, v0.clone())                        # eager work between the replays
+        assert torch.equal(again[0], want[0]) and torch.equal(again[1], want[1])
