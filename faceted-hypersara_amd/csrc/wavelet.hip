@@ -175,7 +175,9 @@ __device__ __forceinline__ void an_tile(const SaraArgs& G, const SaraLevel& B, c
   constexpr int NQ = NS * AT_X;           // coefficients per lane
   constexpr int WW = 2 * AT_X + LF - 2;   // window columns
   constexpr bool NORMS = MODE >= AN_L21;
-  const int lane = threadIdx.x & 63, l = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave = channel
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave = channel
+  const int l = NORMS ? wv : (int)(blockIdx.y * (blockDim.x >> 6)) + wv;
+  if (!NORMS && l >= A.L) return;
   const int k = G.k, iny = B.py, inx = B.px, ny = B.ny, nx = B.nx;
   const int64_t sz = (int64_t)ny * nx;
   const Taps<LF> T = load_taps<LF>(B);
@@ -250,7 +252,7 @@ __device__ __forceinline__ void an_tile(const SaraArgs& G, const SaraLevel& B, c
     }
   }
   // y filter, AT_PAIR columns at a time: output ky0 + lane from rows 2 lane .. 2 lane + LF - 1
-  float* lh = lds + l * AT_LH;
+  float* lh = lds + wv * AT_LH;
   float* dst = lh + (lane & 1) * AT_LD + (lane >> 1);   // row lane; row lane + 64 is 32 further
   const float* src = lh + min(lane, AT_Y - 1);
 #pragma unroll
@@ -314,7 +316,7 @@ __device__ __forceinline__ void an_tile(const SaraArgs& G, const SaraLevel& B, c
 #pragma unroll
     for (int s = 0; s < NS; ++s)
 #pragma unroll
-      for (int q = 0; q < AT_X; ++q) vals[(l * NQ + s * AT_X + q) * 64 + lane] = r[s][q];
+      for (int q = 0; q < AT_X; ++q) vals[(wv * NQ + s * AT_X + q) * 64 + lane] = r[s][q];
     __syncthreads();
     double tot[1] = {0.0};
     for (int e = threadIdx.x; e < NQ * 64; e += blockDim.x) {
@@ -368,7 +370,7 @@ __global__ __launch_bounds__(64 * AN_CHANNELS) void k_analysis(SaraArgs G, AnArg
 }
 
 // The Dirac block: r_l = v1_l + x_l / sqrt(P) (v1 absent in AN_WEIGHT, AN_NORM and
-// AN_SET), then as the modes say.  VEC consecutive pixels per thread with wide
+// AN_SET), then as the modes say, for the 16 channels from 16 blockIdx.y.  VEC consecutive pixels per thread with wide
 // accesses when the block is 16-byte aligned in every channel.
 template <int MODE, int VEC>
 __global__ __launch_bounds__(256) void k_dirac(SaraGeom G, const float* __restrict__ x, float* __restrict__ v1, int L,
@@ -380,10 +382,13 @@ __global__ __launch_bounds__(256) void k_dirac(SaraGeom G, const float* __restri
   constexpr bool KEEP = MODE == AN_ADD || MODE == AN_L21;
   __shared__ double sh[256 / 64];
   const int64_t N = (int64_t)G.Ny * G.Nx, d0 = G.boff[G.nb];
+  x += (int64_t)blockIdx.y * AN_CHANNELS * N;
+  if (KEEP || MODE == AN_SET) v1 += (int64_t)blockIdx.y * AN_CHANNELS * G.s;
+  L = min(L - (int)blockIdx.y * AN_CHANNELS, AN_CHANNELS);
   double tot[1] = {0.0};
   for (int64_t p = VEC * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x); p < N;
        p += VEC * (int64_t)gridDim.x * blockDim.x) {
-    constexpr int LREG = 16;   // channels kept in registers between the norm and the update
+    constexpr int LREG = AN_CHANNELS;   // channels kept in registers between the norm and the update
     Vec r[LREG];
     double ss[VEC];
 #pragma unroll
@@ -701,20 +706,24 @@ unsigned analysis_grid(const SaraGeom& G, int k, int& ty, int& tx) {
 
 template <int MODE>
 void launch_analysis(fhs_ctx* ctx, const fhs_sara* S, int k, const AnArgs& A, unsigned grid, int ty, int tx) {
+  // Waves of a workgroup: all channels, or equal shares of more than AN_CHANNELS,
+  // whose groups share a launch (a chain of launches per 16 channels took 186 us for
+  // the analysis of 128 x 128 x 64, 70 so, and 137 -> 106 at 512 x 512 x 17).
+  const unsigned groups = cdiv(A.L, AN_CHANNELS), waves = cdiv(A.L, groups);
   // LDS: the turning tiles, or every channel's coefficients and the factors
   const bool last = k == S->g.nlevel;
   const size_t nq = (last ? 4 : 3) * AT_X * 64;
-  const size_t lds = std::max<size_t>(A.L * AT_LH, MODE >= AN_L21 ? (A.L + 1) * nq : 0) * sizeof(float);
+  const size_t lds = std::max<size_t>(waves * AT_LH, MODE >= AN_L21 ? (waves + 1) * nq : 0) * sizeof(float);
   auto go = [&](auto kern) {
     allow_dynamic_lds((const void*)kern, lds);
-    kern<<<grid, 64 * A.L, lds, ctx->stream>>>(S->level[k], A, ty, tx);
+    kern<<<dim3(grid, groups), 64 * waves, lds, ctx->stream>>>(S->level[k], A, ty, tx);
     check_launch();
   };
   last ? go(k_analysis<MODE, true>) : go(k_analysis<MODE, false>);
 }
 
-// All levels and the Dirac block in one mode; at most AN_CHANNELS channels for
-// the modes over the channels.  Returns the number of workgroup sums (AN_NORM).
+// All levels and the Dirac block in one mode; at most AN_CHANNELS channels for the
+// modes over the channels.  Returns the number of workgroup sums (AN_NORM).
 template <int MODE>
 unsigned sara_analyse(fhs_ctx* ctx, const fhs_sara* S, const float* x, int L, float* v1, const float* w, double beta,
                       float* wout, double* part) {
@@ -722,31 +731,29 @@ unsigned sara_analyse(fhs_ctx* ctx, const fhs_sara* S, const float* x, int L, fl
   float* scr = (float*)ctx->ws.get("sara_scratch", std::max<int64_t>(1, G.scr_per_chan * L) * sizeof(float));
   const int64_t N = (int64_t)G.Ny * G.Nx;
   unsigned nsum = 0;
-  for (int l0 = 0; l0 < L; l0 += AN_CHANNELS) {
-    AnArgs A;
-    A.L = std::min(AN_CHANNELS, L - l0);
-    A.x = x + (int64_t)l0 * N;
-    A.scr = scr + (int64_t)l0 * G.scr_per_chan;
-    A.v1 = v1 ? v1 + (int64_t)l0 * G.s : nullptr;
-    A.w = w;
-    A.beta = beta;
-    A.wout = wout;
-    for (int k = 1; k <= G.nlevel && G.nb > 0; ++k) {
-      int ty, tx;
-      const unsigned grid = analysis_grid(G, k, ty, tx);
-      A.part = part ? part + nsum : nullptr;
-      launch_analysis<MODE>(ctx, S, k, A, grid, ty, tx);
-      nsum += grid;
-    }
-    if (G.dirac) {
-      const bool vec = N % 4 == 0 && (uintptr_t)A.x % 16 == 0 &&
-                       (MODE > AN_L21 || (G.s % 4 == 0 && G.boff[G.nb] % 4 == 0 && (uintptr_t)A.v1 % 16 == 0));
-      const unsigned grid = std::min<unsigned>(2048, cdiv(vec ? N / 4 : N, 256));
-      (vec ? k_dirac<MODE, 4> : k_dirac<MODE, 1>)<<<grid, 256, 0, ctx->stream>>>(G, A.x, A.v1, A.L, w, beta, wout,
-                                                                                 part ? part + nsum : nullptr);
-      check_launch();
-      nsum += grid;
-    }
+  AnArgs A;
+  A.L = L;
+  A.x = x;
+  A.scr = scr;
+  A.v1 = v1;
+  A.w = w;
+  A.beta = beta;
+  A.wout = wout;
+  for (int k = 1; k <= G.nlevel && G.nb > 0; ++k) {
+    int ty, tx;
+    const unsigned grid = analysis_grid(G, k, ty, tx);
+    A.part = part ? part + nsum : nullptr;
+    launch_analysis<MODE>(ctx, S, k, A, grid, ty, tx);
+    nsum += grid;
+  }
+  if (G.dirac) {
+    const bool vec = N % 4 == 0 && (uintptr_t)x % 16 == 0 &&
+                     (MODE > AN_L21 || (G.s % 4 == 0 && G.boff[G.nb] % 4 == 0 && (uintptr_t)v1 % 16 == 0));
+    const unsigned grid = std::min<unsigned>(2048, cdiv(vec ? N / 4 : N, 256));
+    (vec ? k_dirac<MODE, 4> : k_dirac<MODE, 1>)<<<dim3(grid, cdiv(L, AN_CHANNELS)), 256, 0, ctx->stream>>>(
+        G, x, v1, L, w, beta, wout, part ? part + nsum : nullptr);
+    check_launch();
+    nsum += grid;
   }
   return nsum;
 }

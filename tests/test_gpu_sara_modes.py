@@ -17,7 +17,7 @@ def rel(a, b):
 
 
 @pytest.mark.parametrize('Ny,Nx,L,nlevel', [(5, 3, 1, 2), (112, 8, 2, 1), (113, 9, 5, 4), (30, 250, 4, 4),
-                                            (98, 64, 16, 4), (40, 33, 17, 3)])
+                                            (98, 64, 16, 4), (40, 33, 17, 3), (24, 20, 35, 2)])
 def test_modes(ctx, Ny, Nx, L, nlevel):
     import fhs
     rng = np.random.default_rng(Ny + Nx + L)
@@ -103,3 +103,32 @@ def test_captured_step_outlives_its_dictionary(L):
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
         again = step(S, v0.clone())                        # eager work between the replays
         assert torch.equal(again[0], want[0]) and torch.equal(again[1], want[1])
+
+
+def _captured_nodes(ctx, f):
+    """Nodes of the graph that a call captures."""
+    import ctypes as C
+    import fhs
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        ctx.bind_stream()
+        f()
+    ctx.bind_stream()
+    n = C.c_size_t()
+    assert fhs.lib().hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None, C.byref(n)) == 0
+    return n.value
+
+
+def test_many_channels_take_no_more_launches():
+    """The channels beyond a workgroup's 16 run in the same launches, not in a chain
+    of launches of their own."""
+    import fhs
+    ctx = fhs.Context(0)
+    S = fhs.SaraDictionary(ctx, 32, 24, nlevel=3)
+    nodes = []
+    for L in (16, 17, 64):
+        x, c = torch.rand((L, 24, 32), device='cuda'), torch.empty((L, S.s), device='cuda')
+        S.psit(x, out=c)                       # sizes the context's workspace
+        torch.cuda.synchronize()
+        nodes.append(_captured_nodes(ctx, lambda: S.psit(x, out=c)))
+    assert nodes == [4, 4, 4], nodes           # three levels and the Dirac block
