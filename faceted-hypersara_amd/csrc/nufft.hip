@@ -9,7 +9,8 @@
 //                 and 1/2, zero pad to Kty, FFT of a + i b -> Z (Kty x Nx / 2);
 //             (2) x-pass: one workgroup per B consecutive grid rows: the columns'
 //                 rows from Z[ky] and Z[-ky], FFT of length Ktx -> Fx.
-//   adjoint : (1') x-pass: the real part of the image comes from the Hermitian
+//   adjoint (adj_half; a small launch transforms all rows and single columns):
+//             (1') x-pass: the real part of the image comes from the Hermitian
 //                 part g[ky][kx] + conj g[-ky][-kx]; inverse FFT of its rows
 //                 ky <= Kty / 2, first Nx outputs -> U (half of Kty, x Nx);
 //             (2') y-pass of U[a] + i U[b]: real and imaginary part are the two
@@ -409,44 +410,81 @@ __global__ __launch_bounds__((nt_strided<N, B>())) void k_fwd_x(const float2* __
   }
 }
 
+// The first row of an adjoint x-pass workgroup, its thread's row and where the outputs
+// go: HALF as above, or one of all Kty rows of a launch too small to gain from half of
+// them (adj_half).
+template <int B, bool HALF>
+__device__ __forceinline__ int adj_row0() { return HALF ? xpass_eighth_row0(B) : xpass_row0<B>(); }
+
+template <bool HALF>
+__device__ __forceinline__ HalfRow adj_row(int k, int Kty) {
+  HalfRow row(HALF ? k : 0, Kty);
+  if (!HALF) {
+    row.valid = k < Kty;
+    row.ky = row.valid ? k : 0;
+  }
+  return row;
+}
+
+template <bool HALF>
+__host__ __device__ inline int adj_stride(int Kty) { return HALF ? half_stride(Kty) : Kty; }
+
+template <bool HALF>
+__device__ __forceinline__ void adj_put(float2* __restrict__ col, const HalfRow& row, float2 u) {
+  if (HALF)
+    adj_store(col, row, u);
+  else
+    col[row.ky] = u;
+}
+
+// inputs of an adjoint x-pass thread: its values at columns STEP (PER of them, NT / B
+// apart) + odd, every load issued before the first is used
+template <int N, int B, int NT, int PER, int STEP, bool HALF>
+__device__ __forceinline__ void adj_load(const float2* __restrict__ gl, int Kty, const HalfRow& row, int odd, float2* v) {
+  float2 m[HALF ? PER : 1];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int k = STEP * ((threadIdx.x + j * NT) / B) + odd;
+    v[j] = gl[(size_t)k * Kty + row.ky];
+    if constexpr (HALF) m[j] = gl[(size_t)((N - k) % N) * Kty + row.mirror];
+  }
+  if constexpr (HALF) {
+#pragma unroll
+    for (int j = 0; j < PER; ++j) v[j] = hermitian(v[j], m[j]);
+    if (row.shared)
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        const int k = STEP * ((threadIdx.x + j * NT) / B) + odd;
+        const float2 h = hermitian(gl[(size_t)k * Kty + row.second], gl[(size_t)((N - k) % N) * Kty + row.second]);
+        v[j] = make_float2(v[j].x - h.y, v[j].y + h.x);
+      }
+  }
+}
+
 // (1') adjoint x-pass: N = Ktx, keep the first Nx outputs
-template <int N, int B>
-__global__ __launch_bounds__((nt_strided<N, B>())) void k_adj_x(const float2* __restrict__ g, int Kty,
+// (64 registers of a half's 8 values and their mirrors, for two workgroups of 1024 threads on a CU)
+template <int N, int B, bool HALF>
+__global__ __launch_bounds__((nt_strided<N, B>()), N * B <= 8192 ? 8 : 4) void k_adj_x(const float2* __restrict__ g, int Kty,
                                                           int Nx, const float2* __restrict__ tw,
                                                           float2* __restrict__ U) {
   constexpr int NT = nt_strided<N, B>();
   __shared__ float2 s[N * B];
   __shared__ float2 tws[TW_LDS<N>];
-  const int b = threadIdx.x % B, l = blockIdx.y, ky0 = xpass_eighth_row0(B);
-  if (ky0 >= half_rows(Kty)) return;
-  const HalfRow row(ky0 + b, Kty);
+  const int l = blockIdx.y, ky0 = adj_row0<B, HALF>();
+  if (HALF && ky0 >= half_rows(Kty)) return;
+  const HalfRow row = adj_row<HALF>(ky0 + threadIdx.x % B, Kty);
   const float2* twp = stage_twiddles<N, NT, TW_LDS<N>>(tw, tws);
-  const float2* gl = g + (size_t)l * N * Kty;
-  constexpr int PER = N * B / NT;   // every load issued before the first LDS store
-  float2 v[PER], m[PER];
-#pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    const int k = (threadIdx.x + j * NT) / B;
-    v[j] = gl[(size_t)k * Kty + row.ky];
-    m[j] = gl[(size_t)((N - k) % N) * Kty + row.mirror];
-  }
-#pragma unroll
-  for (int j = 0; j < PER; ++j) v[j] = hermitian(v[j], m[j]);
-  if (row.shared)
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int k = (threadIdx.x + j * NT) / B;
-      const float2 h = hermitian(gl[(size_t)k * Kty + row.second], gl[(size_t)((N - k) % N) * Kty + row.second]);
-      v[j] = make_float2(v[j].x - h.y, v[j].y + h.x);
-    }
+  constexpr int PER = N * B / NT;
+  float2 v[PER];
+  adj_load<N, B, NT, PER, 1, HALF>(g + (size_t)l * N * Kty, Kty, row, 0, v);
 #pragma unroll
   for (int j = 0; j < PER; ++j) s[threadIdx.x + j * NT] = v[j];
   __syncthreads();
   fft_lds<N, B, NT, true>(s, twp);
-  const int hs = half_stride(Kty);
+  const int hs = adj_stride<HALF>(Kty);
   float2* Ul = U + (size_t)l * Nx * hs;
   if (row.valid)
-    for (int t = threadIdx.x; t < Nx * B; t += NT) adj_store(Ul + (size_t)(t / B) * hs, row, s[t]);
+    for (int t = threadIdx.x; t < Nx * B; t += NT) adj_put<HALF>(Ul + (size_t)(t / B) * hs, row, s[t]);
 }
 
 // Split x-passes for N >= X_SPLIT_MIN when the image holds at most half the
@@ -524,8 +562,8 @@ __global__ __launch_bounds__((nt_strided<N, B>()), B == 8 ? 4 : 8) void k_fwd_x_
     }
 }
 
-template <int N, int B>
-__global__ __launch_bounds__((nt_strided<N, B>()), B == 8 ? 4 : 8) void k_adj_x_split(const float2* __restrict__ g, int Kty,
+template <int N, int B, bool HALF>
+__global__ __launch_bounds__((nt_strided<N, B>()), B == 8 || !HALF ? 4 : 8) void k_adj_x_split(const float2* __restrict__ g, int Kty,
                                                                 int Nx, const float2* __restrict__ tw,
                                                                 float2* __restrict__ U) {
   constexpr int H = N / 2;
@@ -533,37 +571,20 @@ __global__ __launch_bounds__((nt_strided<N, B>()), B == 8 ? 4 : 8) void k_adj_x_
   static_assert(H * B % NT == 0 && NT % B == 0, "split x-pass: whole rows per thread");
   __shared__ float2 s[H * B];
   __shared__ float2 tws[3 * H / 4];
-  const int b = threadIdx.x % B, l = blockIdx.y, ky0 = xpass_eighth_row0(B);
-  if (ky0 >= half_rows(Kty)) return;
-  const HalfRow row(ky0 + b, Kty);
+  const int l = blockIdx.y, ky0 = adj_row0<B, HALF>();
+  if (HALF && ky0 >= half_rows(Kty)) return;
+  const HalfRow row = adj_row<HALF>(ky0 + threadIdx.x % B, Kty);
   for (int i = threadIdx.x; i < 3 * H / 4; i += NT) tws[i] = tw[2 * i];
   const float2* gl = g + (size_t)l * N * Kty;
   constexpr int PER = H * B / NT;
   float2 v[PER], e[PER];
-  auto load = [&](int odd) {
-    float2 m[PER];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const int k = 2 * ((threadIdx.x + j * NT) / B) + odd;
-      v[j] = gl[(size_t)k * Kty + row.ky];
-      m[j] = gl[(size_t)((N - k) % N) * Kty + row.mirror];
-    }
-#pragma unroll
-    for (int j = 0; j < PER; ++j) v[j] = hermitian(v[j], m[j]);
-    if (row.shared)
-#pragma unroll
-      for (int j = 0; j < PER; ++j) {
-        const int k = 2 * ((threadIdx.x + j * NT) / B) + odd;
-        const float2 h = hermitian(gl[(size_t)k * Kty + row.second], gl[(size_t)((N - k) % N) * Kty + row.second]);
-        v[j] = make_float2(v[j].x - h.y, v[j].y + h.x);
-      }
-  };
-  load(0);
+  adj_load<N, B, NT, PER, 2, HALF>(gl, Kty, row, 0, v);
 #pragma unroll
   for (int j = 0; j < PER; ++j) s[threadIdx.x + j * NT] = v[j];
+  if (!HALF) adj_load<N, B, NT, PER, 2, HALF>(gl, Kty, row, 1, v);
   __syncthreads();
   fft_lds<H, B, NT, true>(s, tws);
-  load(1);
+  if (HALF) adj_load<N, B, NT, PER, 2, HALF>(gl, Kty, row, 1, v);
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int t = threadIdx.x + j * NT;
@@ -572,7 +593,7 @@ __global__ __launch_bounds__((nt_strided<N, B>()), B == 8 ? 4 : 8) void k_adj_x_
   }
   __syncthreads();
   fft_lds<H, B, NT, true>(s, tws);
-  const int hs = half_stride(Kty);
+  const int hs = adj_stride<HALF>(Kty);
   float2* Ul = U + (size_t)l * Nx * hs;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
@@ -580,7 +601,7 @@ __global__ __launch_bounds__((nt_strided<N, B>()), B == 8 ? 4 : 8) void k_adj_x_
     if (n < Nx && row.valid) {
       float2 w = tw[n];
       w.y = -w.y;
-      adj_store(Ul + (size_t)n * hs, row, cadd(e[j], cmul(s[t], w)));
+      adj_put<HALF>(Ul + (size_t)n * hs, row, cadd(e[j], cmul(s[t], w)));
     }
   }
 }
@@ -593,8 +614,9 @@ __device__ __forceinline__ float2 join_pair(const float2* __restrict__ ua, const
   return mirror ? make_float2(a.x + c.y, c.x - a.y) : make_float2(a.x - c.y, a.y + c.x);
 }
 
-// (2') adjoint y-pass: N = Kty, two columns, keep Ny outputs, scale
-template <int N>
+// (2') adjoint y-pass: N = Kty, two columns (HALF; else one, whole), keep Ny outputs,
+// scale
+template <int N, bool HALF>
 __global__ __launch_bounds__(nt_y<N>()) void k_adj_y(const float2* __restrict__ U,
                                                               const float* __restrict__ sy,
                                                               const float* __restrict__ sx, int Ny, int Nx,
@@ -603,13 +625,13 @@ __global__ __launch_bounds__(nt_y<N>()) void k_adj_y(const float2* __restrict__ 
                                                               float* __restrict__ out) {
   constexpr int NT = fft_threads<N, 1>();
   __shared__ float2 s[fft_lds_slots<N, 1>()];
-  const int ix = 2 * blockIdx.x, l = blockIdx.y, hs = half_stride(N);
-  const bool two = ix + 1 < Nx;
+  const int ix = (HALF ? 2 : 1) * blockIdx.x, l = blockIdx.y, hs = HALF ? half_stride(N) : N;
+  const bool two = HALF && ix + 1 < Nx;
   const float2* __restrict__ ua = U + ((size_t)l * Nx + ix) * hs;
   const float2* __restrict__ ub = two ? ua + hs : nullptr;
-  const float sc = 0.5f * (scale ? scale[l] : 1.f), sa = sc * sx[ix], sb = two ? sc * sx[ix + 1] : 0.f;
+  const float sc = (HALF ? 0.5f : 1.f) * (scale ? scale[l] : 1.f), sa = sc * sx[ix], sb = two ? sc * sx[ix + 1] : 0.f;
   float* __restrict__ o = out + ((size_t)l * Nx + ix) * Ny;
-  auto load = [&](int, int, int, int n) { return join_pair(ua, ub, N, n); };
+  auto load = [&](int, int, int, int n) { return HALF ? join_pair(ua, ub, N, n) : ua[n]; };
   auto store = [&](int, int, int, int n, float2 v) {
     if (n < Ny) {
       o[n] = sa * sy[n] * v.x;
@@ -640,19 +662,49 @@ struct RunFwdY {
     k_fwd_y<N><<<dim3((Nx + 1) / 2, L), nt_y<N>(), 0, st>>>(x, p->sy, p->sx, p->Ny, p->Nx, p->twy, T);
   }
 };
-// Rows per x-pass workgroup: the default first, then the autotuner's other
-// candidates (those whose rows fit in LDS).
+// Rows per x-pass workgroup: the default of a launch that fills the chip first, then
+// the other candidates (those whose rows fit in LDS).
 template <int N, bool SPLIT>
 struct XRows {
-  static constexpr int n = N >= 4096 ? (SPLIT ? 3 : 2) : N == 2048 ? 3 : N == 1024 ? 3 : N == 512 ? 2 : 1;
+  static constexpr int n = N >= 4096 ? (SPLIT ? 3 : 2) : N >= 256 ? 3 : 1;
   static constexpr int at(int i) {
     if (N >= 4096) return i == 0 ? 4 : i == 1 ? 2 : 8;
     if (N == 2048) return i == 0 ? 4 : i == 1 ? 2 : 8;
     if (N == 1024) return i == 0 ? 8 : i == 1 ? 4 : 16;
-    if (N == 512) return i == 0 ? 16 : 8;
+    if (N >= 256) return i == 0 ? 16 : i == 1 ? 8 : 4;
     return 16;
   }
 };
+constexpr int X_FULL = 256;   // workgroups that occupy every CU
+// The rows of a launch without tuning: fewer than the default while CUs would stay
+// idle (forward x-pass of one image, default rows -> these, us: 256 x 256 8.7 -> 5.2,
+// 512 x 512 12.2 -> 8.8, 128 x 1024 12.2 -> 9.8).
+template <int N, bool SPLIT>
+int x_rows(int rows, int L) {
+  using R = XRows<N, SPLIT>;
+  int best = 0;
+  for (int i = 1; i < R::n && (int64_t)cdiv(rows, R::at(best)) * L < X_FULL; ++i)
+    if (R::at(i) < R::at(best)) best = i;
+  return best;
+}
+
+inline bool is_pow2_grid(int n) { return n >= 16 && n <= 4096 && (n & (n - 1)) == 0; }
+
+// Half of the rows and two columns a transform in the adjoint, where that is the
+// faster form.  A launch that does not fill the chip is a chain of latencies, which
+// mirrored rows and a second column lengthen.  And the mirrored rows are not aligned,
+// so that every XCD's eighth of the rows costs a line more in each grid column,
+// which the saved y-pass makes up for on tall grids, on wide ones only if tall enough
+// and many.  All rows against half, us: 256 x 256 images 9.4, 15.6 (16 of them 23.7,
+// 22.3), 512 x 512 13.7, 17.1 (4: 25.4, 25.0; 16: 67, 58), 1024 x 1024 x 4 84, 70;
+// wide ones, 512 x 1024 x 4 45, 48 (16: 168, 142), 512 x 2048 x 4 85, 99 (16: 342,
+// 326), 1024 x 2048 x 4 190, 159, 64 x 2048 x 16 62, 81.
+inline bool adj_half(const fhs_nufft* p, int L) {
+  if (!is_pow2_grid(p->Kty) || !is_pow2_grid(p->Ktx)) return true;
+  const int B = p->Ktx >= 2048 ? 4 : p->Ktx >= 1024 ? 8 : 16;
+  const int64_t groups = (int64_t)cdiv(half_rows(p->Kty), B) * L;
+  return p->Kty >= p->Ktx ? groups >= X_FULL : groups >= 4 * X_FULL && p->Kty >= 1024;
+}
 
 template <int N, bool SPLIT, class F>
 void with_rows(int i, F&& f) {
@@ -684,7 +736,7 @@ struct RunFwdX {
     const bool split = N >= X_SPLIT_MIN && 2 * p->Nx <= N;
     auto go = [&](auto split_c) {
       constexpr bool SP = decltype(split_c)::value;
-      tune_launch(ctx, xpass_key("fft_fwd_x", N, Kty, p->Nx, L), XRows<N, SP>::n, 0, xrow_labels<N, SP>(),
+      tune_launch(ctx, xpass_key("fft_fwd_x", N, Kty, p->Nx, L), XRows<N, SP>::n, x_rows<N, SP>(Kty, L), xrow_labels<N, SP>(),
                   [&](int c) {
                     with_rows<N, SP>(c, [&](auto b_c) {
                       constexpr int B = decltype(b_c)::value;
@@ -711,36 +763,40 @@ template <int N>
 struct RunAdjX {
   static void run(fhs_ctx* ctx, int Kty, int L, const float2* g, const fhs_nufft* p, float2* T) {
     const bool split = N >= X_SPLIT_MIN && 2 * p->Nx <= N;
-    auto go = [&](auto split_c) {
-      constexpr bool SP = decltype(split_c)::value;
-      tune_launch(ctx, xpass_key("fft_adj_x", N, Kty, p->Nx, L), XRows<N, SP>::n, 0, xrow_labels<N, SP>(),
+    auto go = [&](auto split_c, auto half_c) {
+      constexpr bool SP = decltype(split_c)::value, HALF = decltype(half_c)::value;
+      const int rows = HALF ? half_rows(Kty) : Kty;
+      tune_launch(ctx, xpass_key("fft_adj_x", N, Kty, p->Nx, L), XRows<N, SP>::n, x_rows<N, SP>(rows, L), xrow_labels<N, SP>(),
                   [&](int c) {
                     with_rows<N, SP>(c, [&](auto b_c) {
                       constexpr int B = decltype(b_c)::value;
+                      const dim3 grid(HALF ? xpass_eighth_grid(rows, B) : cdiv(rows, B), L);
                       if constexpr (SP)
-                        k_adj_x_split<N, B><<<dim3(xpass_eighth_grid(half_rows(Kty), B), L), nt_strided<N, B>(), 0, ctx->stream>>>(g, Kty, p->Nx,
-                                                                                                    p->twx, T);
+                        k_adj_x_split<N, B, HALF><<<grid, nt_strided<N, B>(), 0, ctx->stream>>>(g, Kty, p->Nx, p->twx, T);
                       else
-                        k_adj_x<N, B><<<dim3(xpass_eighth_grid(half_rows(Kty), B), L), nt_strided<N, B>(), 0, ctx->stream>>>(g, Kty, p->Nx,
-                                                                                              p->twx, T);
+                        k_adj_x<N, B, HALF><<<grid, nt_strided<N, B>(), 0, ctx->stream>>>(g, Kty, p->Nx, p->twx, T);
                       check_launch();
                     });
                   });
     };
+    auto form = [&](auto split_c) { adj_half(p, L) ? go(split_c, std::true_type{}) : go(split_c, std::false_type{}); };
     if constexpr (N >= X_SPLIT_MIN) {
       if (split) {
-        go(std::true_type{});
+        form(std::true_type{});
         return;
       }
     }
-    go(std::false_type{});
+    form(std::false_type{});
   }
 };
 template <int N>
 struct RunAdjY {
   static void run(hipStream_t st, int Nx, int L, const float2* T, const fhs_nufft* p,
                   const float* scale, float* out) {
-    k_adj_y<N><<<dim3((Nx + 1) / 2, L), nt_y<N>(), 0, st>>>(T, p->sy, p->sx, p->Ny, p->Nx, p->twy, scale, out);
+    if (adj_half(p, L))
+      k_adj_y<N, true><<<dim3((Nx + 1) / 2, L), nt_y<N>(), 0, st>>>(T, p->sy, p->sx, p->Ny, p->Nx, p->twy, scale, out);
+    else
+      k_adj_y<N, false><<<dim3(Nx, L), nt_y<N>(), 0, st>>>(T, p->sy, p->sx, p->Ny, p->Nx, p->twy, scale, out);
   }
 };
 
@@ -994,8 +1050,6 @@ __global__ __launch_bounds__(1024) void k_adj_x_rt(const float2* __restrict__ g,
   fft_rt<PT, true>(s_rt, tw, N, B, blockDim.x, load, store);
 }
 
-inline bool is_pow2_grid(int n) { return n >= 16 && n <= 4096 && (n & (n - 1)) == 0; }
-
 void fwd_y_any(fhs_ctx* ctx, const fhs_nufft* p, int L, const float* x, float2* T) {
   if (is_pow2_grid(p->Kty)) {
     dispatch_pow2<RunFwdY>(p->Kty, ctx->stream, p->Nx, L, x, p, T);
@@ -1054,9 +1108,10 @@ void adj_x_any(fhs_ctx* ctx, const fhs_nufft* p, int L, const float2* g, float2*
   });
 }
 
-// Z of the forward, U of the adjoint transform
+// Z of the forward, U of the adjoint transform, in either of its forms
 float2* nufft_workspace(fhs_ctx* ctx, const fhs_nufft* p, int L) {
-  const size_t z = (size_t)((p->Nx + 1) / 2) * p->Kty, u = (size_t)p->Nx * half_stride(p->Kty);
+  const size_t z = (size_t)((p->Nx + 1) / 2) * p->Kty;
+  const size_t u = (size_t)p->Nx * (adj_half(p, L) ? half_stride(p->Kty) : p->Kty);
   return (float2*)ctx->ws.get("nufft_T", L * std::max(z, u) * sizeof(float2));
 }
 

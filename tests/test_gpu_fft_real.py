@@ -31,3 +31,28 @@ def test_scaled_fft(Ny, Nx, Kty, Ktx):
     ref = np.fft.ifft2(g.reshape(L, Ktx, Kty).astype(np.complex128), norm='forward').real[:, :Nx, :Ny] * sn
     ref *= np.array(scale)[:, None, None]
     assert np.linalg.norm(out - ref) < 2e-6 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize('Ny,Nx,Kty,Ktx,L', [
+    (1, 1, 16, 16, 256), (33, 31, 64, 64, 128), (100, 37, 256, 512, 32), (100, 37, 256, 512, 31), (77, 128, 256, 256, 33),
+    (512, 513, 1024, 1024, 4), (512, 513, 1024, 1024, 1), (9, 700, 32, 2048, 64), (6, 2047, 16, 4096, 1),
+    (6, 2047, 1024, 4096, 8), (6, 3001, 1024, 4096, 8), (300, 700, 1024, 2048, 16)])
+def test_adjoint_on_both_sides_of_its_rule(Ny, Nx, Kty, Ktx, L):
+    """Launches that fill the chip transform half of the rows, smaller ones all of them
+    with fewer rows a workgroup: both against FP64, with the bound of test_scaled_fft."""
+    import torch
+    import fhs
+    rng = np.random.default_rng(Ny + Nx + L)
+    ctx = fhs.default_context(0)
+    sy, sx = rng.uniform(0.5, 2, Ny).astype(np.float32), rng.uniform(0.5, 2, Nx).astype(np.float32)
+    plan = fhs.NufftPlan(ctx, Ny, Nx, Kty, Ktx, sy.astype(np.float64), sx.astype(np.float64))
+    sn = torch.from_numpy(sx[:, None].astype(np.float64) * sy).cuda()
+    x = torch.from_numpy(rng.normal(size=(L, Nx, Ny)).astype(np.float32)).cuda()
+    ref = torch.fft.fft2(x.double() * sn, s=(Ktx, Kty))
+    F = plan.A(x).reshape(L, Ktx, Kty)
+    assert torch.linalg.vector_norm(F - ref) < 2e-6 * torch.linalg.vector_norm(ref)
+    del F, ref
+    g = torch.view_as_complex(torch.from_numpy(rng.normal(size=(L, Ktx * Kty, 2)).astype(np.float32)).cuda())
+    out = plan.At_real(g).reshape(L, Nx, Ny)
+    ref = torch.fft.ifft2(g.reshape(L, Ktx, Kty).to(torch.complex128), norm='forward').real[:, :Nx, :Ny] * sn
+    assert torch.linalg.vector_norm(out - ref) < 2e-6 * torch.linalg.vector_norm(ref)
