@@ -875,10 +875,16 @@ __device__ __forceinline__ void fft_stage_rt(float2* s, const float2* __restrict
   constexpr int PMAX = (PT + R - 1) / R;   // butterflies per thread (NT >= B N / PT)
   const int NBF = B * N / R;
   const int TS = N / (NS * R);
+  // The thread's index is opaque to the compiler in each half of a stage: the addresses of
+  // the first loads and last stores of all six radices do not change from stage to
+  // stage, and were kept in registers, 1040 to 2180 bytes of them spilled in every lane
+  // (now none, in 58 registers).
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
   float2 v[PMAX][R];
 #pragma unroll
   for (int q = 0; q < PMAX; ++q) {
-    const int u = threadIdx.x + q * NT;
+    const int u = tid + q * NT;
     if (u < NBF) {
       const int b = u % B, j = u / B;
       const int k = j % NS;
@@ -899,9 +905,10 @@ __device__ __forceinline__ void fft_stage_rt(float2* s, const float2* __restrict
     }
   }
   if (!first && !last) __syncthreads();
+  asm volatile("" : "+v"(tid));
 #pragma unroll
   for (int q = 0; q < PMAX; ++q) {
-    const int u = threadIdx.x + q * NT;
+    const int u = tid + q * NT;
     if (u < NBF) {
       const int b = u % B, j = u / B;
       const int k = j % NS;
@@ -941,8 +948,8 @@ __device__ __forceinline__ void fft_rt(float2* s, const float2* __restrict__ tw,
 
 // Values per thread of a runtime-length workgroup of B transforms, its threads and LDS
 // bytes.  As few values as 1024 threads allow: the stages are a chain of
-// latencies, which more threads shorten (one 1000 x 1440 grid: y-passes 36 -> 24 and 36 ->
-// 20 us, x-passes 50 -> 36, with the column pairs and mirrored rows).
+// latencies, which more threads shorten (one 1000 x 1440 grid, 16 values -> 4, us:
+// x-passes 26 -> 21 and 25 -> 20; 128 pairs of 2000-point columns 16 -> 12 and 19 -> 12).
 inline int fft_rt_values(int N, int B) { return B * N <= 4096 ? 4 : B * N <= 8192 ? 8 : 16; }
 inline int fft_rt_threads(int N, int B) {
   const int t = (int)cdiv(B * N, fft_rt_values(N, B));
