@@ -45,7 +45,11 @@ class AxisInterp:
         self.s = C @ self.alpha
         d = np.subtract.outer(np.arange(J), np.arange(J))
         gram = np.cos(self.gamma * d[..., None] * n) @ (self.s ** 2)
-        self.T = np.linalg.inv(gram)
+        if N >= J:
+            self.T = np.linalg.inv(gram)
+        else:                       # more taps than pixels: the Gram has rank N only
+            val, vec = np.linalg.eigh(gram)
+            self.T = vec[:, -N:] / val[-N:] @ vec[:, -N:].T
 
     def _dirichlet(self, t):
         half = np.sin(0.5 * t)

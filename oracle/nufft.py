@@ -83,10 +83,12 @@ def minmax_gram_inverse(N, J, K, alpha):
     n = np.arange(N) - n0
     d = np.arange(J)[:, None] - np.arange(J)[None, :]
     gram = np.einsum('n,jkn->jk', s ** 2, np.cos(gam * d[:, :, None] * n[None, None, :]))
-    try:
+    if N >= J:
         return np.linalg.inv(gram)
-    except np.linalg.LinAlgError:      # N < J: rank N; whether LU meets an exact zero depends on the host's LAPACK
-        return np.linalg.pinv(gram)
+    # more taps than pixels: rank N, the inverse on its range
+    lam, V = np.linalg.eigh(gram)
+    V = V[:, -N:]
+    return (V / lam[-N:]) @ V.T
 
 
 def minmax_coef_1d(om, N, J, K, alpha, nc):

@@ -442,3 +442,23 @@ def test_faceted_sara_is_the_global_transform(Ny, Nx, ys, xs):
     x2[:max(f['ey0'], 0), :] = 5.0
     x2[:, :max(f['ex0'], 0)] = 5.0
     assert np.allclose(F.glob.psit(x2)[f['global']], g[f['global']], rtol=0, atol=1e-13)
+
+
+@pytest.mark.parametrize('N,K,J', [(1, 16, 7), (2, 16, 7), (3, 16, 7), (4, 16, 7), (5, 16, 7), (6, 16, 7), (6, 20, 8),
+                                   (7, 16, 7), (12, 24, 7)])
+def test_axis_shorter_than_its_taps(N, K, J):
+    """More taps than pixels leave the min-max Gram with rank N on every host: the oracle's
+    and the package's coefficients agree and reproduce each pixel's exponential (exactly,
+    the N equations having J >= N unknowns; to the min-max error beyond)."""
+    from fhs.nufft import AxisInterp
+    om = np.random.default_rng(N + J).uniform(-np.pi, np.pi, 40)
+    alpha = onu.fit_scaling(N, J, K)
+    idx, coef = onu.minmax_coef_1d(om, N, J, K, alpha, N // 2)
+    first, own = AxisInterp(N, K, J).coefficients(om)
+    assert np.array_equal(idx[:, 0], first)
+    X = np.fft.fft(np.diag(onu.scaling_factors(N, K, alpha)), K)         # one pixel a row
+    want = np.exp(-1j * np.outer(om, np.arange(N) - N // 2))
+    for c in (coef, own):
+        got = np.einsum('mj,nmj->mn', c, X[:, idx])
+        assert np.abs(got - want).max() < (1e-6 if N <= J else 1e-2)
+    assert np.abs(coef - own).max() <= 1e-6 * np.abs(coef).max()
