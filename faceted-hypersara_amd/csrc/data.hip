@@ -72,7 +72,11 @@ constexpr int NXCD = 8;   // MI355X: 8 XCDs, each with its own L2
 // an odd L on all eight.  (One XCD per channel whatever L left 7 of 8 idle at
 // L = 1 and half of them at L = 4: the data step of 4 channels took 2.41 ms at
 // 2048 x 2048 with 500k w-projected rows each, 1.00 ms in the DR form of
-// 256 x 256 images, against 1.86 and 0.60 ms with this map.)
+// 256 x 256 images, against 1.86 and 0.60 ms with this map.  Counts that left few
+// slots idle gain too, although their channels meet in more L2s, since a launch
+// lasted as long as the XCD with the most channels: data step of 200k rows on
+// 512 x 512 images, one XCD per channel -> this map, us: 5 channels 362 -> 315, 6
+// 378 -> 345, 7 391 -> 376, 10 552 -> 459, 13 595 -> 533, 14 595 -> 554, 15 612 -> 582.)
 // Units are interleaved over an XCD's channels (unit-major), so the first
 // units of every channel (the heaviest adjoint tiles) start first.
 __host__ __device__ __forceinline__ int xcd_groups(int L) { return L & 1 ? 1 : L & 2 ? 2 : L & 4 ? 4 : NXCD; }

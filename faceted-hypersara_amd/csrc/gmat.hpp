@@ -309,9 +309,6 @@ constexpr int FWD_ITEM = 1024;                       // rows per forward work it
 template <int KM>
 constexpr int fwd_win() { return (TILE_Y + KM - 1) * (TILE_X + KM - 1); }   // forward window (complex)
 
-// LDS of an adjoint workgroup that may run the CSC unit path (bytes)
-constexpr size_t ADJ_CSC_LDS_BYTES = ADJ_LDS * sizeof(float2);
-
 inline bool tile_grid_ok(int Kty, int Ktx, int Ky, int Kx) {
   return Kty % TILE_Y == 0 && Ktx % TILE_X == 0 && Kty >= TILE_Y + Ky - 1 && Ktx >= TILE_X + Kx - 1;
 }

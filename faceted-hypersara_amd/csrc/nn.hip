@@ -733,8 +733,10 @@ int fhs_nn_conv3x3(fhs_ctx* ctx, const float* in, int cin, int NB, int H, int W,
   return guard(ctx, [&] {
     FHS_CHECK(in && w && out && cin > 0 && cout > 0 && NB > 0 && H > 0 && W > 0, "nn_conv3x3: bad argument");
     Scope sc(ctx, "nn_conv3x3");
-    // two rows a wave and two groups of 16 output channels, which share the input
-    // tile, where that still leaves two workgroups a CU
+    // Two rows a wave and two groups of 16 output channels, which share the input
+    // tile, where that still leaves two workgroups a CU (32 -> 32 channels, us, one row
+    // and group, two rows, both: 512 such workgroups 35, 33, 26, 256 of them 18, 16.5,
+    // 19, 64 of them 8.7, 12, 18.5; 16 -> 16 channels, rows: 512 13.7, 12.3, 256 8.9, 9.6)
     const bool rows2 = cdiv(W, CV_W) * cdiv(H, 8) * NB * cdiv(cout, 32) >= 512;
     const bool two = cout > 16 && rows2;
     const unsigned tiles = cdiv(W, CV_W) * cdiv(H, rows2 ? 8 : 4) * NB;

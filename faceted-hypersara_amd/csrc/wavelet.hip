@@ -447,8 +447,9 @@ constexpr int ST_WAVES = 4;                       // tiles per workgroup
 constexpr int ST_PER = ST_Y * ST_X / 64;          // pixels per lane
 constexpr int ST_LD = 66;
 // A tile's bases run one after the other; below this many tiles x channels the chip
-// is not full and the four waves of a workgroup share a tile's bases instead (finest
-// level of SARA 256 x 256, 96 tiles: 22 us in 32 x 32 tiles, 9 us split).
+// is not full and the four waves of a workgroup share a tile's bases instead (whole
+// synthesis, tiles' bases in sequence -> split, us: 96 tiles 35 -> 24, 768 36 -> 27, 1280
+// 45 -> 37, 1920 48 -> 43; beyond the line 2560 tiles 51 -> 47, 3840 64 -> 62, 5120 75 -> 76).
 constexpr int64_t SYN_SPLIT_BELOW = 2048;
 
 struct SynIn {
@@ -629,34 +630,28 @@ __global__ __launch_bounds__(64 * ST_WAVES) void k_synthesis(SaraArgs G, int ty,
 }
 
 // ---- more than 16 channels ---------------------------------------------------
-// The same modes from stored coefficients (mode 0: l21 step, 1: sum of the
-// norms, 2: weights), Dirac analysis fused.
-__global__ __launch_bounds__(256) void k_l21(SaraGeom G, float* __restrict__ v1,
-                                             const float* __restrict__ xhat, int L,
+// The modes over the channels from stored coefficients, Dirac block included (mode 0:
+// l21 step, 1: sum of the norms, 2: weights).
+__global__ __launch_bounds__(256) void k_l21(int64_t s, float* __restrict__ v1, int L,
                                              const float* __restrict__ w, double beta, int mode,
                                              float* __restrict__ wout, double* __restrict__ partial) {
   __shared__ double sh[256 / 64];
   double tot[1] = {0.0};
-  const int64_t s = G.s;
-  const int64_t dstart = G.boff[G.nb];
   for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < s;
        c += (int64_t)gridDim.x * blockDim.x) {
-    const bool dir = G.dirac && c >= dstart;
     constexpr int LREG = 16;   // channels kept in registers between the norm and the update
     float rv[LREG];
     double ss = 0.0;
 #pragma unroll
     for (int l = 0; l < LREG; ++l) {
       if (l < L) {
-        float r = v1[(int64_t)l * s + c];
-        if (dir && xhat) r += xhat[(int64_t)l * G.Ny * G.Nx + (c - dstart)] * G.norm;
+        const float r = v1[(int64_t)l * s + c];
         rv[l] = r;
         ss += (double)r * r;
       }
     }
     for (int l = LREG; l < L; ++l) {
-      float r = v1[(int64_t)l * s + c];
-      if (dir && xhat) r += xhat[(int64_t)l * G.Ny * G.Nx + (c - dstart)] * G.norm;
+      const float r = v1[(int64_t)l * s + c];
       ss += (double)r * r;
     }
     const double l2 = sqrt(ss);
@@ -674,8 +669,7 @@ __global__ __launch_bounds__(256) void k_l21(SaraGeom G, float* __restrict__ v1,
     for (int l = 0; l < LREG; ++l)
       if (l < L) v1[(int64_t)l * s + c] = rv[l] - f * rv[l];
     for (int l = LREG; l < L; ++l) {
-      float r = v1[(int64_t)l * s + c];
-      if (dir && xhat) r += xhat[(int64_t)l * G.Ny * G.Nx + (c - dstart)] * G.norm;
+      const float r = v1[(int64_t)l * s + c];
       v1[(int64_t)l * s + c] = r - f * r;
     }
   }
@@ -797,8 +791,7 @@ void sara_dual_step(fhs_ctx* ctx, const fhs_sara* S, float* v1, const float* xha
       sara_analyse<AN_L21>(ctx, S, xhat, L, v1, w, beta, nullptr, nullptr);
     } else {
       sara_analyse<AN_ADD>(ctx, S, xhat, L, v1, nullptr, 0.0, nullptr, nullptr);
-      k_l21<<<std::min<unsigned>(2048, cdiv(G.s, 256)), 256, 0, ctx->stream>>>(G, v1, nullptr, L, w, beta, 0, nullptr,
-                                                                               nullptr);
+      k_l21<<<std::min<unsigned>(2048, cdiv(G.s, 256)), 256, 0, ctx->stream>>>(G.s, v1, L, w, beta, 0, nullptr, nullptr);
       check_launch();
     }
   }
@@ -923,8 +916,8 @@ int fhs_sara_update_weights(fhs_ctx* ctx, const fhs_sara* S, const float* x, int
     }
     float* c = (float*)ctx->ws.get("sara_prior_coefs", (size_t)G.s * L * sizeof(float));
     sara_analyse<AN_SET>(ctx, S, x, L, c, nullptr, 0.0, nullptr, nullptr);
-    k_l21<<<std::min<unsigned>(2048, cdiv(G.s, 256)), 256, 0, ctx->stream>>>(G, c, nullptr, L, nullptr, upsilon, 2,
-                                                                             weights1, nullptr);
+    k_l21<<<std::min<unsigned>(2048, cdiv(G.s, 256)), 256, 0, ctx->stream>>>(G.s, c, L, nullptr, upsilon, 2, weights1,
+                                                                             nullptr);
     check_launch();
   });
 }
@@ -947,7 +940,7 @@ int fhs_compute_sara_prior(fhs_ctx* ctx, const fhs_sara* S, const float* x, int 
       float* c = (float*)ctx->ws.get("sara_prior_coefs", (size_t)G.s * L * sizeof(float));
       sara_analyse<AN_SET>(ctx, S, x, L, c, nullptr, 0.0, nullptr, nullptr);
       nsum = std::min<unsigned>(2048, cdiv(G.s, 256));
-      k_l21<<<nsum, 256, 0, ctx->stream>>>(G, c, nullptr, L, nullptr, 0.0, 1, nullptr, part);
+      k_l21<<<nsum, 256, 0, ctx->stream>>>(G.s, c, L, nullptr, 0.0, 1, nullptr, part);
       check_launch();
     }
     k_sum_l<<<1, 256, 0, ctx->stream>>>(part, (int)nsum, part + n);
