@@ -629,6 +629,25 @@ __global__ __launch_bounds__(64 * ST_WAVES) void k_synthesis(SaraArgs G, int ty,
   }
 }
 
+// The Dirac basis alone: no tiles (8 images of 512 x 512, dual step 17.3 -> 10.5 us).
+template <int VEC>
+__global__ __launch_bounds__(256) void k_dirac_synthesis(SaraGeom G, const float* __restrict__ v1, float scale,
+                                                         float* __restrict__ out) {
+  struct alignas(4 * VEC) Vec {
+    float v[VEC];
+  };
+  const int64_t N = (int64_t)G.Ny * G.Nx;
+  v1 += blockIdx.y * G.s;
+  out += blockIdx.y * N;
+  for (int64_t p = VEC * (blockIdx.x * (int64_t)blockDim.x + threadIdx.x); p < N;
+       p += VEC * (int64_t)gridDim.x * blockDim.x) {
+    Vec r = *reinterpret_cast<const Vec*>(v1 + p);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) r.v[j] = r.v[j] * G.norm * scale;
+    *reinterpret_cast<Vec*>(out + p) = r;
+  }
+}
+
 // ---- more than 16 channels ---------------------------------------------------
 // The modes over the channels from stored coefficients, Dirac block included (mode 0:
 // l21 step, 1: sum of the norms, 2: weights).
@@ -759,8 +778,15 @@ void sara_synthesis(fhs_ctx* ctx, const fhs_sara* S, const float* v1, int L, flo
   const SaraGeom& G = S->g;
   float* scr = (float*)ctx->ws.get("sara_scratch", std::max<int64_t>(1, G.scr_per_chan * L) * sizeof(float));
   Scope sc(ctx, "wavelet_synthesis");
+  if (G.nb == 0) {   // G.s = Ny Nx
+    const bool vec = G.s % 4 == 0 && ((uintptr_t)v1 | (uintptr_t)out) % 16 == 0;
+    (vec ? k_dirac_synthesis<4> : k_dirac_synthesis<1>)<<<dim3(std::min<unsigned>(2048, cdiv(vec ? G.s / 4 : G.s, 256)), L),
+                                                         256, 0, ctx->stream>>>(G, v1, scale, out);
+    check_launch();
+    return;
+  }
   auto grid = [](int ty, int txg, int z) { return dim3(8 * cdiv((long long)ty * txg * z, 8), 1, 1); };
-  for (int k = G.nlevel; k >= 2 && G.nb > 0; --k) {
+  for (int k = G.nlevel; k >= 2; --k) {
     int py = 0, px = 0;
     for (int b = 0; b < G.nb; ++b) {
       py = std::max(py, G.ny[b][k - 1]);

@@ -132,3 +132,13 @@ def test_many_channels_take_no_more_launches():
         torch.cuda.synchronize()
         nodes.append(_captured_nodes(ctx, lambda: S.psit(x, out=c)))
     assert nodes == [4, 4, 4], nodes           # three levels and the Dirac block
+
+
+@pytest.mark.parametrize('Ny,Nx,L', [(1, 1, 1), (33, 17, 3), (600, 900, 2)])
+def test_dirac_basis_alone(ctx, Ny, Nx, L):
+    """Without wavelets the transforms are the identity, the dual step the threshold."""
+    import fhs
+    S = fhs.SaraDictionary(ctx, Ny, Nx, bases=('self',), nlevel=1)
+    x = torch.randn((L, Nx, Ny), device='cuda')
+    assert torch.equal(S.psit(x).reshape(x.shape), x)
+    assert torch.equal(S.psi(x.reshape(L, -1), scale=0.5), 0.5 * x)
