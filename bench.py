@@ -542,7 +542,7 @@ def cube_main(args):
                      'unit': 'GB/s', 'frac': round(achieved / PEAK_HBM_GBS, 4),
                      'traffic': None if traffic is None else int(traffic),
                      'traffic_source': ('profiles/fhs2048x64_pmc_traffic.json (FETCH_SIZE x 2 + WRITE_SIZE, '
-                                        'copy-calibrated; an upper bound for this gather kernel: its raw '
+                                        'copy-calibrated; an upper bound where a kernel gathers rows: raw '
                                         'FETCH_SIZE is 64 bytes per memory request, and the factor 2 fits the '
                                         'streaming copy)'),
                      'avg_launch_ms': round(avg_ms, 5), 'algorithmic_bytes_per_launch': int(alg[dominant]),

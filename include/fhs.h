@@ -430,6 +430,7 @@ typedef struct {
   const float* weights1;
   const float* Lambda;
 } fhs_pdfb_buffers;
+/* data, sara, lowrank and the buffers must outlive the engine, which reads them. */
 int fhs_pdfb_create(fhs_ctx* ctx, fhs_data* data, fhs_sara* sara, fhs_lowrank* lowrank,
                     const fhs_pdfb_buffers* bufs, fhs_pdfb** out);
 int fhs_pdfb_destroy(fhs_pdfb* p);
